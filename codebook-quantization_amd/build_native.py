@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 SO = os.path.join(HERE, "libcbq_hip.so")
 ARCH = "gfx950"
 SOURCES = ["cbq_fixed.hip", "cbq_huffman.hip", "cbq_prefill.hip", "cbq_prefill_f32.hip",
-           "cbq_decode.hip", "cbq_split.hip", "cbq_tiny.hip"]
+           "cbq_decode.hip", "cbq_split.hip", "cbq_tiny.hip", "cbq_gemm.hip"]
 # host-only C++ (no device code): compiled by the host compiler
 HOST_SOURCES = ["cbq_huff_host.cpp", "cbq_io.cpp"]
 HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-pthread", "-D__HIP_PLATFORM_AMD__=1",

@@ -1080,8 +1080,13 @@ int cbq_prefill_bf16(const uint16_t *x, const uint8_t *packed, const float *cb, 
 size_t cbq_prefill_ws_bytes(int T, int M, int K);
 // fp32 MFMA prefill path (cbq_prefill_f32.hip); -1 = shape not handled there.
 int cbq_prefill_f32(const float *x, const uint8_t *packed, const float *cb, float *out, int T,
-                    int M, int K, int C, int bits, hipStream_t st, int S, float *ws);
-int cbq_prefill_f32_splits(int T, int M, int K);
+                    int M, int K, int C, int bits, hipStream_t st);
+// decode-first GEMM on the bf16 matrix cores, with a workspace (cbq_gemm.hip);
+// -1 = not handled there.
+int cbq_frag_linear(const void *x, bool f32, const uint8_t *packed, const float *cb, void *out,
+                    int T, int M, int K, int C, int bits, void *ws, size_t ws_bytes,
+                    hipStream_t st);
+size_t cbq_frag_ws_bytes(int T, int M, int K, bool f32);
 
 int cbq_num_cus()
 {
@@ -1118,8 +1123,7 @@ int ck_linear_f32(const float *x, const uint8_t *packed, const float *codebook, 
     // T >= 64: the GEMM regime, fp32 MFMA (cbq_prefill_f32.hip)
     if (x && packed && codebook && out && T >= 64 && M > 0 && K > 0 && C > 0 && bits >= 1 &&
         bits <= 16) {
-        const int rc = cbq_prefill_f32(x, packed, codebook, out, T, M, K, C, bits, stream, 1,
-                                       nullptr);
+        const int rc = cbq_prefill_f32(x, packed, codebook, out, T, M, K, C, bits, stream);
         if (rc >= 0) return rc;
     }
     return linear_any_t<float, float>(x, packed, codebook, out, T, M, K, C, bits, stream);
@@ -1128,8 +1132,7 @@ int ck_linear_f32(const float *x, const uint8_t *packed, const float *codebook, 
 size_t cbq_linear_f32_workspace(int T, int M, int K)
 {
     if (T <= 0 || M <= 0 || K <= 0) return 0;
-    const int S = cbq_prefill_f32_splits(T, M, K);
-    return S > 1 ? (size_t)S * T * M * sizeof(float) : 0;
+    return cbq_frag_ws_bytes(T, M, K, true);
 }
 
 int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebook, float *out,
@@ -1138,12 +1141,8 @@ int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebo
 {
     if (x && packed && codebook && out && T >= 64 && M > 0 && K > 0 && C > 0 && bits >= 1 &&
         bits <= 16) {
-        const size_t need = cbq_linear_f32_workspace(T, M, K);
-        const bool split = need > 0 && workspace && ws_bytes >= need &&
-                           ((uintptr_t)workspace & 15) == 0;
-        const int rc = cbq_prefill_f32(x, packed, codebook, out, T, M, K, C, bits, stream,
-                                       split ? cbq_prefill_f32_splits(T, M, K) : 1,
-                                       split ? (float *)workspace : nullptr);
+        const int rc = cbq_frag_linear(x, true, packed, codebook, out, T, M, K, C, bits, workspace,
+                                       ws_bytes, stream);
         if (rc >= 0) return rc;
     }
     return ck_linear_f32(x, packed, codebook, out, T, M, K, C, bits, stream);

@@ -46,16 +46,20 @@ int ck_linear_f32(const float *x, const uint8_t *packed, const float *codebook,
                   float *out, int T, int M, int K, int C, int bits,
                   hipStream_t stream);
 
-/* Workspace bytes cbq_linear_f32_ws splits K with for a T x M x K product
- * (0: no split).  No counterpart in the reference. */
+/* Workspace bytes of cbq_linear_f32_ws for a T x M x K product (0: the shape
+ * runs as ck_linear_f32).  No counterpart in the reference. */
 size_t cbq_linear_f32_workspace(int T, int M, int K);
 
-/* ck_linear_f32 with a caller workspace: for T >= 64 on the fp32 MFMA path
- * (widths 8 and 10..13), grids under two blocks per CU split K across
- * blocks that write fp32 partials to `workspace` (>= cbq_linear_f32_workspace
- * bytes, 16-byte aligned), summed in split order by a second kernel.  With a
- * smaller workspace it is ck_linear_f32.  No counterpart in the reference:
- * batched fp32 tokens through GPUAcceleratedLinear
+/* ck_linear_f32 with a caller workspace (>= cbq_linear_f32_workspace bytes,
+ * 16-byte aligned): for T >= 64 (K % 32 == 0, widths 8 and 10..14, x 16-byte
+ * aligned) x (three exact bf16 parts) and the weights are first written there
+ * in MFMA fragment order, the weights in slabs of at most 384 MiB, and
+ * multiplied on the bf16 matrix cores with fp32 accumulation; K is split
+ * over blocks when the output tiles alone would leave CUs idle (partials in
+ * the workspace, summed in split order).  A codebook with values that are
+ * not bf16 numbers is split into bf16 parts as well.  With a smaller
+ * workspace it is ck_linear_f32.  No counterpart in the reference: batched
+ * fp32 tokens through GPUAcceleratedLinear
  * (src/gpu_accelerated_functions.py:928-950), e.g. a prompt prefill. */
 int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebook, float *out,
                       int T, int M, int K, int C, int bits, void *workspace, size_t ws_bytes,

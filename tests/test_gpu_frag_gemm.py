@@ -1,0 +1,125 @@
+"""The decode-first batched GEMM (cbq_linear_f32_ws with its workspace) at the
+edges of its tiles, column groups, K splits, slabs and codebook kinds, against
+float64 products of the decoded matrix.
+
+Bound for fp32 x: every product is exact (codebooks of bf16 numbers) or short
+of the whole by less than 2^-22 (others), and the sum is rounded to fp32 in
+chains of at most 48 MFMAs and K / 512 additions: rel-L2 <= 5e-7 for random
+signs."""
+import numpy as np
+import pytest
+import torch
+
+import cbq_native as nat
+import codebook_builder as cbb
+
+pytestmark = pytest.mark.gpu
+TOL_F32 = 5e-7
+
+
+def _matrix(cuda, M, K, bits, kind, seed):
+    """(packed, codebook, dense float64 W): indices over the whole width, so
+    some lie past C and clamp."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    C = max(2, (1 << bits) * 5 // 8)
+    cb = torch.randn(C, device=cuda, generator=g) * 0.02
+    if kind != "fp32":
+        cb = cb.bfloat16().float()
+    if kind == "inf":
+        cb[C // 2] = float("inf")
+    idx = torch.randint(0, 1 << bits, (M, K), device=cuda, generator=g)
+    pk = cbb.pack_torch(idx, bits)
+    packed = torch.zeros((pk.numel() + 15) // 16 * 16 + 16, dtype=torch.uint8, device=cuda)
+    packed[:pk.numel()] = pk
+    return packed, cb, cb[idx.clamp_max(C - 1)].double()
+
+
+def _run_f32(cuda, x, packed, cb, M, K, bits):
+    lib = nat.load()
+    T = x.shape[0]
+    n = int(lib.cbq_linear_f32_workspace(T, M, K))
+    assert n > 0
+    ws = torch.full((n,), 0xFF, dtype=torch.uint8, device=cuda)
+    out = torch.full((T, M), float("nan"), device=cuda)
+    nat.check(lib.cbq_linear_f32_ws(x.data_ptr(), packed.data_ptr(), cb.data_ptr(),
+                                    out.data_ptr(), T, M, K, cb.numel(), bits, ws.data_ptr(), n,
+                                    nat.stream_ptr(cuda)), "cbq_linear_f32_ws")
+    return out
+
+
+def _rel(y, ref):
+    return float((y.double() - ref).norm() / ref.norm())
+
+
+@pytest.mark.parametrize("T,M,K,bits", [
+    (64, 1, 32, 13),            # one column group, one row
+    (65, 33, 64, 12),           # a row past a superblock, a token past a tile
+    (127, 257, 96, 14), (129, 300, 4064, 13), (192, 520, 288, 11), (257, 1000, 1056, 10),
+    (64, 4096, 4096, 13), (300, 2048, 2080, 8), (1030, 3000, 544, 13)])
+@pytest.mark.parametrize("kind", ["bf16", "fp32"])
+def test_f32_edges(cuda, T, M, K, bits, kind):
+    print(f"f32 {kind} T{T} M{M} K{K} bits{bits}", flush=True)
+    packed, cb, w = _matrix(cuda, M, K, bits, kind, T + M)
+    x = torch.randn(T, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(K))
+    y = _run_f32(cuda, x, packed, cb, M, K, bits)
+    assert _rel(y, x.double() @ w.T) <= TOL_F32
+
+
+def test_f32_slabs(cuda):
+    """A row so long that the fragments are written slab by slab."""
+    T, M, K, bits = 64, 520, 262176, 12
+    packed, cb, w = _matrix(cuda, M, K, bits, "bf16", 3)
+    x = torch.randn(T, K, device=cuda)
+    assert _rel(_run_f32(cuda, x, packed, cb, M, K, bits), x.double() @ w.T) <= TOL_F32
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp32", "inf"])
+def test_f32_non_finite(cuda, kind):
+    """Infinities and NaNs of x and the codebook reach the outputs that a
+    plain fp32 sum gives them."""
+    T, M, K, bits = 70, 200, 256, 8
+    packed, cb, w = _matrix(cuda, M, K, bits, kind, 5)
+    x = torch.randn(T, K, device=cuda)
+    x[3, 7], x[9, 100], x[11, 0] = float("inf"), float("-inf"), float("nan")
+    x[20] = 0.0
+    y = _run_f32(cuda, x, packed, cb, M, K, bits)
+    ref = x.double() @ w.T
+    assert torch.equal(y.isnan(), ref.isnan())
+    assert torch.equal(y.isposinf(), ref.isposinf()) and torch.equal(y.isneginf(), ref.isneginf())
+    ok = ref.isfinite()
+    assert _rel(y[ok], ref[ok]) <= TOL_F32
+
+
+def test_f32_scales(cuda):
+    """Token rows over 60 decades keep their relative error."""
+    T, M, K, bits = 64, 96, 512, 13
+    packed, cb, w = _matrix(cuda, M, K, bits, "bf16", 6)
+    s = 10.0 ** torch.linspace(-30, 30, T, device=cuda, dtype=torch.float64)
+    x = (torch.randn(T, K, device=cuda).double() * s[:, None]).float()
+    y, ref = _run_f32(cuda, x, packed, cb, M, K, bits), x.double() @ w.T
+    assert float(((y.double() - ref).norm(dim=1) / ref.norm(dim=1)).max()) <= 2 * TOL_F32
+
+
+def test_f32_graph(cuda):
+    """Captured and replayed with other inputs in between: the eager result."""
+    T, M, K, bits = 100, 1024, 2048, 13
+    packed, cb, w = _matrix(cuda, M, K, bits, "bf16", 7)
+    lib = nat.load()
+    x = torch.randn(T, K, device=cuda)
+    n = int(lib.cbq_linear_f32_workspace(T, M, K))
+    ws = torch.empty(n, dtype=torch.uint8, device=cuda)
+    out = torch.empty(T, M, device=cuda)
+
+    def call():
+        nat.check(lib.cbq_linear_f32_ws(x.data_ptr(), packed.data_ptr(), cb.data_ptr(),
+                                        out.data_ptr(), T, M, K, cb.numel(), bits, ws.data_ptr(),
+                                        n, nat.stream_ptr(cuda)), "cbq_linear_f32_ws")
+    call()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for i in range(3):
+        x.copy_(torch.randn(T, K, device=cuda))
+        eager = _run_f32(cuda, x, packed, cb, M, K, bits)
+        graph.replay()
+        assert torch.equal(out, eager)
