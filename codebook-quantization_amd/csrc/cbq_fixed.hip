@@ -1028,11 +1028,21 @@ int linear_any_t(const XT *x, const uint8_t *packed, const float *cb, OT *out, i
 {
     if (!x || !packed || !cb || !out) return CK_ERR_ARG;
     if (T <= 0 || M <= 0 || K <= 0 || C <= 0 || bits < 1 || bits > 16) return CK_ERR_ARG;
-    for (int t0 = 0; t0 < T; t0 += 16) {
-        const int tt = std::min(16, T - t0);
-        int rc = linear_tile<XT, OT>(x + (size_t)t0 * K, packed, cb, out + (size_t)t0 * M,
-                                     tt, M, K, C, bits, st);
+    for (int t0 = 0; t0 < T;) {
+        int tt = std::min(16, T - t0);
+        int rc = -1;
+        if constexpr (sizeof(XT) == 2) {           // bf16: up to 64 tokens share one decode
+            const int t64 = std::min(64, T - t0);
+            if (t64 > 16)
+                rc = cbq_fixed_fewtok_t_bf16(x + (size_t)t0 * K, packed, cb, out + (size_t)t0 * M,
+                                             t64, M, K, C, bits, st);
+            if (rc >= 0) tt = t64;
+        }
+        if (rc < 0)
+            rc = linear_tile<XT, OT>(x + (size_t)t0 * K, packed, cb, out + (size_t)t0 * M, tt, M,
+                                     K, C, bits, st);
         if (rc) return rc;
+        t0 += tt;
     }
     return CK_SUCCESS;
 }
@@ -1318,12 +1328,17 @@ int cbq_linear_affine_f32(const float *x, const uint8_t *packed, uint32_t lo, ui
 int ck_linear_bf16(const void *x_bf16, const uint8_t *packed, const float *codebook,
                    void *out_bf16, int T, int M, int K, int C, int bits, hipStream_t stream)
 {
-    // T >= 64: the GEMM regime, bf16 MFMA with fp32 accumulation (cbq_prefill.hip)
-    if (x_bf16 && packed && codebook && out_bf16 && T >= 64 && M > 0 && K > 0 && C > 0 &&
+    if (x_bf16 && packed && codebook && out_bf16 && T > 16 && M > 0 && K > 0 && C > 0 &&
         bits >= 1 && bits <= 16) {
-        const int rc = cbq_prefill_bf16((const uint16_t *)x_bf16, packed, codebook,
-                                        (uint16_t *)out_bf16, T, M, K, C, bits, stream, nullptr,
-                                        0);
+        // up to 64 tokens on one decode of the weights (cbq_tiny.hip); from 64
+        // on the GEMM regime, bf16 MFMA with fp32 accumulation (cbq_prefill.hip)
+        int rc = -1;
+        if (T <= 64)
+            rc = cbq_fixed_fewtok_t_bf16((const uint16_t *)x_bf16, packed, codebook,
+                                         (uint16_t *)out_bf16, T, M, K, C, bits, stream);
+        if (rc < 0 && T >= 64)
+            rc = cbq_prefill_bf16((const uint16_t *)x_bf16, packed, codebook,
+                                  (uint16_t *)out_bf16, T, M, K, C, bits, stream, nullptr, 0);
         if (rc >= 0) return rc;
     }
     return linear_any_t<uint16_t, uint16_t>((const uint16_t *)x_bf16, packed, codebook,

@@ -1,5 +1,5 @@
-// Fixed-width GEMM for a few tokens (2 <= T <= 16; ck_linear_f32 and
-// ck_linear_bf16 send it tiles of 2..16) on the matrix cores of gfx950
+// Fixed-width GEMM for a few tokens (2 <= T <= 16, bf16 up to 64;
+// ck_linear_f32 and ck_linear_bf16 send it tiles) on the matrix cores of gfx950
 // (rocm/compressed_kernel.hip:607-627 is the reference entry point; its
 // kernel runs one block per output scalar).
 //
@@ -26,6 +26,11 @@
 //   - MFMA c of a tile-step takes chunk c (indices 8c .. 8c+7) of each of the
 //     step's four groups, for the weights (A: row l % 16) and for x (B: token
 //     l % 16) alike.  x of a step is split once and serves the R tiles.
+//   - bf16 x: up to four blocks of 16 tokens a launch (NT), each with its own
+//     accumulators.  The decode of a tile-step (unpack, 32 random LDS reads a
+//     lane) is what bounds one block, so the others cost little beside
+//     reading the weights again: 12288 x 4096, bf16, T = 40: 62 -> 26 us
+//     (three 16-token launches before), T = 64: 75 -> 32 us.
 //   - The 8 waves' partial tiles are summed through LDS in wave order.
 // Measured against the per-lane loads of one 52-byte group each (16 rows x
 // 4 groups per instruction): 44.6 us for the 163.6 MB stacked gate+up read
@@ -101,8 +106,9 @@ template <> struct FtX<uint16_t> {
 };
 
 // R row tiles per block, Q tile-steps of weights in flight per wave (Q
-// divides R, so every ring slot is a compile-time register array).
-template <int BITS, int R, int Q, typename XT, typename OT>
+// divides R, so every ring slot is a compile-time register array), NT blocks
+// of 16 tokens: a decoded tile-step is multiplied with each of them.
+template <int BITS, int R, int Q, int NT, typename XT, typename OT>
 __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
     const XT *__restrict__ x, const uint32_t *__restrict__ words,
     const float *__restrict__ cb, OT *__restrict__ out, int T, int M, int K, int C)
@@ -116,7 +122,7 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
     __shared__ __attribute__((aligned(16))) float s_cb[PADDED ? (1 << BITS) : kTinyMaxCodebook];
     __shared__ __attribute__((aligned(16))) uint32_t s_tr[kFtWaves][64 * BITS];
     __shared__ int s_flag[kFtWaves];
-    extern __shared__ __attribute__((aligned(16))) f4 s_part[];     // [8][R][64]
+    extern __shared__ __attribute__((aligned(16))) f4 s_part[];     // [8][R][NT][64]
 
     const int tid = threadIdx.x;
     const int lane = tid & (CBQ_WAVE - 1);
@@ -128,12 +134,12 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
     const int tile0 = blockIdx.x * R;
     const size_t rowstride = (size_t)G * BITS;    // words of a packed row
     const int C_eff = C < (1 << BITS) ? C : (1 << BITS);
-    const int NT = PADDED ? (1 << BITS) : ((C_eff + 63) & ~63);
+    const int TE = PADDED ? (1 << BITS) : ((C_eff + 63) & ~63);     // table entries
 
     // codebook loads first, so that waiting for them leaves the weight and
     // x loads below in flight
     constexpr int kMaxNE = ((PADDED ? (1 << BITS) : kTinyMaxCodebook) + kFtThreads - 1) / kFtThreads;
-    const int NE = (NT + kFtThreads - 1) / kFtThreads;
+    const int NE = (TE + kFtThreads - 1) / kFtThreads;
     float cv[kMaxNE];
 #pragma unroll
     for (int e = 0; e < kMaxNE; e++) {
@@ -168,27 +174,34 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
             __builtin_memcpy(&dst[k], words + (size_t)row * rowstride + col + 4 * cpiece[k], 16);
         }
     };
-    auto load_x = [&](int s, uint32_t (&xw)[XW]) {
-        if (rsub < T) {
-            __builtin_memcpy(xw, x + (size_t)rsub * K + (size_t)(4 * gstep(s) + j) * 32,
-                             sizeof(xw));
-        } else {
+    auto load_x = [&](int s, uint32_t (&xw)[NT][XW]) {
 #pragma unroll
-            for (int i = 0; i < XW; i++) xw[i] = 0u;
+        for (int b = 0; b < NT; b++) {
+            const int t = b * 16 + rsub;
+            if (t < T) {
+                __builtin_memcpy(xw[b], x + (size_t)t * K + (size_t)(4 * gstep(s) + j) * 32,
+                                 sizeof(xw[b]));
+            } else {
+#pragma unroll
+                for (int i = 0; i < XW; i++) xw[b][i] = 0u;
+            }
         }
     };
     u32x4 wr[Q][NI];
 #pragma unroll
     for (int q = 0; q < Q; q++) load_item(0, q, wr[q]);
-    uint32_t xn[XW];
-    load_x(0, xn);
+    // up to two token blocks: x a step ahead; more would not fit the
+    // registers, and the decode of the step's first tile covers their loads
+    constexpr bool XAHEAD = NT <= 2;
+    uint32_t xn[NT][XW];
+    if constexpr (XAHEAD) load_x(0, xn);
     __builtin_amdgcn_sched_barrier(0);
 
     int inexact = 0;
 #pragma unroll
     for (int e = 0; e < kMaxNE; e++) {
         const int i = e * kFtThreads + tid;
-        if (e < NE && i < NT) {
+        if (e < NE && i < TE) {
             s_cb[i] = cv[e];
             inexact |= (__float_as_uint(cv[e]) & 0xffffu) != 0;
         }
@@ -203,15 +216,19 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
     for (int w = 0; w < kFtWaves; w++) wsplit |= s_flag[w] != 0;
     const uint32_t cmax4 = (uint32_t)(C_eff - 1) << 2;
 
-    f4 acc[R];
+    f4 acc[R][NT];
 #pragma unroll
-    for (int t = 0; t < R; t++) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < R; t++)
+#pragma unroll
+        for (int b = 0; b < NT; b++) acc[t][b] = f4{0.f, 0.f, 0.f, 0.f};
     uint32_t *tr = s_tr[wave];
 
     for (int s = 0; s < Sw; s++) {
-        u32x4 xb[4][3];
-        FtX<XT>::parts(xn, xb);
-        load_x(s + 1, xn);                         // next step's x, one step ahead
+        u32x4 xb[NT][4][3];
+        if constexpr (!XAHEAD) load_x(s, xn);
+#pragma unroll
+        for (int b = 0; b < NT; b++) FtX<XT>::parts(xn[b], xb[b]);
+        if constexpr (XAHEAD) load_x(s + 1, xn);   // next step's x, one step ahead
 #pragma unroll
         for (int t = 0; t < R; t++) {
             u32x4 (&slot)[NI] = wr[t % Q];
@@ -242,7 +259,10 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
 #pragma unroll
             for (int c = 0; c < 4; c++)
 #pragma unroll
-                for (int p = 0; p < FtX<XT>::kParts; p++) acc[t] = cbq_mfma_bf16(a[c], xb[c][p], acc[t]);
+                for (int p = 0; p < FtX<XT>::kParts; p++)
+#pragma unroll
+                    for (int b = 0; b < NT; b++)
+                        acc[t][b] = cbq_mfma_bf16(a[c], xb[b][c][p], acc[t][b]);
             if (wsplit) {                          // codebook not bf16: w = wh + wm + wl
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
@@ -251,9 +271,13 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
                     for (int e = 0; e < 8; e++) q8[e] = wv[8 * c + e];
                     u32x4 wh, wm, wl;
                     cbq_split3(q8, wh, wm, wl);
-                    acc[t] = cbq_mfma_bf16(wm, xb[c][0], acc[t]);
-                    acc[t] = cbq_mfma_bf16(wl, xb[c][0], acc[t]);
-                    if (FtX<XT>::kParts > 1) acc[t] = cbq_mfma_bf16(wm, xb[c][1], acc[t]);
+#pragma unroll
+                    for (int b = 0; b < NT; b++) {
+                        acc[t][b] = cbq_mfma_bf16(wm, xb[b][c][0], acc[t][b]);
+                        acc[t][b] = cbq_mfma_bf16(wl, xb[b][c][0], acc[t][b]);
+                        if (FtX<XT>::kParts > 1)
+                            acc[t][b] = cbq_mfma_bf16(wm, xb[b][c][1], acc[t][b]);
+                    }
                 }
             }
         }
@@ -261,25 +285,27 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
 
     // the 8 waves' partial tiles, summed in wave order
 #pragma unroll
-    for (int t = 0; t < R; t++) s_part[(wave * R + t) * CBQ_WAVE + lane] = acc[t];
+    for (int t = 0; t < R; t++)
+#pragma unroll
+        for (int b = 0; b < NT; b++)
+            s_part[((wave * R + t) * NT + b) * CBQ_WAVE + lane] = acc[t][b];
     __syncthreads();
-    if (wave < R) {
-        const int t = wave;
-        f4 sum = s_part[t * CBQ_WAVE + lane];
+    for (int u = wave; u < R * NT; u += kFtWaves) {
+        f4 sum = s_part[u * CBQ_WAVE + lane];
 #pragma unroll
         for (int w = 1; w < kFtWaves; w++) {
-            const f4 v = s_part[(w * R + t) * CBQ_WAVE + lane];
+            const f4 v = s_part[(w * R * NT + u) * CBQ_WAVE + lane];
             sum.x += v.x;
             sum.y += v.y;
             sum.z += v.z;
             sum.w += v.w;
         }
         // D[m][n]: lane l, element v holds row m = 4 (l / 16) + v, token n = l % 16
-        const int n = lane & 15;
+        const int n = (u % NT) * 16 + (lane & 15);
         const float vals[4] = {sum.x, sum.y, sum.z, sum.w};
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            const int row = (tile0 + t) * 16 + 4 * j + v;
+            const int row = (tile0 + u / NT) * 16 + 4 * j + v;
             if (row < M && n < T) out[(size_t)n * M + row] = from_f32<OT>(vals[v]);
         }
     }
@@ -447,14 +473,14 @@ int tiny_launch(const XT *x, const uint8_t *packed, const float *cb, OT *out, in
     return cbq_launch_status("fixed_tiny_mfma_kernel");
 }
 
-template <int R, int Q, typename XT, typename OT>
+template <int R, int Q, int NT, typename XT, typename OT>
 int fewtok_launch_r(const XT *x, const uint8_t *packed, const float *cb, OT *out, int T, int M,
                     int K, int C, int bits, int blocks, hipStream_t st)
 {
-    const size_t lds = (size_t)kFtWaves * R * CBQ_WAVE * sizeof(f4);
+    const size_t lds = (size_t)kFtWaves * R * NT * CBQ_WAVE * sizeof(f4);
 #define CBQ_FT(B)                                                                              \
-    hipLaunchKernelGGL((fixed_fewtok_kernel<B, R, Q, XT, OT>), dim3(blocks), dim3(kFtThreads),  \
-                       lds, st, x, (const uint32_t *)packed, cb, out, T, M, K, C)
+    hipLaunchKernelGGL((fixed_fewtok_kernel<B, R, Q, NT, XT, OT>), dim3(blocks),                \
+                       dim3(kFtThreads), lds, st, x, (const uint32_t *)packed, cb, out, T, M, K, C)
     switch (bits) {
     case 8: CBQ_FT(8); break;
     case 10: CBQ_FT(10); break;
@@ -470,25 +496,25 @@ int fewtok_launch_r(const XT *x, const uint8_t *packed, const float *cb, OT *out
 }
 
 // Row tiles per block R (6, 3, 2 or 1; a block holds one CU: 8 waves, up to
-// 141 KiB of LDS): the R of least rounds x (R + 1), rounds =
+// 155 KiB of LDS): the R of least rounds x (R + 1), rounds =
 // ceil(ceil(tiles / R) / CUs) and the + 1 a block's fixed cost in tiles
 // (codebook staging, the first loads, the partial-tile sums), larger R on a
 // tie.  E.g. 384 tiles on 256 CUs take R = 2 (one round of 192 blocks, 16
 // us for the 9B stacked q/k/v at 2 tokens) rather than two rounds of R = 1
-// (20 us); 1536 tiles take R = 6.
-template <typename XT, typename OT>
-int fewtok_launch(const XT *x, const uint8_t *packed, const float *cb, OT *out, int T, int M,
-                  int K, int C, int bits, hipStream_t st)
+// (20 us); 1536 tiles take R = 6.  Several token blocks: R * NT partial tiles
+// a wave beside the table and the re-lay buffers, at most 6 at 14 and 16
+// bits (92 and 96 KiB) and 12 below (59 KiB at 13).
+template <int NT, typename XT, typename OT>
+int fewtok_launch_n(const XT *x, const uint8_t *packed, const float *cb, OT *out, int T, int M,
+                    int K, int C, int bits, hipStream_t st)
 {
-    if (T < 2 || T > 16 || M <= 0 || K <= 0 || K % 128 || C <= 0 || C > kTinyMaxCodebook)
-        return -1;
-    if (((uintptr_t)x & 15) != 0 || ((uintptr_t)packed & 15) != 0) return -1;
-    if (bits != 8 && (bits < 10 || bits > 14) && bits != 16) return -1;
     const long tiles = (M + 15) / 16;
     const long ncu = cbq_num_cus();
+    const int rmax = NT == 1 ? 6 : std::min(3, (bits >= 14 ? 6 : 12) / NT);
     int R = 1;
     long best = -1;
     for (const int r : {1, 2, 3, 6}) {
+        if (r > rmax) break;
         const long cost = ((tiles + r - 1) / r + ncu - 1) / ncu * (r + 1);
         if (best < 0 || cost <= best) {
             best = cost;
@@ -497,12 +523,31 @@ int fewtok_launch(const XT *x, const uint8_t *packed, const float *cb, OT *out, 
     }
     const long blocks = (tiles + R - 1) / R;
     if (blocks > 0x7fffffffL) return -1;
+    if constexpr (NT == 1)
+        if (R == 6)
+            return fewtok_launch_r<6, 2, NT>(x, packed, cb, out, T, M, K, C, bits, (int)blocks, st);
     switch (R) {
-    case 6: return fewtok_launch_r<6, 2>(x, packed, cb, out, T, M, K, C, bits, (int)blocks, st);
-    case 3: return fewtok_launch_r<3, 3>(x, packed, cb, out, T, M, K, C, bits, (int)blocks, st);
-    case 2: return fewtok_launch_r<2, 2>(x, packed, cb, out, T, M, K, C, bits, (int)blocks, st);
-    default: return fewtok_launch_r<1, 1>(x, packed, cb, out, T, M, K, C, bits, (int)blocks, st);
+    case 3: return fewtok_launch_r<3, (NT > 3 ? 1 : 3), NT>(x, packed, cb, out, T, M, K, C, bits, (int)blocks, st);
+    case 2: return fewtok_launch_r<2, 2, NT>(x, packed, cb, out, T, M, K, C, bits, (int)blocks, st);
+    default: return fewtok_launch_r<1, 1, NT>(x, packed, cb, out, T, M, K, C, bits, (int)blocks, st);
     }
+}
+
+template <typename XT, typename OT>
+int fewtok_launch(const XT *x, const uint8_t *packed, const float *cb, OT *out, int T, int M,
+                  int K, int C, int bits, hipStream_t st)
+{
+    if (T < 2 || T > (sizeof(XT) == 2 ? 64 : 16) || M <= 0 || K <= 0 || K % 128 || C <= 0 ||
+        C > kTinyMaxCodebook)
+        return -1;
+    if (((uintptr_t)x & 15) != 0 || ((uintptr_t)packed & 15) != 0) return -1;
+    if (bits != 8 && (bits < 10 || bits > 14) && bits != 16) return -1;
+    if constexpr (sizeof(XT) == 2) {
+        if (T > 48) return fewtok_launch_n<4>(x, packed, cb, out, T, M, K, C, bits, st);
+        if (T > 32) return fewtok_launch_n<3>(x, packed, cb, out, T, M, K, C, bits, st);
+        if (T > 16) return fewtok_launch_n<2>(x, packed, cb, out, T, M, K, C, bits, st);
+    }
+    return fewtok_launch_n<1>(x, packed, cb, out, T, M, K, C, bits, st);
 }
 
 }  // namespace
@@ -522,8 +567,8 @@ int cbq_fixed_tiny_t_bf16(const uint16_t *x, const uint8_t *packed, const float 
     return tiny_launch<uint16_t, uint16_t>(x, packed, cb, out, T, M, K, C, bits, st);
 }
 
-// 2 <= T <= 16 tokens (fp32, or bf16 x and out), K % 128 == 0, 16-byte
-// aligned x and stream, widths 8, 10-14 and 16, C <= 16384: the bf16
+// 2 <= T <= 16 tokens of fp32, or 2 <= T <= 64 of bf16 x and out,
+// K % 128 == 0, 16-byte aligned x and stream, widths 8, 10-14 and 16, C <= 16384: the bf16
 // matrix-core kernel above; returns -1 for shapes it does not take.
 int cbq_fixed_fewtok_t(const float *x, const uint8_t *packed, const float *cb, float *out, int T,
                        int M, int K, int C, int bits, hipStream_t st)
