@@ -1096,7 +1096,7 @@ int cbq_prefill_f32(const float *x, const uint8_t *packed, const float *cb, floa
 int cbq_frag_linear(const void *x, bool f32, const uint8_t *packed, const float *cb, void *out,
                     int T, int M, int K, int C, int bits, void *ws, size_t ws_bytes,
                     hipStream_t st);
-size_t cbq_frag_ws_bytes(int T, int M, int K, bool f32);
+size_t cbq_frag_ws_bytes(int T, int M, int K, int bits, bool f32);
 
 int cbq_num_cus()
 {
@@ -1142,15 +1142,14 @@ int ck_linear_f32(const float *x, const uint8_t *packed, const float *codebook, 
 size_t cbq_linear_f32_workspace(int T, int M, int K)
 {
     if (T <= 0 || M <= 0 || K <= 0) return 0;
-    return cbq_frag_ws_bytes(T, M, K, true);
+    return cbq_frag_ws_bytes(T, M, K, 0, true);
 }
 
 int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebook, float *out,
                       int T, int M, int K, int C, int bits, void *workspace, size_t ws_bytes,
                       hipStream_t stream)
 {
-    if (x && packed && codebook && out && T >= 64 && M > 0 && K > 0 && C > 0 && bits >= 1 &&
-        bits <= 16) {
+    if (x && packed && codebook && out && M > 0 && K > 0 && C > 0 && bits >= 1 && bits <= 16) {
         const int rc = cbq_frag_linear(x, true, packed, codebook, out, T, M, K, C, bits, workspace,
                                        ws_bytes, stream);
         if (rc >= 0) return rc;
@@ -1351,17 +1350,28 @@ size_t cbq_linear_bf16_workspace(int T, int M, int K)
     return cbq_prefill_ws_bytes(T, M, K);
 }
 
+size_t cbq_linear_bf16_gemm_workspace(int T, int M, int K, int bits)
+{
+    if (T <= 0 || M <= 0 || K <= 0) return 0;
+    return std::max(cbq_prefill_ws_bytes(T, M, K), cbq_frag_ws_bytes(T, M, K, bits, false));
+}
+
 int cbq_linear_bf16_ws(const void *x_bf16, const uint8_t *packed, const float *codebook,
                        void *out_bf16, int T, int M, int K, int C, int bits, void *workspace,
                        size_t ws_bytes, hipStream_t stream)
 {
+    // (64 tokens that the few-token kernel takes go there)
     if (x_bf16 && packed && codebook && out_bf16 && T >= 64 && M > 0 && K > 0 && C > 0 &&
-        bits >= 1 && bits <= 16) {
-        // workspace = [x in fragment order][fp32 split partials]; a smaller one
-        // runs as ck_linear_bf16
-        const int rc = cbq_prefill_bf16((const uint16_t *)x_bf16, packed, codebook,
-                                        (uint16_t *)out_bf16, T, M, K, C, bits, stream, workspace,
-                                        ws_bytes);
+        bits >= 1 && bits <= 16 && (T > 64 || K % 128 != 0)) {
+        // a workspace of cbq_linear_bf16_gemm_workspace: decode first; of
+        // cbq_linear_bf16_workspace: [x in fragment order][fp32 split
+        // partials] of the fused kernel; a smaller one runs as ck_linear_bf16
+        int rc = cbq_frag_linear(x_bf16, false, packed, codebook, out_bf16, T, M, K, C, bits,
+                                 workspace, ws_bytes, stream);
+        if (rc < 0)
+            rc = cbq_prefill_bf16((const uint16_t *)x_bf16, packed, codebook,
+                                  (uint16_t *)out_bf16, T, M, K, C, bits, stream, workspace,
+                                  ws_bytes);
         if (rc >= 0) return rc;
     }
     return ck_linear_bf16(x_bf16, packed, codebook, out_bf16, T, M, K, C, bits, stream);

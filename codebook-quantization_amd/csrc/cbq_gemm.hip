@@ -27,6 +27,9 @@
 
 #include <algorithm>
 
+// Estimated time of the fused bf16 kernel with its workspace (cbq_prefill.hip).
+float cbq_prefill_us(int T, int M, int K);
+
 namespace {
 
 constexpr int kGBlock = 512;                   // GEMM: 8 waves, two per SIMD
@@ -36,13 +39,15 @@ constexpr int kPrepBlocks = 5;                 // prep blocks per CU (30 KiB of 
 constexpr int kPrepGroups = 8;                 // column groups (of 32) per W prep tile
 constexpr size_t kFrag = 1024;                 // bytes of one fragment
 constexpr size_t kSlabBytes = (size_t)384 << 20;
-// fp32 x: the accumulators are added to totals and cleared every 48 MFMAs.
-// An MFMA rounds its accumulator; one chain of 3 K / 32 roundings at the
-// magnitude of the whole sum left rel-L2 6.2e-7 at K = 4096 and 1.2e-6 at
-// 12288 against 64 bits (the fp32 matrix cores: 4.1e-7 and 7.0e-7 at 512
-// tokens); the short chains leave 2.5e-7 at every K, for one addition per
-// accumulator and 48 MFMAs (T = 512, 4096 x 12288: 130 -> 142 us).
-constexpr int kFoldSteps = 16;                 // column groups (even)
+// fp32 x: the accumulators are added to totals and cleared every 4, 8 or 16
+// column groups (fold_groups).  An MFMA rounds its accumulator; one chain of
+// 3 K / 32 roundings at the magnitude of the whole sum left rel-L2 6.2e-7 at
+// K = 4096 and 1.2e-6 at 12288 against 64 bits (the fp32 matrix cores: 4.1e-7
+// and 7.0e-7 at 512 tokens).  With a fold of f groups of n the variance goes
+// as 3 f / 2 (the chains) + n / (2 f) (the totals), least at f = sqrt(n / 3):
+// 1.8e-7 at K = 2048, 2.5e-7 at 12288, for one addition per accumulator and
+// 3 f MFMAs (T = 512, 4096 x 12288: 130 -> 142 us at f = 16).
+int fold_groups(int n) { return n < 96 ? 4 : n < 400 ? 8 : 16; }
 constexpr int kHeader = 256;                   // workspace header: the W part count
 
 typedef unsigned short g_u16x2 __attribute__((ext_vector_type(2)));
@@ -311,6 +316,9 @@ template <int NP_, int TB_, int MB_, int WT_, int WM_, int NST_> struct GemmCfg 
 // The K loop's stages for WP parts of W: one column group, all its parts.
 template <class C, int WP> struct GemmStage {
     static constexpr int NST = WP == 1 ? C::NST : 2;
+    // stages between a buffer's last read and its reuse: 1 leaves the reads in
+    // flight over the barrier, at the price of a stage of LDS
+    static constexpr int LAG = NST >= 4 ? 1 : 0;
     static constexpr int PIECES = C::NA * C::NP + C::NB * WP;
     static constexpr int PL = (PIECES + kGWaves - 1) / kGWaves;   // copies per wave and stage
     static constexpr int BYTES = PIECES * (int)kFrag;
@@ -331,6 +339,7 @@ struct GemmArgs {
     float *part;            // split-K partials [S][tiles] in fragment order
     const void *x;          // the caller's x (non-finite codebooks only)
     int T, M, ldo, G, nT, nM, S;
+    int fold;               // column groups per chain (even)
 };
 
 // One fragment (1 KiB, lane l's 16 bytes at + 16 l) from global memory to LDS
@@ -346,11 +355,14 @@ __device__ __forceinline__ void lds_copy_frag(uint32_t dst, const uint8_t *src, 
                  :: "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(lane16), "s"(q) : "m0");
 }
 
-// The wave's loads but the newest N have landed in LDS and its LDS reads are
-// done; then the block's barrier: every wave's.
-template <int N> __device__ __forceinline__ void stage_barrier()
+// The wave's copies but the newest N have landed in LDS (READS: and its LDS
+// reads are done); then the block's barrier: every wave's.
+template <int N, bool READS> __device__ __forceinline__ void stage_barrier()
 {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
+    if constexpr (READS)
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
+    else
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(N) : "memory");
 }
 
 __device__ __forceinline__ uint32_t bf16_pair(float a, float b)
@@ -482,6 +494,7 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
     auto all = [&](auto WPc) {
         using St = GemmStage<Cfg, decltype(WPc)::value>;
         constexpr int WP = decltype(WPc)::value, NST = St::NST, PL = St::PL, NS = St::NS;
+        constexpr int LAG = St::LAG;
         constexpr int STAGE = St::BYTES;
         // This wave's pieces of a stage: piece p goes to LDS offset p KiB,
         // the W fragments first (part by part), then x's.
@@ -525,10 +538,13 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
                 f[j] = *(const cbq_u32x4 *)(rdb + buf + (j + p * Cfg::NB) * (int)kFrag);
         };
         uint32_t cur = 0;                                   // LDS offset of the running stage
+        uint32_t old = (NST - 1) * STAGE;                   // and of the one before it
         // One stage whose first fragments are in fa[P0] / fb[Q0]: the next
-        // product's fragments are read while the current one runs; before
-        // the last product's MFMAs the stage is fully read, so the barrier
-        // frees its LDS for the stage NST ahead and publishes the next.
+        // product's fragments are read while the current one runs.  Before
+        // the last product's MFMAs every wave has read the stage (LAG 0:
+        // waited for here) or at least the one before it, whose MFMAs have
+        // been issued (LAG 1), so the barrier frees that LDS for the next
+        // copies and publishes the next stage.
         auto stage = [&](auto P0, auto Q0) {
             constexpr int p0 = decltype(P0)::value, q0 = decltype(Q0)::value;
 #pragma unroll
@@ -543,8 +559,9 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
                         reads += MB;
                     }
                 } else {
-                    stage_barrier<(NST - 2) * PL>();
-                    issue(cur);
+                    stage_barrier<(NST - 2 - LAG) * PL, LAG == 0>();
+                    issue(LAG ? old : cur);
+                    old = cur;
                     cur = cur + STAGE == NST * STAGE ? 0u : cur + STAGE;
                     read_a(cur, 0, fa[NP > 1 ? k ^ 1 : p0 ^ 1]);
                     read_b(cur, 0, fb[q ^ 1]);
@@ -567,12 +584,12 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
         constexpr int P1 = NP > 1 ? NS & 1 : 1, Q1 = WP & 1;
         const std::integral_constant<int, 0> I0{};
 #pragma unroll
-        for (int i = 0; i < NST; i++) issue(i * STAGE);
-        stage_barrier<(NST - 1) * PL>();
+        for (int i = 0; i < NST - LAG; i++) issue(i * STAGE);
+        stage_barrier<(NST - 1 - LAG) * PL, true>();
         read_a(0, 0, fa[0]);
         read_b(0, 0, fb[0]);
         for (int s = 0; s < n;) {
-            const int e = FOLD ? min(n, s + kFoldSteps * 3 / NS) : n;
+            const int e = FOLD ? min(n, s + a.fold) : n;
             for (; s + 2 <= e; s += 2) {
                 stage(I0, I0);
                 stage(std::integral_constant<int, P1>{}, std::integral_constant<int, Q1>{});
@@ -671,12 +688,12 @@ __global__ __launch_bounds__(256) void frag_reduce_kernel(GemmArgs a, int TB, in
 
 // Block tiles (tokens x features), largest first: x parts, TB, MB, WT, WM, stages
 using Gemm1a = GemmCfg<1, 8, 4, 2, 4, 4>;      // 256 x 256
-using Gemm1b = GemmCfg<1, 4, 4, 4, 2, 4>;      // 256 x 128
+using Gemm1b = GemmCfg<1, 4, 4, 4, 2, 5>;      // 256 x 128
 using Gemm1c = GemmCfg<1, 4, 2, 2, 4, 4>;      // 128 x 128
 using Gemm1d = GemmCfg<1, 2, 2, 2, 4, 4>;      // 64 x 128
-using Gemm1e = GemmCfg<1, 4, 6, 4, 2, 4>;      // 256 x 192
+using Gemm1e = GemmCfg<1, 4, 6, 4, 2, 5>;      // 256 x 192
 using Gemm3a = GemmCfg<3, 4, 4, 4, 2, 2>;      // 256 x 128
-using Gemm3b = GemmCfg<3, 4, 4, 2, 4, 3>;      // 128 x 256
+using Gemm3b = GemmCfg<3, 4, 4, 2, 4, 4>;      // 128 x 256
 using Gemm3c = GemmCfg<3, 4, 2, 2, 4, 4>;      // 128 x 128
 using Gemm3d = GemmCfg<3, 2, 4, 2, 4, 4>;      // 64 x 256
 using Gemm3e = GemmCfg<3, 2, 2, 2, 4, 4>;      // 64 x 128
@@ -692,16 +709,17 @@ template <class C> constexpr GemmShape shape_of(float step)
 constexpr int kShapes = 5;
 // step: a launch of whole rounds at K = 4096 (T = 2048 x M = 8192 for one x
 // part, T = 1024 x M = 8192 for three), time / rounds / 128
-const GemmShape kShape1[kShapes] = {shape_of<Gemm1a>(0.84f), shape_of<Gemm1b>(0.51f),
-                                    shape_of<Gemm1c>(0.27f), shape_of<Gemm1d>(0.19f),
-                                    shape_of<Gemm1e>(0.72f)};
+const GemmShape kShape1[kShapes] = {shape_of<Gemm1a>(0.86f), shape_of<Gemm1b>(0.49f),
+                                    shape_of<Gemm1c>(0.26f), shape_of<Gemm1d>(0.19f),
+                                    shape_of<Gemm1e>(0.66f)};
 const GemmShape kShape3[kShapes] = {shape_of<Gemm3a>(1.45f), shape_of<Gemm3b>(1.37f),
-                                    shape_of<Gemm3c>(0.85f), shape_of<Gemm3d>(0.78f),
-                                    shape_of<Gemm3e>(0.42f)};
+                                    shape_of<Gemm3c>(0.82f), shape_of<Gemm3d>(0.76f),
+                                    shape_of<Gemm3e>(0.40f)};
 
 struct GemmPlan {
     int shape, S;
     int rows;               // rows per slab (a multiple of 256, or all M)
+    float us;               // estimated time of the GEMM over all slabs
 };
 
 template <class C>
@@ -799,6 +817,7 @@ GemmPlan gemm_plan(int T, int M, int K, int NP)
                 best = t;
                 p.shape = i;
                 p.S = S;
+                p.us = t * slabs;
             }
         }
     }
@@ -822,6 +841,7 @@ int frag_linear(int NP, const void *x, const uint32_t *words, const float *cb, v
     a.ldo = M;
     a.G = K >> 5;
     a.S = p.S;
+    a.fold = fold_groups((a.G + p.S - 1) / p.S);
     for (int r0 = 0; r0 < M; r0 += p.rows) {
         a.M = std::min(p.rows, M - r0);
         a.out = (uint8_t *)out + (size_t)r0 * (NP == 3 ? 4 : 2);
@@ -833,17 +853,36 @@ int frag_linear(int NP, const void *x, const uint32_t *words, const float *cb, v
     return CK_SUCCESS;
 }
 
-bool frag_shape(int T, int M, int K) { return T >= 64 && M > 0 && K > 0 && K % 32 == 0; }
+// Below 33 tokens of fp32 (65 of bf16) the few-token kernels of cbq_tiny.hip
+// read the weights in place: T = 32 fp32, 12288 x 4096: 52 us against 66 here;
+// T = 48: 77 against 68.
+bool frag_shape(int T, int M, int K, bool f32)
+{
+    return T >= (f32 ? 33 : 64) && M > 0 && K > 0 && K % 32 == 0;
+}
 
 }  // namespace
 
 // Workspace bytes of the fragment GEMM for fp32 (f32) or bf16 x; 0: the shape
-// does not take it.
-size_t cbq_frag_ws_bytes(int T, int M, int K, bool f32)
+// does not take it.  bf16 x has the fused kernel of cbq_prefill.hip beside
+// it, which reads the index stream alone: decoding first pays unless the
+// matrix is large against the tokens and K long (T = 512: 4096 x 12288 111
+// against 97 us fused, 12288 x 4096 100 / 100, 4096 x 4096 51 / 62; T = 2048,
+// 12288 x 4096: 221 / 263), so the smaller estimate is taken: 13-bit indices
+// read and fragments written at 4.8 TB/s, two launches, the GEMM's plan.
+// 8-bit codebooks are taken to be fp32 values (two parts of W: T = 512,
+// 4096 x 4096: 82 against 62 us fused).
+size_t cbq_frag_ws_bytes(int T, int M, int K, int bits, bool f32)
 {
-    if (!frag_shape(T, M, K)) return 0;
+    if (!frag_shape(T, M, K, f32)) return 0;
     const int NP = f32 ? 3 : 1;
     const GemmPlan p = gemm_plan(T, M, K, NP);
+    if (!f32) {
+        const bool two = bits == 8;
+        const float prep = (float)M * (float)K * (two ? 5.f : 3.6f) / 4.8e6f;
+        const float fused = cbq_prefill_us(T, M, K);
+        if (fused > 0.f && prep + 6.f + p.us * (two ? 1.9f : 1.f) > fused) return 0;
+    }
     return kHeader + round256(x_bytes(T, K, NP)) + round256(w_bytes(p.rows, K, NP)) +
            part_bytes(p, T, NP);
 }
@@ -854,7 +893,7 @@ int cbq_frag_linear(const void *x, bool f32, const uint8_t *packed, const float 
                     int T, int M, int K, int C, int bits, void *ws, size_t ws_bytes,
                     hipStream_t st)
 {
-    const size_t need = cbq_frag_ws_bytes(T, M, K, f32);
+    const size_t need = cbq_frag_ws_bytes(T, M, K, bits, f32);
     if (!need || !ws || ws_bytes < need || (((uintptr_t)ws | (uintptr_t)x) & 15) != 0 ||
         ((uintptr_t)packed & 3) != 0)
         return -1;

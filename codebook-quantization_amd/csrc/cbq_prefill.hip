@@ -650,6 +650,28 @@ static bool prefill_takes(int T, int M, int K, int bits)
            (uint64_t)M * (K / kPK) * bits < (1ull << 30);   // index words within one 4 GiB buffer
 }
 
+// Estimated microseconds of a call with the workspace (0: not taken).  A
+// launch costs about 25 us beside its K steps (x copy, codebook staging,
+// prologue, epilogue, gaps), a K step 0.94 us with all eight waves
+// multiplying and 0.77 with one, and the partials of the tokens in use are
+// written and read at about 5 TB/s.  Against measurements (us, estimate /
+// measured): T = 512 4096 x 12288 97 / 96, 12288 x 4096 105 / 100,
+// 4096 x 4096 67 / 62; T = 2048 12288 x 4096 257 / 263.
+float cbq_prefill_us(int T, int M, int K)
+{
+    if (!prefill_shape(T, M, K)) return 0.f;
+    const PrefillPlan p = prefill_plan(T, M, K);
+    const int cus = cbq_num_cus(), G = K / kPK, waves = (std::min(T, kPT) + kWT - 1) / kWT;
+    const float step = 0.75f + 0.024f * (float)waves;
+    const float used = (float)T / (float)(p.nT * kPT);
+    float us = 0.f;
+    if (p.full > 0) us += 25.f + (float)((p.full + cus - 1) / cus * G) * step;
+    if (p.S > 1)
+        us += 25.f + (float)((G + p.S - 1) / p.S) * step +
+              (float)prefill_partial_bytes(p) * used * 4e-7f;
+    return us;
+}
+
 // Workspace bytes of the MFMA prefill with a caller workspace: x in fragment
 // order, then the split partials (0: the shape does not take this path).
 size_t cbq_prefill_ws_bytes(int T, int M, int K)

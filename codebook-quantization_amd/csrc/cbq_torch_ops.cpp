@@ -71,9 +71,8 @@ at::Tensor linear(const at::Tensor &x, const at::Tensor &packed, const at::Tenso
     const hipStream_t st = current_stream(x);
     const bool bf16 = x.scalar_type() == at::kBFloat16;
     // batched tokens: MFMA path with its workspace from torch's allocator
-    const size_t nws = T < 64 ? 0
-                       : bf16 ? cbq_linear_bf16_workspace((int)T, (int)M, (int)K)
-                              : cbq_linear_f32_workspace((int)T, (int)M, (int)K);
+    const size_t nws = bf16 ? cbq_linear_bf16_gemm_workspace((int)T, (int)M, (int)K, (int)bits)
+                            : cbq_linear_f32_workspace((int)T, (int)M, (int)K);
     at::Tensor ws;
     if (nws) ws = at::empty({(int64_t)((nws + 255) / 256 * 256)}, x.options().dtype(at::kByte));
     int rc;

@@ -499,8 +499,8 @@ def from_synthetic(cfg: DecoderConfig, tensors: Dict[str, object], device="cuda"
             x = x.reshape(-1, K).contiguous()
             T = x.shape[0]
             out = torch.empty(T, M, device=dev)
-            # a prompt (T >= 64) may split K: fp32 partials in a torch workspace
-            nws = int(lib.cbq_linear_f32_workspace(T, M, K)) if T >= 64 else 0
+            # a prompt's decoded fragments and partials: a torch workspace
+            nws = int(lib.cbq_linear_f32_workspace(T, M, K))
             ws = torch.empty(max(1, nws // 4), device=dev) if nws else None
             nat.check(lib.cbq_linear_f32_ws(x.data_ptr(), t.packed.data_ptr(),
                                             t.codebook.data_ptr(), out.data_ptr(), T, M, K,

@@ -329,7 +329,7 @@ def linear_from_packed(x: torch.Tensor, packed: torch.Tensor, bits: int, M: int,
     T = x.shape[0]
     C = int(codebook.numel())
     out = torch.empty(T, M, dtype=torch.float32, device=dev)
-    nws = int(lib.cbq_linear_f32_workspace(T, M, K)) if T >= 64 else 0
+    nws = int(lib.cbq_linear_f32_workspace(T, M, K))
     ws = torch.empty(max(1, nws // 4), dtype=torch.float32, device=dev) if nws else None
     nat.check(lib.cbq_linear_f32_ws(x.data_ptr(), packed.data_ptr(), codebook.data_ptr(),
                                     out.data_ptr(), T, M, K, C, bits,

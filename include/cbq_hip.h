@@ -51,7 +51,7 @@ int ck_linear_f32(const float *x, const uint8_t *packed, const float *codebook,
 size_t cbq_linear_f32_workspace(int T, int M, int K);
 
 /* ck_linear_f32 with a caller workspace (>= cbq_linear_f32_workspace bytes,
- * 16-byte aligned): for T >= 64 (K % 32 == 0, widths 8 and 10..14, x 16-byte
+ * 16-byte aligned): for T >= 33 (K % 32 == 0, widths 8 and 10..14, x 16-byte
  * aligned) x (three exact bf16 parts) and the weights are first written there
  * in MFMA fragment order, the weights in slabs of at most 384 MiB, and
  * multiplied on the bf16 matrix cores with fp32 accumulation; K is split
@@ -88,6 +88,12 @@ int ck_linear_bf16(const void *x_bf16, const uint8_t *packed, const float *codeb
  * copy of x in MFMA fragment order, plus fp32 partials when K is split (0:
  * the shape does not take the MFMA path).  No counterpart in the reference. */
 size_t cbq_linear_bf16_workspace(int T, int M, int K);
+
+/* Workspace bytes with which cbq_linear_bf16_ws takes the fastest path it has
+ * for the shape: the decode-first GEMM of cbq_linear_f32_ws where that wins
+ * (x as one bf16 part), else cbq_linear_bf16_workspace.  No counterpart in
+ * the reference. */
+size_t cbq_linear_bf16_gemm_workspace(int T, int M, int K, int bits);
 
 /* ck_linear_bf16 with a caller workspace (>= cbq_linear_bf16_workspace
  * bytes, 256-byte aligned).  For T >= 64 on the MFMA path x is first copied

@@ -47,12 +47,25 @@ def _run_f32(cuda, x, packed, cb, M, K, bits):
     return out
 
 
+def _run_bf16(cuda, x, packed, cb, M, K, bits):
+    lib = nat.load()
+    T = x.shape[0]
+    n = int(lib.cbq_linear_bf16_gemm_workspace(T, M, K, bits))
+    ws = torch.full((max(n, 16),), 0xFF, dtype=torch.uint8, device=cuda)
+    out = torch.full((T, M), float("nan"), dtype=torch.bfloat16, device=cuda)
+    nat.check(lib.cbq_linear_bf16_ws(x.data_ptr(), packed.data_ptr(), cb.data_ptr(),
+                                     out.data_ptr(), T, M, K, cb.numel(), bits, ws.data_ptr(), n,
+                                     nat.stream_ptr(cuda)), "cbq_linear_bf16_ws")
+    return out
+
+
 def _rel(y, ref):
     return float((y.double() - ref).norm() / ref.norm())
 
 
 @pytest.mark.parametrize("T,M,K,bits", [
     (64, 1, 32, 13),            # one column group, one row
+    (33, 4096, 2048, 13), (48, 31, 96, 12),
     (65, 33, 64, 12),           # a row past a superblock, a token past a tile
     (127, 257, 96, 14), (129, 300, 4064, 13), (192, 520, 288, 11), (257, 1000, 1056, 10),
     (64, 4096, 4096, 13), (300, 2048, 2080, 8), (1030, 3000, 544, 13)])
@@ -123,3 +136,24 @@ def test_f32_graph(cuda):
         eager = _run_f32(cuda, x, packed, cb, M, K, bits)
         graph.replay()
         assert torch.equal(out, eager)
+
+
+@pytest.mark.parametrize("T,M,K,bits", [
+    (17, 33, 128, 13), (32, 1000, 4224, 14), (33, 16, 256, 12), (48, 300, 1152, 13),
+    (49, 12288, 128, 10), (64, 520, 2048, 16), (64, 4100, 1024, 13),     # few-token kernel
+    (63, 70, 96, 13),                                                    # refused by it
+    (65, 33, 64, 12), (127, 257, 96, 14), (129, 300, 4064, 13), (257, 1000, 1056, 10),
+    (300, 2048, 2080, 8), (700, 1030, 544, 11), (1030, 3000, 544, 13), (2050, 520, 96, 13)])
+@pytest.mark.parametrize("kind", ["bf16", "fp32"])
+def test_bf16_edges(cuda, T, M, K, bits, kind):
+    """bf16 x: within the rounding of a bf16 output (2^-9 at most, 1.7e-3 in
+    the 2-norm for random values)."""
+    print(f"bf16 {kind} T{T} M{M} K{K} bits{bits}", flush=True)
+    packed, cb, w = _matrix(cuda, M, K, bits, kind, T + M)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn(T, K, device=cuda, generator=g).bfloat16()
+    y, ref = _run_bf16(cuda, x, packed, cb, M, K, bits), x.double() @ w.T
+    assert _rel(y, ref) <= 2.0 ** -9
+    # against one rounding of the exact value: at most one step apart
+    near = ref.bfloat16().double()
+    assert float(((y.double() - near).abs() <= 2.0 ** -7 * near.abs() + 1e-30).double().mean()) > 0.99
