@@ -101,6 +101,9 @@ SIGNATURES = {
     "cbq_split_linear_fewtok_f32": (_i, [_vp, _i, _i, _vp, _vp, _vp, _i, _vp, ctypes.c_size_t,
                                          _vp]),
     "cbq_split_fewtok_ws_bytes": (ctypes.c_size_t, [_i]),
+    "cbq_split_linear_gemm": (_i, [_vp, _i, _i, ctypes.POINTER(SplitMatrix), _vp, _i, _i, _vp,
+                                   ctypes.c_size_t, _vp]),
+    "cbq_split_linear_gemm_ws_bytes": (ctypes.c_size_t, [_i, _i, _i, _i]),
     "cbq_split_pack": (_i, [_vp, _i64, _vp, _vp, _i, _vp, _vp, _vp, _vp]),
     "cbq_split_linear_f32": (_i, [_vp, _vp, _vp, _i, ctypes.c_float, _i, _vp, _vp, _vp, _i,
                                   _vp]),

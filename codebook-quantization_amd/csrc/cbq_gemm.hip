@@ -333,12 +333,13 @@ template <class C, int WP> struct GemmStage {
 
 struct GemmArgs {
     const uint8_t *xf;      // [T / 16][G][NP] fragments
-    const uint8_t *wf;      // [M / 16][NW][G] fragments of the slab
+    const uint8_t *wf;      // [M / 16][nw][G] fragments of the slab
     const int *flag;        // W parts in use; 0: a non-finite codebook value
     void *out;              // out + slab offset, row stride ldo
     float *part;            // split-K partials [S][tiles] in fragment order
     const void *x;          // the caller's x (non-finite codebooks only)
     int T, M, ldo, G, nT, nM, S;
+    int nw;                 // W parts the slab has room for
     int fold;               // column groups per chain (even)
 };
 
@@ -422,7 +423,7 @@ __device__ float scalar_dot(const GemmArgs &a, int t, int m)
 {
     float s = 0.f;
     const int mm = m & 31;
-    const uint8_t *w0 = a.wf + (size_t)((m >> 5) * 2 + frag_of(mm)) * Cfg::NW * a.G * kFrag +
+    const uint8_t *w0 = a.wf + (size_t)((m >> 5) * 2 + frag_of(mm)) * a.nw * a.G * kFrag +
                         frag_row(mm) * 16;
     for (int k = 0; k < a.G * 32; k++) {
         float w = 0.f;
@@ -510,7 +511,7 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
             step[i] = (uint32_t)kFrag * (q >= 0 ? NP : 1);
             base[i] =
                 q >= 0 ? a.xf + ((size_t)min((t0 >> 4) + q % Cfg::NA, nTB - 1) * a.G * NP + q / Cfg::NA) * kFrag
-                       : a.wf + ((size_t)min((m0 >> 4) + p % Cfg::NB, nMB - 1) * Cfg::NW + p / Cfg::NB) *
+                       : a.wf + ((size_t)min((m0 >> 4) + p % Cfg::NB, nMB - 1) * a.nw + p / Cfg::NB) *
                                     a.G * kFrag;
         }
         const uint32_t lane16 = lane * 16;
@@ -777,10 +778,12 @@ int launch_prep(int NP, const void *x, uint8_t *xf, int T, int K, bool with_x,
 
 size_t round256(size_t n) { return (n + 255) & ~(size_t)255; }
 size_t x_bytes(int T, int K, int NP) { return (size_t)((T + 15) >> 4) * (K >> 5) * NP * kFrag; }
-size_t w_bytes(int rows, int K, int NP)
+size_t w_bytes(int rows, int K, int nw)
 {
-    return (size_t)((rows + 31) >> 5) * 2 * (K >> 5) * (NP == 3 ? 3 : 2) * kFrag;
+    return (size_t)((rows + 31) >> 5) * 2 * (K >> 5) * nw * kFrag;
 }
+// W parts a fixed-width slab has room for
+int w_parts(int NP) { return NP == 3 ? 3 : 2; }
 size_t part_bytes(const GemmPlan &p, int T, int NP)
 {
     if (p.S <= 1) return 0;
@@ -793,10 +796,10 @@ size_t part_bytes(const GemmPlan &p, int T, int NP)
 // groups of a block x the shape's step + 5 us of prologue and epilogue), plus
 // the partials' write and read at about 5 TB/s and 3 us for the extra launch.
 // A split holds at least 8 column groups (a shorter chain is all prologue).
-GemmPlan gemm_plan(int T, int M, int K, int NP)
+GemmPlan gemm_plan(int T, int M, int K, int NP, int nw)
 {
     GemmPlan p;
-    const size_t row = (size_t)(K >> 5) * (NP == 3 ? 3 : 2) * kFrag / 16;
+    const size_t row = (size_t)(K >> 5) * nw * kFrag / 16;
     const int fit = (int)std::max<size_t>(256, kSlabBytes / row / 256 * 256);
     const int slabs = (M + fit - 1) / fit;
     p.rows = slabs == 1 ? M : ((M + slabs - 1) / slabs + 255) / 256 * 256;
@@ -824,33 +827,61 @@ GemmPlan gemm_plan(int T, int M, int K, int NP)
     return p;
 }
 
+// Workspace: header (W part count), x fragments, a slab of W fragments, the
+// split-K partials.
+GemmArgs gemm_args(const GemmPlan &p, int NP, int nw, const void *x, int T, int M, int K,
+                   uint8_t *ws)
+{
+    GemmArgs a;
+    uint8_t *const wf = ws + kHeader + round256(x_bytes(T, K, NP));
+    a.xf = ws + kHeader;
+    a.wf = wf;
+    a.flag = (const int *)ws;
+    a.out = nullptr;
+    a.part = (float *)(wf + round256(w_bytes(p.rows, K, nw)));
+    a.x = x;
+    a.T = T;
+    a.M = 0;
+    a.ldo = M;
+    a.G = K >> 5;
+    a.S = p.S;
+    a.nT = a.nM = 0;
+    a.nw = nw;
+    a.fold = fold_groups((a.G + p.S - 1) / p.S);
+    return a;
+}
+
+size_t gemm_ws_bytes(const GemmPlan &p, int NP, int nw, int T, int K)
+{
+    return kHeader + round256(x_bytes(T, K, NP)) + round256(w_bytes(p.rows, K, nw)) +
+           part_bytes(p, T, NP);
+}
+
 // out [T][M] = x @ W^T over the slabs of W; BITS-wide indices.
 template <int BITS>
 int frag_linear(int NP, const void *x, const uint32_t *words, const float *cb, void *out, int T,
                 int M, int K, int C, uint8_t *ws, hipStream_t st)
 {
-    const GemmPlan p = gemm_plan(T, M, K, NP);
-    uint8_t *const xf = ws + kHeader, *const wf = xf + round256(x_bytes(T, K, NP));
-    GemmArgs a;
-    a.xf = xf;
-    a.wf = wf;
-    a.flag = (const int *)ws;
-    a.part = (float *)(wf + round256(w_bytes(p.rows, K, NP)));
-    a.x = x;
-    a.T = T;
-    a.ldo = M;
-    a.G = K >> 5;
-    a.S = p.S;
-    a.fold = fold_groups((a.G + p.S - 1) / p.S);
+    const GemmPlan p = gemm_plan(T, M, K, NP, w_parts(NP));
+    GemmArgs a = gemm_args(p, NP, w_parts(NP), x, T, M, K, ws);
     for (int r0 = 0; r0 < M; r0 += p.rows) {
         a.M = std::min(p.rows, M - r0);
         a.out = (uint8_t *)out + (size_t)r0 * (NP == 3 ? 4 : 2);
-        int rc = launch_prep<BITS>(NP, x, xf, T, K, r0 == 0, words, cb, C, wf, (int *)ws, r0, a.M,
-                                   st);
+        int rc = launch_prep<BITS>(NP, x, (uint8_t *)a.xf, T, K, r0 == 0, words, cb, C,
+                                   (uint8_t *)a.wf, (int *)ws, r0, a.M, st);
         if (!rc) rc = launch_gemm(NP, p.shape, a, st);
         if (rc) return rc;
     }
     return CK_SUCCESS;
+}
+
+// x alone (the split format's matrices are decoded by cbq_split.hip)
+template <int NP>
+__global__ __launch_bounds__(kPBlock) void frag_x_kernel(const void *__restrict__ x,
+                                                         uint8_t *__restrict__ xf, int T, int K)
+{
+    prep_x<NP>(x, xf, T, K, (int64_t)blockIdx.x * (kPBlock / CBQ_WAVE) + threadIdx.x / CBQ_WAVE,
+               (int64_t)((T + 15) >> 4) * (K >> 5), (int64_t)gridDim.x * (kPBlock / CBQ_WAVE));
 }
 
 // Below 33 tokens of fp32 (65 of bf16) the few-token kernels of cbq_tiny.hip
@@ -876,15 +907,14 @@ size_t cbq_frag_ws_bytes(int T, int M, int K, int bits, bool f32)
 {
     if (!frag_shape(T, M, K, f32)) return 0;
     const int NP = f32 ? 3 : 1;
-    const GemmPlan p = gemm_plan(T, M, K, NP);
+    const GemmPlan p = gemm_plan(T, M, K, NP, w_parts(NP));
     if (!f32) {
         const bool two = bits == 8;
         const float prep = (float)M * (float)K * (two ? 5.f : 3.6f) / 4.8e6f;
         const float fused = cbq_prefill_us(T, M, K);
         if (fused > 0.f && prep + 6.f + p.us * (two ? 1.9f : 1.f) > fused) return 0;
     }
-    return kHeader + round256(x_bytes(T, K, NP)) + round256(w_bytes(p.rows, K, NP)) +
-           part_bytes(p, T, NP);
+    return gemm_ws_bytes(p, NP, w_parts(NP), T, K);
 }
 
 // The batched linear over fixed-width indices with a workspace of at least
@@ -906,4 +936,55 @@ int cbq_frag_linear(const void *x, bool f32, const uint8_t *packed, const float 
     default: return -1;
     }
 #undef CBQ_FL
+}
+
+// ---- split-format matrices -------------------------------------------------------
+
+// cbq_split.hip: rows [row0, row0 + M) of the matrix as fragments
+// [M / 16][1][G] at wf, and the part count 1 at flag.
+int cbq_split_frags(const cbq_split_matrix *m, int row0, int M, int K, uint8_t *wf, int *flag,
+                    hipStream_t st);
+
+static bool split_gemm_shape(int T, int M, int K)
+{
+    return T >= 1 && M > 0 && K > 0 && K % 1024 == 0 && (int64_t)M * K % 4096 == 0;
+}
+
+extern "C" size_t cbq_split_linear_gemm_ws_bytes(int T, int M, int K, int x_bf16)
+{
+    if (!split_gemm_shape(T, M, K)) return 0;
+    const int NP = x_bf16 ? 1 : 3;
+    return gemm_ws_bytes(gemm_plan(T, M, K, NP, 1), NP, 1, T, K);
+}
+
+extern "C" int cbq_split_linear_gemm(const void *x, int x_bf16, int T, const cbq_split_matrix *m,
+                                     void *out, int M, int K, void *ws, size_t ws_bytes,
+                                     hipStream_t stream)
+{
+    if (!x || !m || !out || !ws || !split_gemm_shape(T, M, K) || !m->cwords || !m->row_off ||
+        !m->raw || !m->lut || m->n_chunks != (int64_t)M * K / 4096)
+        return CK_ERR_ARG;
+    if ((((uintptr_t)x | (uintptr_t)ws | (uintptr_t)m->cwords | (uintptr_t)m->raw |
+          (uintptr_t)m->lut) & 15) != 0)
+        return CK_ERR_ARG;
+    if (ws_bytes < cbq_split_linear_gemm_ws_bytes(T, M, K, x_bf16)) return CK_ERR_ARG;
+    const int NP = x_bf16 ? 1 : 3;
+    const GemmPlan p = gemm_plan(T, M, K, NP, 1);
+    GemmArgs a = gemm_args(p, NP, 1, x, T, M, K, (uint8_t *)ws);
+    const int64_t units = (int64_t)((T + 15) >> 4) * (K >> 5);
+    const int nxb = (int)std::min<int64_t>((units + 3) / 4, kPrepBlocks * cbq_num_cus());
+    if (x_bf16)
+        hipLaunchKernelGGL(frag_x_kernel<1>, dim3(nxb), dim3(kPBlock), 0, stream, x,
+                           (uint8_t *)a.xf, T, K);
+    else
+        hipLaunchKernelGGL(frag_x_kernel<3>, dim3(nxb), dim3(kPBlock), 0, stream, x,
+                           (uint8_t *)a.xf, T, K);
+    int rc = cbq_launch_status("frag_x_kernel");
+    for (int r0 = 0; r0 < M && !rc; r0 += p.rows) {
+        a.M = std::min(p.rows, M - r0);
+        a.out = (uint8_t *)out + (size_t)r0 * (NP == 3 ? 4 : 2);
+        rc = cbq_split_frags(m, r0, a.M, K, (uint8_t *)a.wf, (int *)ws, stream);
+        if (!rc) rc = launch_gemm(NP, p.shape, a, stream);
+    }
+    return rc;
 }

@@ -737,6 +737,161 @@ __global__ __launch_bounds__(kPackWaves * CBQ_WAVE) void split_to_packed_kernel(
     }
 }
 
+// ---- split format -> bf16 MFMA fragments (batched tokens) ------------------------
+//
+// Rows [row0, row0 + M) as 1 KiB fragments of 16 rows x 32 columns (lane l's
+// 16 bytes: fragment row l % 16, columns 8 (l / 16) .. +7), fragment tile t
+// at wf + t * (K / 32) KiB.  Fragment row r of tile t = 2 s + f stands for
+// row 32 s + 8 (r / 4) + 4 f + r % 4 (frag_row of cbq_gemm.hip): four quads
+// of consecutive rows.  K % 1024 == 0, so a quad is K / 1024 whole chunks.
+//
+// Block: 16 waves (one block per CU), each decoding one chunk per item in
+// eight phases of 8 weights per lane, as split_fewtok_kernel does; a phase's
+// 16-byte pieces go to an LDS tile and leave in fragment order, 256
+// contiguous bytes (16 fragment rows) where the item holds all of them.  A
+// lane writing its own pieces would spread every store over 64 lines of
+// other rows' fragments.
+//   - K % 4096 == 0 or 4096 % K == 0 (rpc > 0): a chunk holds rpc rows (1, 2
+//     or 4) and the 16 waves hold every row of rpc tiles over the same
+//     columns.
+//   - otherwise (rpc = 0): wave 4 q + j takes chunk 4 it + j of quad q, and
+//     the pieces of four quads (64 bytes apart) leave together.
+// A chunk past the matrix (the last tile's missing rows) decodes the last
+// chunk instead: its outputs are never stored.
+// Bound: the decode chain (three waves' worth of chunks for 12288 x 4096) and
+// the 2 bytes a weight written.  Measured in place of the transient index
+// stream and its GEMM: T = 300, 4096 x 4096, bf16 x 84 -> 49 us, fp32 x
+// 87 -> 59.
+constexpr int kFgPhase = 16 * CBQ_WAVE * 4;        // words of a phase tile
+
+struct FragGeo {
+    int rpc;      // rows per chunk, 0: chunks straddle rows
+    int cpr;      // items per tile group: chunks per row, or rounds of 4 chunks a quad
+    int per_row;  // sub-blocks per row
+    int units;    // tile groups x cpr
+    int tiles;    // fragment tiles of the slab
+};
+
+__global__ __launch_bounds__(16 * CBQ_WAVE) void split_frag_kernel(SplitSeg S, int64_t n_chunks,
+                                                                   int row0, FragGeo G,
+                                                                   uint8_t *__restrict__ wf,
+                                                                   int *__restrict__ flag)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t
+        s_lds[kSLut + 16 * kSSlotWords + 2 * kFgPhase];
+    uint32_t *const s_ph = s_lds + kSLut + 16 * kSSlotWords;
+    const int tid = threadIdx.x, lane = tid & (CBQ_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / CBQ_WAVE);
+    uint32_t *const s_slot = s_lds + kSLut + wave * kSSlotWords;
+    const int lane_addr =
+        __builtin_amdgcn_readfirstlane(4 * (kSLut + wave * kSSlotWords)) + 4 * lane;
+    if (blockIdx.x == 0 && tid == 0) *flag = 1;
+    for (int i = wave; i < kSLut / (4 * CBQ_WAVE); i += 16)
+        __builtin_amdgcn_global_load_lds(S.lut + i * 4 * CBQ_WAVE + 4 * lane,
+                                         (__attribute__((address_space(3))) void *)(s_lds + i * 4 * CBQ_WAVE),
+                                         16, 0, 0);
+    const int per_row = G.per_row;
+    const int64_t tile_bytes = (int64_t)per_row * 2048;      // K / 32 fragments
+    // waves per tile and quad
+    const int wpt = G.rpc ? 16 / G.rpc : 16, wpq = wpt / 4;
+    const int q = wave % wpt / wpq, j = wave % wpq;
+    const int tpi = 16 / wpt;
+    // this wave's chunk of unit k
+    auto chunk_of = [&](int k) {
+        const int tg = k / G.cpr, it = k - tg * G.cpr;
+        const int tile = tg * tpi + wave / wpt;
+        const int64_t r = row0 + (tile >> 1) * 32 + 8 * q + 4 * (tile & 1);   // quad's first row
+        int64_t c;
+        if (G.rpc == 1) c = (r + j) * G.cpr + it;
+        else if (G.rpc) c = (r + j * G.rpc) / G.rpc;
+        else c = r / 4 * (per_row / 16) + min(4 * it + j, per_row / 16 - 1);
+        return c < n_chunks ? c : n_chunks - 1;
+    };
+    const __attribute__((address_space(4))) uint32_t *const ro =
+        (const __attribute__((address_space(4))) uint32_t *)S.row_off;
+    auto load_item = [&](int k, SplitItem &it, uint32_t &H) {
+        const int64_t c = __builtin_amdgcn_readfirstlane((int)chunk_of(k < G.units ? k : 0));
+        const uint32_t r0 = ro[c];
+        H = ro[c + 1] - r0;
+        H = H < (uint32_t)kSRows ? H : (uint32_t)kSRows;
+        split_load_all(it, S, c, r0, H, lane);
+    };
+    // phase tile slot of (wave w, lane l): the lanes of a store's 16 rows hit
+    // distinct bank groups
+    auto slot = [](int w, int l) { return (w * CBQ_WAVE + (l ^ (w & 15))) * 4; };
+
+    SplitItem A;
+    uint32_t hA = 0;
+    load_item(blockIdx.x, A, hA);
+    __syncthreads();                               // table staged
+    for (int k = blockIdx.x; k < G.units; k += gridDim.x) {
+        // where this thread's piece of every phase comes from and goes to
+        const int tg = k / G.cpr, it = k - tg * G.cpr;
+        int src_w, src_l, tile, sub, fr;
+        bool on;
+        if (G.rpc) {
+            const int n = 1024 / tpi, u = tid % n, r = u & 15, e = r & 3;
+            const int ti = tid / n, rpc = G.rpc;
+            sub = u >> 4;
+            fr = r;
+            src_w = ti * wpt + (r >> 2) * wpq + e / rpc;
+            src_l = (e % rpc) * (CBQ_WAVE / rpc) + sub;
+            sub += rpc == 1 ? it * CBQ_WAVE : 0;
+            tile = tg * tpi + ti;
+            on = tile < G.tiles;
+        } else {
+            const int id = 4 * it + (tid >> 8), l = (tid & 255) >> 2, qq = tid & 3;
+            const int flat = id * CBQ_WAVE + l, e = flat / per_row;
+            src_w = 4 * qq + (tid >> 8);
+            src_l = l;
+            sub = flat - e * per_row;
+            fr = 4 * qq + e;
+            tile = tg;
+            on = id < per_row / 16;
+        }
+        uint8_t *const dst = wf + tile * tile_bytes + (int64_t)sub * 2048 + fr * 16;
+        split_stage_all(A, s_slot, lane);
+        uint32_t raw[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) raw[i] = A.raw[i];
+        load_item(k + gridDim.x, A, hA);
+        uint32_t pos = 30, d1 = 0;                  // as split_decode
+        const char *base = (const char *)s_lds + lane_addr;
+        uint32_t w0 = *(const uint32_t *)(base - 4 * kSSub);
+        uint32_t w1 = *(const uint32_t *)base;
+#pragma unroll
+        for (int p = 0; p < 8; p++) {
+            uint32_t pr[4];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int g = 2 * p + h;
+                const uint32_t w2 = *(const uint32_t *)(base + (d1 + 1) * (4 * kSSub));
+                uint32_t w = __builtin_amdgcn_alignbit(w1, w0, pos);
+#pragma unroll
+                for (int u = 0; u < 4; u += 2) {
+                    const uint32_t e =
+                        *(const uint32_t *)((const char *)s_lds + (w & (4u * kSLut - 4u)));
+                    pr[2 * h + (u >> 1)] = __builtin_amdgcn_perm(
+                        e, raw[g], 0x06000700u | (uint32_t)u | ((uint32_t)(u + 1) << 16));
+                    w >>= (e & 31u);
+                    pos += e;
+                }
+                const uint32_t dn = __builtin_amdgcn_ubfe(pos, 5, 11);
+                w0 = dn != d1 ? w1 : w0;
+                w1 = dn != d1 ? w2 : w1;
+                d1 = dn;
+            }
+            uint32_t *const ph = s_ph + (p & 1) * kFgPhase;
+            *(u4 *)(ph + slot(wave, lane)) = u4{pr[0], pr[1], pr[2], pr[3]};
+            // one barrier a phase: the other tile's pieces were read before
+            // this phase's writes of the next use of it
+            lds_barrier();
+            if (on)
+                *(u4 *)(dst + (p >> 2) * 1024 + (p & 3) * 256) = *(const u4 *)(ph + slot(src_w, src_l));
+        }
+    }
+}
+
 // ---- a few tokens straight from the split format -------------------------------
 //
 // y[t, r] = W[r, :] . x[t, :] for up to 16 tokens on the bf16 matrix cores,
@@ -1200,6 +1355,32 @@ int cbq_split_to_packed(const cbq_split_matrix *m, const uint16_t *inv, int bits
 #undef CBQ_S2P
     return cbq_launch_status("split_to_packed_kernel");
 }
+
+}  // extern "C"
+
+// Rows [row0, row0 + M) of a split matrix as fragments (cbq_gemm.hip).
+int cbq_split_frags(const cbq_split_matrix *m, int row0, int M, int K, uint8_t *wf, int *flag,
+                    hipStream_t st)
+{
+    SplitSeg g = {};
+    g.cwords = m->cwords;
+    g.row_off = m->row_off;
+    g.raw = m->raw;
+    g.lut = m->lut;
+    FragGeo G;
+    G.rpc = K % kSChunk == 0 ? 1 : kSChunk % K == 0 ? kSChunk / K : 0;
+    G.cpr = K % kSChunk == 0 ? K / kSChunk : G.rpc ? 1 : (K / 1024 + 3) / 4;
+    G.per_row = K / kSSub;
+    G.tiles = ((M + 31) >> 5) * 2;
+    const int tpi = G.rpc ? G.rpc : 1;
+    G.units = (G.tiles + tpi - 1) / tpi * G.cpr;
+    const int blocks = std::min(G.units, cbq_num_cus());
+    hipLaunchKernelGGL(split_frag_kernel, dim3(blocks), dim3(16 * CBQ_WAVE), 0, st, g, m->n_chunks,
+                       row0, G, wf, flag);
+    return cbq_launch_status("split_frag_kernel");
+}
+
+extern "C" {
 
 size_t cbq_split_fewtok_ws_bytes(int K) { return K > 0 ? (size_t)K * 96 : 0; }
 

@@ -11,12 +11,13 @@
 //   linear(x, packed, codebook, M, bits) -> out          ck_linear_f32 / ck_linear_bf16
 //   embedding(ids, packed, codebook, vocab, bits, H) -> out     cbq_embedding_f32
 //   split_linear(x, cwords, row_off, raw, lut, M) -> out         cbq_split_linear_f32
+//   split_gemm(x, cwords, row_off, raw, lut, M) -> out       cbq_split_linear_gemm
 //   huff_linear(x, words, chunk_off, sub_len, lut1, lut2, canon, canon_pay,
 //               value_cb, C, stage_words, M) -> out               cbq_huff_linear_f32
 //   huff_embedding(ids, words, ..., vocab, H) -> out              cbq_huff_embedding_f32
 //
 // Outputs are new tensors on the inputs' device; fp32 unless x is bf16
-// (linear only).  A HIP library error raises RuntimeError with the entry
+// (linear and split_gemm).  A HIP library error raises RuntimeError with the entry
 // point's name and return code.
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
@@ -167,6 +168,40 @@ at::Tensor split_linear(const at::Tensor &x, const at::Tensor &cwords, const at:
     return out;
 }
 
+// Batched tokens (fp32 or bf16 x): the matrix decoded to MFMA fragments in a
+// workspace from torch's allocator, then one GEMM.
+at::Tensor split_gemm(const at::Tensor &x, const at::Tensor &cwords, const at::Tensor &row_off,
+                      const at::Tensor &raw, const at::Tensor &lut, int64_t M)
+{
+    TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.size(0) >= 1 && x.is_contiguous() &&
+                    (x.scalar_type() == at::kFloat || x.scalar_type() == at::kBFloat16),
+                "cbq::split_gemm: x must be a contiguous [T, K] float32 or bfloat16 device tensor");
+    for (const auto &p : {std::make_pair(&cwords, "cwords"), std::make_pair(&row_off, "row_off"),
+                          std::make_pair(&raw, "raw"), std::make_pair(&lut, "lut")})
+        check_dev(*p.first, x, p.second);
+    const int64_t T = x.size(0), K = x.size(1);
+    TORCH_CHECK(T < (1ll << 31) && M > 0 && M < (1ll << 31) && K < (1ll << 31) && K % 1024 == 0 &&
+                    (M * K) % 4096 == 0 && row_off.numel() == M * K / 4096 + 1 &&
+                    raw.numel() == M * K && lut.numel() == 16384,
+                "cbq::split_gemm: tensors do not describe a ", M, "x", K,
+                " split matrix with K % 1024 == 0");
+    c10::DeviceGuard guard(x.device());
+    const int bf16 = x.scalar_type() == at::kBFloat16;
+    at::Tensor out = at::empty({T, M}, x.options());
+    cbq_split_matrix m;
+    m.cwords = cptr<uint32_t>(cwords);
+    m.row_off = cptr<uint32_t>(row_off);
+    m.raw = cptr<uint8_t>(raw);
+    m.lut = cptr<uint32_t>(lut);
+    m.n_chunks = M * K / 4096;
+    const size_t nws = cbq_split_linear_gemm_ws_bytes((int)T, (int)M, (int)K, bf16);
+    at::Tensor ws = at::empty({(int64_t)nws}, x.options().dtype(at::kByte));
+    check_rc(cbq_split_linear_gemm(x.data_ptr(), bf16, (int)T, &m, out.data_ptr(), (int)M, (int)K,
+                                   ws.data_ptr(), nws, current_stream(x)),
+             "cbq_split_linear_gemm");
+    return out;
+}
+
 cbq_huff_stream stream_desc(const at::Tensor &ref, const at::Tensor &words,
                             const at::Tensor &chunk_off, const at::Tensor &sub_len,
                             const at::Tensor &lut1, const at::Tensor &lut2,
@@ -275,6 +310,8 @@ TORCH_LIBRARY(cbq, m)
           "-> Tensor");
     m.def("split_linear(Tensor x, Tensor cwords, Tensor row_off, Tensor raw, Tensor lut, "
           "int M) -> Tensor");
+    m.def("split_gemm(Tensor x, Tensor cwords, Tensor row_off, Tensor raw, Tensor lut, "
+          "int M) -> Tensor");
     m.def("huff_linear(Tensor x, Tensor words, Tensor chunk_off, Tensor sub_len, Tensor lut1, "
           "Tensor lut2, Tensor canon, Tensor canon_pay, Tensor? value_cb, int C, "
           "int stage_words, int M) -> Tensor");
@@ -289,6 +326,7 @@ TORCH_LIBRARY_IMPL(cbq, CUDA, m)
     m.impl("linear", &linear);
     m.impl("embedding", &embedding);
     m.impl("split_linear", &split_linear);
+    m.impl("split_gemm", &split_gemm);
     m.impl("huff_linear", &huff_linear);
     m.impl("huff_embedding", &huff_embedding);
 }

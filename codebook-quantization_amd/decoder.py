@@ -565,16 +565,17 @@ def from_synthetic(cfg: DecoderConfig, tensors: Dict[str, object], device="cuda"
 
     def split_linear(sp, M, K, cbt):
         """A split-format matrix: one token on the split GEMV, batched tokens
-        through its transient fixed-width stream.  Captures only the split
-        format, so the tensor's stream can be freed."""
+        through its transient fragments.  Captures only the split format, so
+        the tensor's stream can be freed."""
         inv = inv_of(cbt)
+        finite = bool(torch.isfinite(cbt).all())
         one, sxform = split_fns([sp], [M], K)
 
         def f(x):
             x = x.reshape(-1, K).contiguous()
             if x.shape[0] == 1:
                 return one(x)
-            return split_prefill(sp, inv, x, M, K, cbt)
+            return split_prefill(sp, inv, x, M, K, cbt, finite)
 
         def xform_argmax(x0, x1, mode, ids32, toks, pos, first, out=None, keep=sp):
             """One token, then the greedy pick in the GEMV's epilogue."""

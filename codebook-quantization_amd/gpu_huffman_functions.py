@@ -350,6 +350,21 @@ def huffman_prefill(sym: "SymbolDecoder", x: torch.Tensor, M: int, K: int,
 
 
 FEWTOK_MAX_T = 32       # up to two 16-token launches of the fused kernel
+# From here on the matrix is decoded once to MFMA fragments (split_gemm).  Up
+# to 32 fp32 tokens one or two launches of the fused kernel read it in place:
+# 17 to 32 tokens, 12288 x 4096, 70 us against 68; 33 tokens 143 against 68.
+# bf16 x, widened for the fused kernel, changes over at its second launch
+# (61 us).
+SPLIT_GEMM_MIN_T = {torch.float32: 33, torch.bfloat16: 17}
+
+
+def split_gemm(split, x: torch.Tensor, M: int) -> torch.Tensor:
+    """y [T, M] = x [T, K] @ W^T (fp32, or bf16 in and out) through
+    torch.ops.cbq.split_gemm; finite weights."""
+    x = x.contiguous()
+    if x.data_ptr() % 16:                          # a view into the middle of a buffer
+        x = x.clone()
+    return cbq_ops.load().split_gemm(x, *split[0], M)
 
 
 def split_fewtok_eligible(K: int) -> bool:
@@ -371,8 +386,10 @@ def split_fewtok_eligible(K: int) -> bool:
 
 
 def split_prefill(split, inv: torch.Tensor, x: torch.Tensor, M: int, K: int,
-                  codebook: torch.Tensor) -> torch.Tensor:
-    """y [T, M] for batched fp32 tokens from the split format.  Up to 32
+                  codebook: torch.Tensor, finite: bool = False) -> torch.Tensor:
+    """y [T, M] for batched fp32 tokens from the split format.  From 33 tokens
+    on and finite codebook values (finite=True): decoded to MFMA fragments
+    and multiplied in one GEMM (split_gemm).  Else up to 32
     tokens (and a shape it takes): one fused launch per 16 tokens
     (cbq_split_linear_fewtok_f32), every weight decoded once into LDS and
     multiplied on the matrix cores, no transient buffer.  Otherwise the
@@ -380,6 +397,8 @@ def split_prefill(split, inv: torch.Tensor, x: torch.Tensor, M: int, K: int,
     one table read per two weights) and multiplied by ck_linear_f32's
     kernels."""
     T = int(x.shape[0])
+    if finite and T >= SPLIT_GEMM_MIN_T[torch.float32]:
+        return split_gemm(split, x, M)
     if 1 <= T <= FEWTOK_MAX_T and split_fewtok_eligible(K) and x.data_ptr() % 16 == 0:
         return split_fewtok([split], x, [M], K)[0]
     packed, bits = _packed_for_gemm(split, M * K, int(codebook.numel()), x.device, inv)
@@ -469,8 +488,10 @@ class HuffmanCodebookLinear:
       values, every symbol < C, K % 1024 == 0, whole 4096-symbol chunks): the
       split format alone, ~11.5 bits per weight, built on the device from the
       stream, after which the stream is freed.  One token runs the split
-      GEMV; batched tokens decode it to a transient fixed-width stream for
-      ck_linear_f32's kernels; decode_indices() maps the values back to their
+      GEMV, up to 32 the fused few-token kernel; more are multiplied with the
+      matrix decoded to transient MFMA fragments (bf16 x stays bf16; not for
+      infinite codebook values, which take a transient fixed-width stream
+      and ck_linear_f32's kernels); decode_indices() maps the values back to their
       indices.
     - "stream": the reference stream in device words plus its chunk index
       (~10.8 bits per weight).  Every call runs the fused stream kernels
@@ -513,6 +534,7 @@ class HuffmanCodebookLinear:
         self.split = None
         self.cols = None
         self._inv = None
+        self._finite = bool(np.isfinite(self._cb_np).all())
         if layout in ("auto", "split") and split_eligible(self.M, self.K):
             idx = SymbolDecoder(dev.words, dev.chunk_off, dev.sub_len, self._lengths,
                                 device).indices(self.M * self.K)
@@ -550,6 +572,7 @@ class HuffmanCodebookLinear:
         self.device = cb.device
         self._cb_dev = cb
         self._cb_np = cb.cpu().numpy()
+        self._finite = bool(np.isfinite(self._cb_np).all())
         self._lengths = np.ascontiguousarray(t.lengths, np.uint8)
         self.cols = None
         if isinstance(t, dfm.SplitTensor):
@@ -589,6 +612,11 @@ class HuffmanCodebookLinear:
         if x.shape[-1] != self.K:
             raise ValueError(f"{self.name}: expected last dim {self.K}, got {x.shape[-1]}")
         T = int(x.numel() // self.K)
+        gemm_dtype = torch.bfloat16 if in_dtype == torch.bfloat16 else torch.float32
+        if self.split is not None and self._finite and T >= SPLIT_GEMM_MIN_T[gemm_dtype]:
+            xg = x.reshape(T, self.K).to(gemm_dtype)
+            out = split_gemm(self.split, xg, self.M).reshape(*lead, self.M)
+            return out if out.dtype == in_dtype else out.to(in_dtype)
         xc = x.reshape(T, self.K).to(torch.float32).contiguous()
         st = nat.stream_ptr(self.device)
         if T == 0:

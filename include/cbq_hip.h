@@ -428,6 +428,24 @@ int cbq_split_linear_fewtok_f32(const float *x, int T, int n, const cbq_split_ma
  * counterpart in the reference. */
 size_t cbq_split_fewtok_ws_bytes(int K);
 
+/* y [T, M] = x [T, K] @ W^T for one split-format matrix and any T >= 1 (meant
+ * for more tokens than the few-token kernel takes in one launch): x (fp32 as
+ * three exact bf16 parts, or x_bf16 != 0: bf16) and the decoded weights go to
+ * the workspace in MFMA fragment order, the weights in slabs of at most 384
+ * MiB, and are multiplied on the bf16 matrix cores with fp32 accumulation.
+ * out is fp32 (bf16 for bf16 x).  K % 1024 == 0, M * K a whole number of
+ * chunks, x and ws 16-byte aligned, ws of at least
+ * cbq_split_linear_gemm_ws_bytes; CK_ERR_ARG otherwise.  Weights are finite
+ * (fp32 x: an infinite weight gives NaN where x's lower parts are zero).
+ * Replaces the batched-token path of HuffmanCodebookLinear.__call__
+ * (src/gpu_huffman_functions.py:834-855), which decodes to int32 indices
+ * first. */
+int cbq_split_linear_gemm(const void *x, int x_bf16, int T, const cbq_split_matrix *m, void *out,
+                          int M, int K, void *ws, size_t ws_bytes, hipStream_t stream);
+
+/* Workspace bytes of cbq_split_linear_gemm (0: the shape is not taken). */
+size_t cbq_split_linear_gemm_ws_bytes(int T, int M, int K, int x_bf16);
+
 /* ==== upload helpers ===================================================== */
 
 /* Allocate device memory (hipMalloc) and copy `nbytes` host bytes into it

@@ -157,3 +157,61 @@ def test_bf16_edges(cuda, T, M, K, bits, kind):
     # against one rounding of the exact value: at most one step apart
     near = ref.bfloat16().double()
     assert float(((y.double() - near).abs() <= 2.0 ** -7 * near.abs() + 1e-30).double().mean()) > 0.99
+
+
+def _split_matrix(cuda, M, K, seed):
+    import device_formats as dfm
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    w = (torch.randn(M, K, device=cuda, generator=g) * 0.02).bfloat16()
+    cb, lut = cbb.codebook_from_counts_torch(cbb.counts_torch(w))
+    idx = lut[cbb.patterns_torch(w).reshape(-1).to(torch.int64)]
+    t = dfm.to_split(dfm.encode_huffman("w", idx, cb, (M, K), "mlp_ffn"), idx)
+    assert t is not None
+    return t, w.double()
+
+
+@pytest.mark.parametrize("T,M,K", [
+    (17, 4, 1024), (33, 100, 1024), (64, 2, 2048), (40, 300, 2048), (130, 132, 3072),
+    (17, 1, 4096), (64, 33, 4096), (300, 520, 4096), (20, 68, 5120), (50, 258, 6144),
+    (96, 40, 7168), (70, 37, 8192), (18, 132, 9216), (1, 64, 2048)])
+def test_split_gemm(cuda, T, M, K):
+    """Split-format matrices of every chunk geometry (rows of whole chunks,
+    chunks of whole rows, chunks across rows), rows off every tile: fp32 and
+    bf16 x."""
+    import cbq_ops
+    print(f"split T{T} M{M} K{K}", flush=True)
+    t, w = _split_matrix(cuda, M, K, M + K)
+    x = torch.randn(T, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(T))
+    op = cbq_ops.load().split_gemm
+    y = op(x, *t.keep, M)
+    assert _rel(y, x.double() @ w.T) <= TOL_F32
+    xb = x.bfloat16()
+    yb, ref = op(xb, *t.keep, M), xb.double() @ w.T
+    assert yb.dtype == torch.bfloat16 and _rel(yb, ref) <= 2.0 ** -8 / 3 ** 0.5 * 1.1
+
+
+def test_split_gemm_refuses(cuda):
+    import cbq_ops
+    t, _ = _split_matrix(cuda, 4, 1024, 1)
+    op = cbq_ops.load().split_gemm
+    with pytest.raises(RuntimeError):
+        op(torch.zeros(20, 512, device=cuda), *t.keep, 8)
+    with pytest.raises(RuntimeError):
+        op(torch.zeros(20, 1024, device=cuda, dtype=torch.float16), *t.keep, 4)
+
+
+def test_split_module_views_and_types(cuda):
+    """The module over strided, misaligned and float16 x equals its result on
+    a fresh contiguous copy."""
+    from compressed_modules import AdaptiveCodebookLinear
+    t, w = _split_matrix(cuda, 64, 2048, 9)
+    layer = AdaptiveCodebookLinear.from_device("w", t)
+    base = torch.randn(40 * 2048 + 1, device=cuda)
+    odd = base[1:].view(40, 2048)                       # 4-byte aligned
+    assert torch.equal(layer(odd), layer(odd.clone()))
+    tr = torch.randn(2048, 40, device=cuda).t()         # column-major
+    assert torch.equal(layer(tr), layer(tr.contiguous()))
+    h = torch.randn(2, 20, 2048, device=cuda).half()
+    y = layer(h)
+    assert y.dtype == torch.float16 and y.shape == (2, 20, 64)
+    assert _rel(y.reshape(40, 64), h.reshape(40, 2048).double() @ w.T) <= 2.0 ** -11
