@@ -171,6 +171,22 @@ __device__ __forceinline__ void copy_to_lds(uint32_t *dst, const uint32_t *__res
     }
 }
 
+// n words global -> LDS without registers: the waves of the block take whole
+// KiB by direct copies (landed after a later __syncthreads) and the rest, or
+// everything when an end is not 16-byte aligned, through registers.
+__device__ __forceinline__ void dma_to_lds(uint32_t *dst, const uint32_t *__restrict__ src, int n,
+                                           int wave, int lane)
+{
+    int whole = 0;
+    if ((((uintptr_t)src | (uintptr_t)dst) & 15) == 0) {
+        whole = n & ~255;
+        for (int i = wave * 256; i < whole; i += (int)(blockDim.x / CBQ_WAVE) * 256)
+            __builtin_amdgcn_global_load_lds(
+                src + i + 4 * lane, (__attribute__((address_space(3))) void *)(dst + i), 16, 0, 0);
+    }
+    if (whole < n) copy_to_lds(dst + whole, src + whole, n - whole);
+}
+
 __device__ __forceinline__ void load_tables(uint32_t *s_lut1, uint32_t *s_lut2,
                                             const uint32_t *__restrict__ lut1,
                                             const uint32_t *__restrict__ lut2, int n_lut2,
@@ -975,6 +991,13 @@ __global__ __launch_bounds__(NW * CBQ_WAVE) void huff_col_kernel(const float *__
 
 // ---------------------------------------------------------------------------
 // Embedding: one wave per requested row (H % 64 == 0)
+//
+// Bound: the chain of a lane's 64 symbols, two dependent LDS table reads each
+// (about 10 us), after a chain of three global reads (id, chunk index, words).
+// So the tables come by direct copies beside the first row's index and words,
+// a symbol's window words are in registers before it, and rows go to the
+// blocks before they go to a block's waves.  H = 2048: 17.7 -> 15.5 us for one
+// token, 20.6 -> 17.3 for 512; H = 4096, 2048 tokens 42.4 -> 25.7.
 // ---------------------------------------------------------------------------
 
 template <bool VALUE_MODE>
@@ -988,62 +1011,95 @@ __global__ __launch_bounds__(kHBlock) void huff_embedding_kernel(
     const int lut2_slots = lut2_lds ? ((a.n_lut2 + 3) & ~3) : 0;
     float *s_cb = (float *)(s_lut2 + lut2_slots);
     uint32_t *s_stg = (uint32_t *)(s_cb + ((n_cb + 3) & ~3));
-    load_tables(s_lut1, s_lut2, a.lut1, a.lut2, a.n_lut2, lut2_lds, s_cb, a.value_cb, n_cb);
-    lds_barrier();
+    const int lane = threadIdx.x & (CBQ_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / CBQ_WAVE);
+    // rows are dealt over the blocks first: few tokens spread over the CUs
+    int t = blockIdx.x + wave * gridDim.x, r0 = 0;
+    int id = ids[t < T ? t : 0];
+    __builtin_amdgcn_sched_barrier(0);       // the id is under way before the tables
+    dma_to_lds(s_lut1, a.lut1, kLutSize, wave, lane);
+    if (lut2_lds) dma_to_lds(s_lut2, a.lut2, a.n_lut2, wave, lane);
+    if (n_cb > 0) dma_to_lds((uint32_t *)s_cb, (const uint32_t *)a.value_cb, n_cb, wave, lane);
 
     const Tabs tb{s_lut1, lut2_lds ? s_lut2 : a.lut2, (uint32_t)a.n_lut2, a.canon, a.canon_pay};
-    const int lane = threadIdx.x & (CBQ_WAVE - 1);
-    const int wave = threadIdx.x / CBQ_WAVE;
     uint32_t *stg = s_stg + wave * stg_words;
     const int KS = H / kSub;                 // sub-blocks per row
 
-    for (int t = blockIdx.x * kHWaves + wave; t < T; t += gridDim.x * kHWaves) {
-        int id = ids[t];
+    // Sub-blocks r0 .. r0 + 63 of row id: where this lane's sub-block starts,
+    // and the wave's words in its LDS slot
+    bool staged = false, active = false;
+    int64_t w0 = 0;
+    uint32_t pos = 0;
+    auto stage = [&]() {
         id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
-        const int64_t s_first = (int64_t)id * KS;
-        for (int r0 = 0; r0 < KS; r0 += CBQ_WAVE) {
-            // sub-blocks s_first + r0 + lane lie in at most two chunks: scan both
-            const int64_t sA = s_first + r0;
-            const int64_t cA = sA / kSub;
-            uint32_t lenA, lenB = 0;
-            const uint64_t startA = subblock_start(a, cA, lane, lenA);
-            const uint64_t startB = cA + 1 < a.n_chunks ? subblock_start(a, cA + 1, lane, lenB) : 0;
-            const int64_t s = sA + lane;
-            const bool active = (r0 + lane) < KS && s < a.n_sub;
-            const int src = (int)(s & (kSub - 1));
-            const bool inA = (s / kSub) == cA;
-            // every lane takes part in every shuffle (a shuffle reading a lane
-            // that skipped it returns nothing useful); select afterwards
-            const uint64_t stA = __shfl(startA, src, CBQ_WAVE);
-            const uint64_t stB = __shfl(startB, src, CBQ_WAVE);
-            const uint32_t lnA = __shfl(lenA, src, CBQ_WAVE);
-            const uint32_t lnB = __shfl(lenB, src, CBQ_WAVE);
-            const uint64_t my_start = inA ? stA : stB;
-            const uint32_t my_len = inA ? lnA : lnB;
-            const int n_act = std::min(CBQ_WAVE, KS - r0);
-            const uint64_t lo = __shfl(my_start, 0, CBQ_WAVE);
-            const uint64_t hi = __shfl(my_start + my_len, n_act - 1, CBQ_WAVE);
-            const bool staged = stage_words(stg, stg_words, a.words, a.n_words, lo, hi, lane);
-            const int64_t w0 = (int64_t)(lo >> 5);
-            uint32_t pos = (uint32_t)(my_start - ((uint64_t)w0 << 5));
-            if (active) {
-                float *dst = out + (size_t)t * H + (size_t)(r0 + lane) * kSub;
-#pragma unroll 4
+        // sub-blocks sA + lane lie in at most two chunks: scan both
+        const int64_t sA = (int64_t)id * KS + r0;
+        const int64_t cA = sA / kSub;
+        uint32_t lenA, lenB = 0;
+        const uint64_t startA = subblock_start(a, cA, lane, lenA);
+        const uint64_t startB = cA + 1 < a.n_chunks ? subblock_start(a, cA + 1, lane, lenB) : 0;
+        const int64_t s = sA + lane;
+        active = (r0 + lane) < KS && s < a.n_sub;
+        const int src = (int)(s & (kSub - 1));
+        const bool inA = (s / kSub) == cA;
+        // every lane takes part in every shuffle (a shuffle reading a lane
+        // that skipped it returns nothing useful); select afterwards
+        const uint64_t stA = __shfl(startA, src, CBQ_WAVE);
+        const uint64_t stB = __shfl(startB, src, CBQ_WAVE);
+        const uint32_t lnA = __shfl(lenA, src, CBQ_WAVE);
+        const uint32_t lnB = __shfl(lenB, src, CBQ_WAVE);
+        const uint64_t my_start = inA ? stA : stB;
+        const uint32_t my_len = inA ? lnA : lnB;
+        const int n_act = std::min(CBQ_WAVE, KS - r0);
+        const uint64_t lo = __shfl(my_start, 0, CBQ_WAVE);
+        const uint64_t hi = __shfl(my_start + my_len, n_act - 1, CBQ_WAVE);
+        staged = stage_words(stg, stg_words, a.words, a.n_words, lo, hi, lane);
+        w0 = (int64_t)(lo >> 5);
+        pos = (uint32_t)(my_start - ((uint64_t)w0 << 5));
+    };
+
+    if (t < T) stage();
+    __syncthreads();                         // the tables have landed
+    while (t < T) {
+        if (active) {
+            float *dst = out + (size_t)t * H + (size_t)(r0 + lane) * kSub;
+            if (staged) {
+                // the two words of the window stay in registers, the third
+                // is read a symbol ahead: only the table reads are on the
+                // chain of a symbol
+                uint32_t d = pos >> 5;
+                uint32_t q0 = stg[d], q1 = stg[d + 1];
                 for (int i = 0; i < kSub; i += 4) {
                     float v[4];
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
-                        const uint32_t w = staged ? window_lds(stg, pos)
-                                                  : window_global(a.words, a.n_words, w0, pos);
-                        const uint32_t e = decode_entry(w, tb);
+                        const uint32_t q2 = stg[min(d + 2, (uint32_t)stg_words - 1)];
+                        const uint32_t e = decode_entry(funnel(q1, q0, pos), tb);
                         pos += e & 63u;
+                        const bool step = (pos >> 5) != d;
+                        q0 = step ? q1 : q0;
+                        q1 = step ? q2 : q1;
+                        d = pos >> 5;
                         v[j] = payload_value<VALUE_MODE>(e, s_cb);
                     }
                     __builtin_memcpy(dst + i, v, sizeof(v));
                 }
+            } else {
+                for (int i = 0; i < kSub; i++) {
+                    const uint32_t e = decode_entry(window_global(a.words, a.n_words, w0, pos), tb);
+                    pos += e & 63u;
+                    dst[i] = payload_value<VALUE_MODE>(e, s_cb);
+                }
             }
-            wave_sync_lds();
         }
+        wave_sync_lds();
+        r0 += CBQ_WAVE;
+        if (r0 >= KS) {
+            r0 = 0;
+            t += gridDim.x * kHWaves;
+            if (t < T) id = ids[t];
+        }
+        if (t < T) stage();
     }
 }
 
@@ -1443,7 +1499,7 @@ int cbq_huff_embedding_f32(const int32_t *token_ids, const cbq_huff_stream *hs, 
     if (!value_mode && (a.C <= 0 || a.C > 16384)) return CK_ERR_ARG;
     const LdsPlan p = plan_lds(a.n_lut2, n_cb, stage_words_of(hs));
     if (p.bytes > 160 * 1024) return CK_ERR_ARG;
-    const int blocks = std::max(1, std::min((T + kHWaves - 1) / kHWaves, cbq_num_cus()));
+    const int blocks = std::min(T, cbq_num_cus());
     if (value_mode)
         hipLaunchKernelGGL((huff_embedding_kernel<true>), dim3(blocks), dim3(kHBlock), p.bytes,
                            stream, token_ids, out, a, T, vocab, H, p.stg_words, p.lut2_lds, 0);
