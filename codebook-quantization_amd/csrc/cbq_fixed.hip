@@ -24,6 +24,11 @@ int cbq_fixed_fewtok_t(const float *x, const uint8_t *packed, const float *cb, f
                        int M, int K, int C, int bits, hipStream_t st);
 int cbq_fixed_fewtok_t_bf16(const uint16_t *x, const uint8_t *packed, const float *cb,
                             uint16_t *out, int T, int M, int K, int C, int bits, hipStream_t st);
+// the first with x's fragments in a workspace (0 bytes: not worth it)
+size_t cbq_fewtok_ws_bytes(int T, int M, int K, int bits, bool f32);
+int cbq_fixed_fewtok_ws(const void *x, bool f32, const uint8_t *packed, const float *cb, void *out,
+                        int T, int M, int K, int C, int bits, void *ws, size_t ws_bytes,
+                        hipStream_t st);
 int cbq_fixed_tiny_t(const float *x, const uint8_t *packed, const float *cb, float *out, int T,
                      int M, int K, int C, int bits, hipStream_t st);
 int cbq_fixed_tiny_t_bf16(const uint16_t *x, const uint8_t *packed, const float *cb,
@@ -1142,7 +1147,7 @@ int ck_linear_f32(const float *x, const uint8_t *packed, const float *codebook, 
 size_t cbq_linear_f32_workspace(int T, int M, int K)
 {
     if (T <= 0 || M <= 0 || K <= 0) return 0;
-    return cbq_frag_ws_bytes(T, M, K, 0, true);
+    return std::max(cbq_fewtok_ws_bytes(T, M, K, 0, true), cbq_frag_ws_bytes(T, M, K, 0, true));
 }
 
 int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebook, float *out,
@@ -1150,8 +1155,11 @@ int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebo
                       hipStream_t stream)
 {
     if (x && packed && codebook && out && M > 0 && K > 0 && C > 0 && bits >= 1 && bits <= 16) {
-        const int rc = cbq_frag_linear(x, true, packed, codebook, out, T, M, K, C, bits, workspace,
-                                       ws_bytes, stream);
+        int rc = cbq_fixed_fewtok_ws(x, true, packed, codebook, out, T, M, K, C, bits, workspace,
+                                     ws_bytes, stream);
+        if (rc < 0)
+            rc = cbq_frag_linear(x, true, packed, codebook, out, T, M, K, C, bits, workspace,
+                                 ws_bytes, stream);
         if (rc >= 0) return rc;
     }
     return ck_linear_f32(x, packed, codebook, out, T, M, K, C, bits, stream);
@@ -1353,13 +1361,21 @@ size_t cbq_linear_bf16_workspace(int T, int M, int K)
 size_t cbq_linear_bf16_gemm_workspace(int T, int M, int K, int bits)
 {
     if (T <= 0 || M <= 0 || K <= 0) return 0;
-    return std::max(cbq_prefill_ws_bytes(T, M, K), cbq_frag_ws_bytes(T, M, K, bits, false));
+    return std::max(cbq_fewtok_ws_bytes(T, M, K, bits, false),
+                    std::max(cbq_prefill_ws_bytes(T, M, K),
+                             cbq_frag_ws_bytes(T, M, K, bits, false)));
 }
 
 int cbq_linear_bf16_ws(const void *x_bf16, const uint8_t *packed, const float *codebook,
                        void *out_bf16, int T, int M, int K, int C, int bits, void *workspace,
                        size_t ws_bytes, hipStream_t stream)
 {
+    if (x_bf16 && packed && codebook && out_bf16 && M > 0 && K > 0 && C > 0 && bits >= 1 &&
+        bits <= 16) {
+        const int rc = cbq_fixed_fewtok_ws(x_bf16, false, packed, codebook, out_bf16, T, M, K, C,
+                                           bits, workspace, ws_bytes, stream);
+        if (rc >= 0) return rc;
+    }
     // (64 tokens that the few-token kernel takes go there)
     if (x_bf16 && packed && codebook && out_bf16 && T >= 64 && M > 0 && K > 0 && C > 0 &&
         bits >= 1 && bits <= 16 && (T > 64 || K % 128 != 0)) {

@@ -938,6 +938,20 @@ int cbq_frag_linear(const void *x, bool f32, const uint8_t *packed, const float 
 #undef CBQ_FL
 }
 
+// x [T][K] as fragments: fp32 as three parts, bf16 as one.
+int cbq_frag_x(const void *x, bool f32, void *xf, int T, int K, hipStream_t st)
+{
+    const int64_t units = (int64_t)((T + 15) >> 4) * (K >> 5);
+    const int blocks = (int)std::min<int64_t>((units + 3) / 4, kPrepBlocks * cbq_num_cus());
+    if (f32)
+        hipLaunchKernelGGL(frag_x_kernel<3>, dim3(blocks), dim3(kPBlock), 0, st, x, (uint8_t *)xf, T,
+                           K);
+    else
+        hipLaunchKernelGGL(frag_x_kernel<1>, dim3(blocks), dim3(kPBlock), 0, st, x, (uint8_t *)xf, T,
+                           K);
+    return cbq_launch_status("frag_x_kernel");
+}
+
 // ---- split-format matrices -------------------------------------------------------
 
 // cbq_split.hip: rows [row0, row0 + M) of the matrix as fragments
@@ -971,15 +985,7 @@ extern "C" int cbq_split_linear_gemm(const void *x, int x_bf16, int T, const cbq
     const int NP = x_bf16 ? 1 : 3;
     const GemmPlan p = gemm_plan(T, M, K, NP, 1);
     GemmArgs a = gemm_args(p, NP, 1, x, T, M, K, (uint8_t *)ws);
-    const int64_t units = (int64_t)((T + 15) >> 4) * (K >> 5);
-    const int nxb = (int)std::min<int64_t>((units + 3) / 4, kPrepBlocks * cbq_num_cus());
-    if (x_bf16)
-        hipLaunchKernelGGL(frag_x_kernel<1>, dim3(nxb), dim3(kPBlock), 0, stream, x,
-                           (uint8_t *)a.xf, T, K);
-    else
-        hipLaunchKernelGGL(frag_x_kernel<3>, dim3(nxb), dim3(kPBlock), 0, stream, x,
-                           (uint8_t *)a.xf, T, K);
-    int rc = cbq_launch_status("frag_x_kernel");
+    int rc = cbq_frag_x(x, !x_bf16, (void *)a.xf, T, K, stream);
     for (int r0 = 0; r0 < M && !rc; r0 += p.rows) {
         a.M = std::min(p.rows, M - r0);
         a.out = (uint8_t *)out + (size_t)r0 * (NP == 3 ? 4 : 2);

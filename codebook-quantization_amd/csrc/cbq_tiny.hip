@@ -52,6 +52,9 @@
 
 #include <algorithm>
 
+// x as MFMA fragments (cbq_gemm.hip): [T / 16][K / 32][parts] of 1 KiB.
+int cbq_frag_x(const void *x, bool f32, void *xf, int T, int K, hipStream_t st);
+
 namespace {
 
 constexpr int kTinyWaves = 8;                 // 2 row tiles x 4 column quarters
@@ -108,9 +111,11 @@ template <> struct FtX<uint16_t> {
 // R row tiles per block, Q tile-steps of weights in flight per wave (Q
 // divides R, so every ring slot is a compile-time register array), NT blocks
 // of 16 tokens: a decoded tile-step is multiplied with each of them.
-template <int BITS, int R, int Q, int NT, typename XT, typename OT>
+// XF: x comes as MFMA fragments (cbq_frag_x: 1 KiB per 16 tokens, 32 columns
+// and part) instead of rows.
+template <int BITS, int R, int Q, int NT, bool XF, typename XT, typename OT>
 __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
-    const XT *__restrict__ x, const uint32_t *__restrict__ words,
+    const void *__restrict__ xv, const uint32_t *__restrict__ words,
     const float *__restrict__ cb, OT *__restrict__ out, int T, int M, int K, int C)
 {
     static_assert(R % Q == 0, "ring slots are static: Q divides R");
@@ -118,7 +123,10 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
     constexpr bool PADDED = BITS <= 14;           // 2^BITS-entry table: the clamp is free
     constexpr int NI = (BITS + 3) / 4;            // 16-byte loads per lane and tile-step
     constexpr int CH = 16 * BITS;                 // 16-byte chunks of a tile-step
-    constexpr int XW = FtX<XT>::kWords;
+    constexpr int NP = FtX<XT>::kParts;
+    constexpr bool FOLD = XF && NP == 3;
+    constexpr int XW = XF ? 16 * NP : FtX<XT>::kWords;
+    const XT *const x = (const XT *)xv;
     __shared__ __attribute__((aligned(16))) float s_cb[PADDED ? (1 << BITS) : kTinyMaxCodebook];
     __shared__ __attribute__((aligned(16))) uint32_t s_tr[kFtWaves][64 * BITS];
     __shared__ int s_flag[kFtWaves];
@@ -177,6 +185,16 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
     auto load_x = [&](int s, uint32_t (&xw)[NT][XW]) {
 #pragma unroll
         for (int b = 0; b < NT; b++) {
+            if constexpr (XF) {
+                const uint8_t *f = (const uint8_t *)xv +
+                                   ((size_t)b * G + 4 * gstep(s) + j) * (NP * 1024) + rsub * 16;
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+#pragma unroll
+                    for (int p = 0; p < NP; p++)
+                        __builtin_memcpy(&xw[b][4 * (c * NP + p)], f + p * 1024 + c * 256, 16);
+                continue;
+            }
             const int t = b * 16 + rsub;
             if (t < T) {
                 __builtin_memcpy(xw[b], x + (size_t)t * K + (size_t)(4 * gstep(s) + j) * 32,
@@ -190,9 +208,9 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
     u32x4 wr[Q][NI];
 #pragma unroll
     for (int q = 0; q < Q; q++) load_item(0, q, wr[q]);
-    // up to two token blocks: x a step ahead; more would not fit the
-    // registers, and the decode of the step's first tile covers their loads
-    constexpr bool XAHEAD = NT <= 2;
+    // one block of fp32 or two of bf16 tokens: x a step ahead; more would not
+    // fit the registers, and the decode of the step's first tile covers their loads
+    constexpr bool XAHEAD = NP == 3 ? NT == 1 && !(XF && R > 3) : NT <= 2;
     uint32_t xn[NT][XW];
     if constexpr (XAHEAD) load_x(0, xn);
     __builtin_amdgcn_sched_barrier(0);
@@ -227,7 +245,18 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
         u32x4 xb[NT][4][3];
         if constexpr (!XAHEAD) load_x(s, xn);
 #pragma unroll
-        for (int b = 0; b < NT; b++) FtX<XT>::parts(xn[b], xb[b]);
+        for (int b = 0; b < NT; b++) {
+            if constexpr (XF) {
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+#pragma unroll
+                    for (int p = 0; p < NP; p++)
+                        xb[b][c][p] = u32x4{xn[b][4 * (c * NP + p)], xn[b][4 * (c * NP + p) + 1],
+                                            xn[b][4 * (c * NP + p) + 2], xn[b][4 * (c * NP + p) + 3]};
+            } else {
+                FtX<XT>::parts(xn[b], xb[b]);
+            }
+        }
         if constexpr (XAHEAD) load_x(s + 1, xn);   // next step's x, one step ahead
 #pragma unroll
         for (int t = 0; t < R; t++) {
@@ -256,13 +285,17 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
                              cbq_hi_pair(__float_as_uint(wv[8 * c + 2]), __float_as_uint(wv[8 * c + 3])),
                              cbq_hi_pair(__float_as_uint(wv[8 * c + 4]), __float_as_uint(wv[8 * c + 5])),
                              cbq_hi_pair(__float_as_uint(wv[8 * c + 6]), __float_as_uint(wv[8 * c + 7]))};
+            // FOLD: a step's MFMAs round at the step's magnitude, not the sum's
+            f4 run[NT];
+#pragma unroll
+            for (int b = 0; b < NT; b++) run[b] = FOLD ? f4{0.f, 0.f, 0.f, 0.f} : acc[t][b];
 #pragma unroll
             for (int c = 0; c < 4; c++)
 #pragma unroll
-                for (int p = 0; p < FtX<XT>::kParts; p++)
+                for (int p = 0; p < NP; p++)
 #pragma unroll
                     for (int b = 0; b < NT; b++)
-                        acc[t][b] = cbq_mfma_bf16(a[c], xb[b][c][p], acc[t][b]);
+                        run[b] = cbq_mfma_bf16(a[c], xb[b][c][p], run[b]);
             if (wsplit) {                          // codebook not bf16: w = wh + wm + wl
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
@@ -273,12 +306,16 @@ __global__ __launch_bounds__(kFtThreads) void fixed_fewtok_kernel(
                     cbq_split3(q8, wh, wm, wl);
 #pragma unroll
                     for (int b = 0; b < NT; b++) {
-                        acc[t][b] = cbq_mfma_bf16(wm, xb[b][c][0], acc[t][b]);
-                        acc[t][b] = cbq_mfma_bf16(wl, xb[b][c][0], acc[t][b]);
-                        if (FtX<XT>::kParts > 1)
-                            acc[t][b] = cbq_mfma_bf16(wm, xb[b][c][1], acc[t][b]);
+                        run[b] = cbq_mfma_bf16(wm, xb[b][c][0], run[b]);
+                        run[b] = cbq_mfma_bf16(wl, xb[b][c][0], run[b]);
+                        if (NP > 1) run[b] = cbq_mfma_bf16(wm, xb[b][c][1], run[b]);
                     }
                 }
+            }
+#pragma unroll
+            for (int b = 0; b < NT; b++) {
+                if constexpr (FOLD) acc[t][b] += run[b];
+                else acc[t][b] = run[b];
             }
         }
     }
@@ -473,13 +510,13 @@ int tiny_launch(const XT *x, const uint8_t *packed, const float *cb, OT *out, in
     return cbq_launch_status("fixed_tiny_mfma_kernel");
 }
 
-template <int R, int Q, int NT, typename XT, typename OT>
-int fewtok_launch_r(const XT *x, const uint8_t *packed, const float *cb, OT *out, int T, int M,
+template <int R, int Q, int NT, bool XF, typename XT, typename OT>
+int fewtok_launch_r(const void *x, const uint8_t *packed, const float *cb, OT *out, int T, int M,
                     int K, int C, int bits, int blocks, hipStream_t st)
 {
     const size_t lds = (size_t)kFtWaves * R * NT * CBQ_WAVE * sizeof(f4);
 #define CBQ_FT(B)                                                                              \
-    hipLaunchKernelGGL((fixed_fewtok_kernel<B, R, Q, NT, XT, OT>), dim3(blocks),                \
+    hipLaunchKernelGGL((fixed_fewtok_kernel<B, R, Q, NT, XF, XT, OT>), dim3(blocks),            \
                        dim3(kFtThreads), lds, st, x, (const uint32_t *)packed, cb, out, T, M, K, C)
     switch (bits) {
     case 8: CBQ_FT(8); break;
@@ -504,9 +541,7 @@ int fewtok_launch_r(const XT *x, const uint8_t *packed, const float *cb, OT *out
 // (20 us); 1536 tiles take R = 6.  Several token blocks: R * NT partial tiles
 // a wave beside the table and the re-lay buffers, at most 6 at 14 and 16
 // bits (92 and 96 KiB) and 12 below (59 KiB at 13).
-template <int NT, typename XT, typename OT>
-int fewtok_launch_n(const XT *x, const uint8_t *packed, const float *cb, OT *out, int T, int M,
-                    int K, int C, int bits, hipStream_t st)
+int fewtok_rows(int M, int NT, int bits)
 {
     const long tiles = (M + 15) / 16;
     const long ncu = cbq_num_cus();
@@ -521,33 +556,57 @@ int fewtok_launch_n(const XT *x, const uint8_t *packed, const float *cb, OT *out
             R = r;
         }
     }
-    const long blocks = (tiles + R - 1) / R;
-    if (blocks > 0x7fffffffL) return -1;
-    if constexpr (NT == 1)
-        if (R == 6)
-            return fewtok_launch_r<6, 2, NT>(x, packed, cb, out, T, M, K, C, bits, (int)blocks, st);
-    switch (R) {
-    case 3: return fewtok_launch_r<3, (NT > 3 ? 1 : 3), NT>(x, packed, cb, out, T, M, K, C, bits, (int)blocks, st);
-    case 2: return fewtok_launch_r<2, 2, NT>(x, packed, cb, out, T, M, K, C, bits, (int)blocks, st);
-    default: return fewtok_launch_r<1, 1, NT>(x, packed, cb, out, T, M, K, C, bits, (int)blocks, st);
-    }
+    return R;
 }
 
-template <typename XT, typename OT>
-int fewtok_launch(const XT *x, const uint8_t *packed, const float *cb, OT *out, int T, int M,
-                  int K, int C, int bits, hipStream_t st)
+template <int NT, bool XF, typename XT, typename OT>
+int fewtok_launch_n(const void *x, const uint8_t *packed, const float *cb, OT *out, int T, int M,
+                    int K, int C, int bits, hipStream_t st)
 {
-    if (T < 2 || T > (sizeof(XT) == 2 ? 64 : 16) || M <= 0 || K <= 0 || K % 128 || C <= 0 ||
-        C > kTinyMaxCodebook)
-        return -1;
-    if (((uintptr_t)x & 15) != 0 || ((uintptr_t)packed & 15) != 0) return -1;
-    if (bits != 8 && (bits < 10 || bits > 14) && bits != 16) return -1;
-    if constexpr (sizeof(XT) == 2) {
-        if (T > 48) return fewtok_launch_n<4>(x, packed, cb, out, T, M, K, C, bits, st);
-        if (T > 32) return fewtok_launch_n<3>(x, packed, cb, out, T, M, K, C, bits, st);
-        if (T > 16) return fewtok_launch_n<2>(x, packed, cb, out, T, M, K, C, bits, st);
+    const int R = fewtok_rows(M, NT, bits);
+    const long blocks = ((M + 15) / 16 + R - 1) / R;
+    if (blocks > 0x7fffffffL) return -1;
+    constexpr int Q3 = NT > (sizeof(XT) == 4 ? 1 : 3) ? 1 : 3;   // registers
+#define CBQ_FN(R, Q)                                                                           \
+    return fewtok_launch_r<R, Q, NT, XF, XT, OT>(x, packed, cb, out, T, M, K, C, bits,          \
+                                                 (int)blocks, st)
+    if constexpr (NT == 1)
+        if (R == 6) CBQ_FN(6, 2);
+    switch (R) {
+    case 3: CBQ_FN(3, Q3);
+    case 2: CBQ_FN(2, 2);
+    default: CBQ_FN(1, 1);
     }
-    return fewtok_launch_n<1>(x, packed, cb, out, T, M, K, C, bits, st);
+#undef CBQ_FN
+}
+
+bool fewtok_takes(int T, int M, int K, int C, int bits, bool f32)
+{
+    return T >= 2 && T <= (f32 ? 32 : 64) && M > 0 && K > 0 && K % 128 == 0 && C > 0 &&
+           C <= kTinyMaxCodebook && (bits == 8 || (bits >= 10 && bits <= 14) || bits == 16);
+}
+
+// xf: x's fragments, or null (fp32: at most 16 tokens then)
+template <typename XT, typename OT>
+int fewtok_launch(const XT *x, const void *xf, const uint8_t *packed, const float *cb, OT *out,
+                  int T, int M, int K, int C, int bits, hipStream_t st)
+{
+    constexpr bool f32 = sizeof(XT) == 4;
+    if (!fewtok_takes(T, M, K, C, bits, f32) || (f32 && !xf && T > 16)) return -1;
+    if (((uintptr_t)x & 15) != 0 || ((uintptr_t)packed & 15) != 0) return -1;
+#define CBQ_FW(NT)                                                                             \
+    return xf ? fewtok_launch_n<NT, true, XT, OT>(xf, packed, cb, out, T, M, K, C, bits, st)    \
+              : fewtok_launch_n<NT, false, XT, OT>(x, packed, cb, out, T, M, K, C, bits, st)
+    if constexpr (f32) {
+        if (T > 16)
+            return fewtok_launch_n<2, true, XT, OT>(xf, packed, cb, out, T, M, K, C, bits, st);
+    } else {
+        if (T > 48) CBQ_FW(4);
+        if (T > 32) CBQ_FW(3);
+        if (T > 16) CBQ_FW(2);
+    }
+    CBQ_FW(1);
+#undef CBQ_FW
 }
 
 }  // namespace
@@ -573,11 +632,53 @@ int cbq_fixed_tiny_t_bf16(const uint16_t *x, const uint8_t *packed, const float 
 int cbq_fixed_fewtok_t(const float *x, const uint8_t *packed, const float *cb, float *out, int T,
                        int M, int K, int C, int bits, hipStream_t st)
 {
-    return fewtok_launch<float, float>(x, packed, cb, out, T, M, K, C, bits, st);
+    return fewtok_launch<float, float>(x, nullptr, packed, cb, out, T, M, K, C, bits, st);
 }
 
 int cbq_fixed_fewtok_t_bf16(const uint16_t *x, const uint8_t *packed, const float *cb,
                             uint16_t *out, int T, int M, int K, int C, int bits, hipStream_t st)
 {
-    return fewtok_launch<uint16_t, uint16_t>(x, packed, cb, out, T, M, K, C, bits, st);
+    return fewtok_launch<uint16_t, uint16_t>(x, nullptr, packed, cb, out, T, M, K, C, bits, st);
+}
+
+// Workspace bytes (x's fragments) with which cbq_fixed_fewtok_ws runs this
+// shape in one launch beside the copy of x; 0: not worth it or not taken.
+// Reading x by rows, a load takes a line per lane, 4 T lines, where a
+// contiguous KiB of fragments takes 16 clocks; a block does 8 (fp32) or 4
+// (bf16) such loads for each of its K / 128 steps.  The copy's launch costs
+// 4 to 5 us; measured break-even at 12000 (fp32, which also saves the split
+// in the kernel) and 16000 lines saved per CU: bf16 T = 40 4096 x 4096
+// (14300) 15.8 by rows against 16.6, T = 48 (18400) 17.1 / 15.8, T = 64
+// 4096 x 12288 51.7 / 30.2; fp32 T = 16 4096 x 12288 35.0 / 31.4, 4096 x 1024
+// (10200) 14.0 / 14.7.  17 to 32 fp32 tokens have no one-launch path without
+// it (12288 x 4096, T = 32: 51 us in two launches, 29 here).
+size_t cbq_fewtok_ws_bytes(int T, int M, int K, int bits, bool f32)
+{
+    if (!fewtok_takes(T, M, K, 1, bits ? bits : 13, f32)) return 0;
+    const int nt = (T + 15) / 16, parts = f32 ? 3 : 1;
+    const long steps = K / 128;
+    const int R = fewtok_rows(M, nt, bits ? bits : 13);
+    const long rounds = (((M + 15) / 16 + R - 1) / R + cbq_num_cus() - 1) / cbq_num_cus();
+    const long saved = steps * rounds * ((f32 ? 8 : 4) * 4 * T - 64 * parts * nt);
+    if (!(f32 && T > 16) && saved < (f32 ? 12000 : 16000)) return 0;
+    return (size_t)nt * (K >> 5) * parts * 1024;
+}
+
+// The few-token product with x's fragments written to ws first (16-byte
+// aligned, cbq_fewtok_ws_bytes); -1: not handled here.
+int cbq_fixed_fewtok_ws(const void *x, bool f32, const uint8_t *packed, const float *cb, void *out,
+                        int T, int M, int K, int C, int bits, void *ws, size_t ws_bytes,
+                        hipStream_t st)
+{
+    const size_t need = cbq_fewtok_ws_bytes(T, M, K, bits, f32);
+    if (!need || !ws || ws_bytes < need || !fewtok_takes(T, M, K, C, bits, f32) ||
+        (((uintptr_t)ws | (uintptr_t)x | (uintptr_t)packed) & 15) != 0)
+        return -1;
+    const int rc = cbq_frag_x(x, f32, ws, T, K, st);
+    if (rc) return rc;
+    if (f32)
+        return fewtok_launch<float, float>((const float *)x, ws, packed, cb, (float *)out, T, M, K,
+                                           C, bits, st);
+    return fewtok_launch<uint16_t, uint16_t>((const uint16_t *)x, ws, packed, cb, (uint16_t *)out,
+                                             T, M, K, C, bits, st);
 }

@@ -51,7 +51,8 @@ int ck_linear_f32(const float *x, const uint8_t *packed, const float *codebook,
 size_t cbq_linear_f32_workspace(int T, int M, int K);
 
 /* ck_linear_f32 with a caller workspace (>= cbq_linear_f32_workspace bytes,
- * 16-byte aligned): for T >= 33 (K % 32 == 0, widths 8 and 10..14, x 16-byte
+ * 16-byte aligned): 17 to 32 tokens (fewer where it pays; K % 128 == 0) run in
+ * one launch with x's bf16 parts there in MFMA fragment order; for T >= 33 (K % 32 == 0, widths 8 and 10..14, x 16-byte
  * aligned) x (three exact bf16 parts) and the weights are first written there
  * in MFMA fragment order, the weights in slabs of at most 384 MiB, and
  * multiplied on the bf16 matrix cores with fp32 accumulation; K is split

@@ -65,6 +65,8 @@ def _rel(y, ref):
 
 @pytest.mark.parametrize("T,M,K,bits", [
     (64, 1, 32, 13),            # one column group, one row
+    (17, 33, 128, 13), (32, 1000, 4224, 14), (24, 520, 2048, 16),   # few tokens, x as fragments
+    (16, 40, 12288, 13), (10, 4100, 12416, 10), (29, 24600, 256, 8),
     (33, 4096, 2048, 13), (48, 31, 96, 12),
     (65, 33, 64, 12),           # a row past a superblock, a token past a tile
     (127, 257, 96, 14), (129, 300, 4064, 13), (192, 520, 288, 11), (257, 1000, 1056, 10),
@@ -142,6 +144,7 @@ def test_f32_graph(cuda):
     (17, 33, 128, 13), (32, 1000, 4224, 14), (33, 16, 256, 12), (48, 300, 1152, 13),
     (49, 12288, 128, 10), (64, 520, 2048, 16), (64, 4100, 1024, 13),     # few-token kernel
     (63, 70, 96, 13),                                                    # refused by it
+    (16, 70, 20480, 12), (30, 1000, 12288, 13), (64, 300, 12288, 14),    # x as fragments
     (65, 33, 64, 12), (127, 257, 96, 14), (129, 300, 4064, 13), (257, 1000, 1056, 10),
     (300, 2048, 2080, 8), (700, 1030, 544, 11), (1030, 3000, 544, 13), (2050, 520, 96, 13)])
 @pytest.mark.parametrize("kind", ["bf16", "fp32"])
