@@ -516,27 +516,21 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
         }
         const uint32_t lane16 = lane * 16;
         const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
-        // the next column group into LDS offset buf; past the end the last
-        // one is copied again, so every wave keeps as many copies in flight
+        // copy i of the next column group into LDS offset buf; past the end
+        // the last one is copied again, so every wave keeps as many in flight
         int gi = g0;
-        auto issue = [&](uint32_t buf) {
-#pragma unroll
-            for (int i = 0; i < PL; i++)
-                lds_copy_frag(lds0 + buf + dst[i], base[i] + (uint32_t)gi * step[i], lane16);
-            gi += gi + 1 < g0 + n ? 1 : 0;
+        auto copy = [&](uint32_t buf, int i) {
+            lds_copy_frag(lds0 + buf + dst[i], base[i] + (uint32_t)gi * step[i], lane16);
         };
+        auto advance = [&]() { gi += gi + 1 < g0 + n ? 1 : 0; };
         const uint8_t *const rda = lds + (Cfg::NB * WP + wt * TB) * (int)kFrag + lane16;
         const uint8_t *const rdb = lds + wm * MB * (int)kFrag + lane16;
         cbq_u32x4 fa[2][TB], fb[2][MB];
-        auto read_a = [&](uint32_t buf, int p, cbq_u32x4 (&f)[TB]) {
-#pragma unroll
-            for (int i = 0; i < TB; i++)
-                f[i] = *(const cbq_u32x4 *)(rda + buf + (i + p * Cfg::NA) * (int)kFrag);
+        auto read_a = [&](uint32_t buf, int p, int i, cbq_u32x4 (&f)[TB]) {
+            f[i] = *(const cbq_u32x4 *)(rda + buf + (i + p * Cfg::NA) * (int)kFrag);
         };
-        auto read_b = [&](uint32_t buf, int p, cbq_u32x4 (&f)[MB]) {
-#pragma unroll
-            for (int j = 0; j < MB; j++)
-                f[j] = *(const cbq_u32x4 *)(rdb + buf + (j + p * Cfg::NB) * (int)kFrag);
+        auto read_b = [&](uint32_t buf, int p, int j, cbq_u32x4 (&f)[MB]) {
+            f[j] = *(const cbq_u32x4 *)(rdb + buf + (j + p * Cfg::NB) * (int)kFrag);
         };
         uint32_t cur = 0;                                   // LDS offset of the running stage
         uint32_t old = (NST - 1) * STAGE;                   // and of the one before it
@@ -546,49 +540,83 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
         // waited for here) or at least the one before it, whose MFMAs have
         // been issued (LAG 1), so the barrier frees that LDS for the next
         // copies and publishes the next stage.
+        // With three x parts the copies into it are spread over that
+        // product's MFMAs: a wave that issues them all at once waits in the
+        // memory pipeline's queue before its MFMAs (T = 1024, 8192 x 4096:
+        // 184 -> 165 us; over the next stage's products too: 168). With one
+        // part the stage is a third as long and the earlier copies matter
+        // more (T = 333, 4096 x 4096: 51 us against 53 spread).
         auto stage = [&](auto P0, auto Q0) {
             constexpr int p0 = decltype(P0)::value, q0 = decltype(Q0)::value;
 #pragma unroll
             for (int i = 0; i < NS; i++) {
                 const int k = (p0 + i) & 1, q = (q0 + St::wpart(i)) & 1;
-                int reads = TB;
-                if (i < NS - 1) {
-                    if (NP > 1) read_a(cur, St::xpart(i + 1), fa[k ^ 1]);
-                    else reads = 0;
-                    if (St::wpart(i + 1) != St::wpart(i)) {
-                        read_b(cur, St::wpart(i + 1), fb[q ^ 1]);
-                        reads += MB;
-                    }
-                } else {
+                const bool last = i == NS - 1;
+                const bool next_a = last || NP > 1;
+                const bool next_b = last || St::wpart(i + 1) != St::wpart(i);
+                const int na = next_a ? TB : 0, nb = next_b ? MB : 0;
+                const int np = last ? 0 : St::xpart(i + 1), nw = last ? 0 : St::wpart(i + 1);
+                cbq_u32x4 (&an)[TB] = fa[NP > 1 ? k ^ 1 : p0 ^ 1];
+                cbq_u32x4 (&bn)[MB] = fb[q ^ 1];
+                const uint32_t free_buf = LAG ? old : cur;
+                if (last) {
                     stage_barrier<(NST - 2 - LAG) * PL, LAG == 0>();
-                    issue(LAG ? old : cur);
                     old = cur;
                     cur = cur + STAGE == NST * STAGE ? 0u : cur + STAGE;
-                    read_a(cur, 0, fa[NP > 1 ? k ^ 1 : p0 ^ 1]);
-                    read_b(cur, 0, fb[q ^ 1]);
-                    reads += MB;
+                }
+                auto read = [&](int r) {
+                    if (r < nb) read_b(cur, nw, r, bn);
+                    else read_a(cur, np, r - nb, an);
+                };
+                constexpr int NM = TB * MB;
+                if constexpr (NP == 1) {
+                    if (last)
+#pragma unroll
+                        for (int c = 0; c < PL; c++) copy(free_buf, c);
+#pragma unroll
+                    for (int r = 0; r < nb + na; r++) read(r);
                 }
 #pragma unroll
-                for (int x = 0; x < TB; x++)
+                for (int m = 0; m < NM; m++) {
+                    if constexpr (NP > 1) {
+                        // reads over the first half of the MFMAs, copies over all
 #pragma unroll
-                    for (int w = 0; w < MB; w++)
-                        acc[x][w] = cbq_mfma_bf16(fb[q][w], fa[NP > 1 ? k : p0][x], acc[x][w]);
+                        for (int r = m * 2 * (na + nb) / NM;
+                             r < (m + 1) * 2 * (na + nb) / NM && r < na + nb; r++)
+                            read(r);
+                        if (last)
 #pragma unroll
-                for (int r = 0; r < reads; r++) {
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                            for (int c = m * PL / NM; c < (m + 1) * PL / NM; c++)
+                                copy(free_buf, c);
+                    }
+                    const int x = m / MB, w = m % MB;
+                    acc[x][w] = cbq_mfma_bf16(fb[q][w], fa[NP > 1 ? k : p0][x], acc[x][w]);
+                    if constexpr (NP > 1) __builtin_amdgcn_sched_barrier(0);
                 }
-                __builtin_amdgcn_sched_group_barrier(0x008, TB * MB, 0);
+                if constexpr (NP == 1) {
+#pragma unroll
+                    for (int r = 0; r < na + nb; r++) {
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                    }
+                    __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
+                }
+                if (last) advance();
             }
         };
         // fragment registers in use at the start of every second stage
         constexpr int P1 = NP > 1 ? NS & 1 : 1, Q1 = WP & 1;
         const std::integral_constant<int, 0> I0{};
+        for (int b = 0; b < NST - LAG; b++) {
 #pragma unroll
-        for (int i = 0; i < NST - LAG; i++) issue(i * STAGE);
+            for (int i = 0; i < PL; i++) copy(b * STAGE, i);
+            advance();
+        }
         stage_barrier<(NST - 1 - LAG) * PL, true>();
-        read_a(0, 0, fa[0]);
-        read_b(0, 0, fb[0]);
+#pragma unroll
+        for (int i = 0; i < TB; i++) read_a(0, 0, i, fa[0]);
+#pragma unroll
+        for (int j = 0; j < MB; j++) read_b(0, 0, j, fb[0]);
         for (int s = 0; s < n;) {
             const int e = FOLD ? min(n, s + a.fold) : n;
             for (; s + 2 <= e; s += 2) {
@@ -713,8 +741,8 @@ constexpr int kShapes = 5;
 const GemmShape kShape1[kShapes] = {shape_of<Gemm1a>(0.86f), shape_of<Gemm1b>(0.49f),
                                     shape_of<Gemm1c>(0.26f), shape_of<Gemm1d>(0.19f),
                                     shape_of<Gemm1e>(0.66f)};
-const GemmShape kShape3[kShapes] = {shape_of<Gemm3a>(1.45f), shape_of<Gemm3b>(1.37f),
-                                    shape_of<Gemm3c>(0.82f), shape_of<Gemm3d>(0.76f),
+const GemmShape kShape3[kShapes] = {shape_of<Gemm3a>(1.36f), shape_of<Gemm3b>(1.25f),
+                                    shape_of<Gemm3c>(0.72f), shape_of<Gemm3d>(0.67f),
                                     shape_of<Gemm3e>(0.40f)};
 
 struct GemmPlan {
