@@ -433,7 +433,7 @@ def from_synthetic(cfg: DecoderConfig, tensors: Dict[str, object], device="cuda"
     import synthetic
     from gpu_huffman_functions import (SymbolDecoder, build_split, huffman_prefill,
                                        split_bytes, split_eligible, split_inverse,
-                                       split_prefill, stack_split)
+                                       split_prefill, stack_split, stacked_parts)
     lib = nat.load()
     dev = torch.device(device)
     resident: Dict[str, int] = {}               # device bytes of each matrix's format
@@ -640,7 +640,7 @@ def from_synthetic(cfg: DecoderConfig, tensors: Dict[str, object], device="cuda"
             st = stack_split(sps, cbs[0], Ms, K, dev)
             if st is not None:
                 keep, sdesc, parts = st
-                sps = [(keep, parts[0]), (keep, parts[1])]
+                sps = stacked_parts(keep, parts)
                 for t in ts:
                     resident.pop(t.name, None)
                 resident[name] = split_bytes(keep)

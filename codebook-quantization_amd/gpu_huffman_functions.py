@@ -467,6 +467,19 @@ def stack_split(splits, codebook: np.ndarray, Ms, K: int, device):
     return keep, desc, parts
 
 
+def stacked_parts(keep, parts):
+    """(tensors, descriptor) of each part of a stack_split: views of the
+    stacked arrays that hold that part's chunks, as split_gemm takes them."""
+    cwords, row_off, raw, lut = keep
+    pairs, c0 = [], 0
+    for d in parts:
+        c1 = c0 + int(d.n_chunks)
+        pairs.append(((cwords, row_off[c0:c1 + 1],
+                       raw[c0 * hc.CHUNK_SYMBOLS:c1 * hc.CHUNK_SYMBOLS], lut), d))
+        c0 = c1
+    return pairs
+
+
 def columns_eligible(desc: "nat.HuffStream", K: int) -> bool:
     """The column GEMV serves T = 1 rows of whole 4096-symbol chunks with
     bf16-value payloads and a second table level that fits its LDS."""

@@ -193,6 +193,24 @@ def test_split_gemm(cuda, T, M, K):
     assert yb.dtype == torch.bfloat16 and _rel(yb, ref) <= 2.0 ** -8 / 3 ** 0.5 * 1.1
 
 
+@pytest.mark.parametrize("M,K", [(4, 1024), (36, 3072), (40, 4096)])
+def test_split_gemm_stacked_parts(cuda, M, K):
+    """The parts of two matrices stacked under one shared table: each part's
+    product is its own matrix's, bit for bit (the decoded values are)."""
+    from gpu_huffman_functions import build_split, split_prefill, stack_split, stacked_parts
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    ws = [(torch.randn(M, K, device=cuda, generator=g) * 0.02).bfloat16() for _ in range(2)]
+    cb, lut = cbb.codebook_from_counts_torch(cbb.counts_torch(ws[0]) + cbb.counts_torch(ws[1]))
+    sps = [build_split(lut[cbb.patterns_torch(w).reshape(-1).to(torch.int64)].to(torch.int32),
+                       cb.cpu().numpy(), cuda) for w in ws]
+    keep, _, parts = stack_split(sps, cb.cpu().numpy(), [M, M], K, cuda)
+    x = torch.randn(33, K, device=cuda, generator=g)
+    for own, part, w in zip(sps, stacked_parts(keep, parts), ws):
+        y = split_prefill(part, None, x, M, K, cb, finite=True)
+        assert torch.equal(y, split_prefill(own, None, x, M, K, cb, finite=True))
+        assert _rel(y, x.double() @ w.double().T) <= TOL_F32
+
+
 def test_split_gemm_refuses(cuda):
     import cbq_ops
     t, _ = _split_matrix(cuda, 4, 1024, 1)
