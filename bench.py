@@ -336,18 +336,12 @@ def huffman_sweep(torch, nat, lib, dev, huff, splits, plan, steps, warmup):
 
 # ---- sections ------------------------------------------------------------------
 
-def xf_bytes(T, K):
-    """Bytes of the fragment-order copy of x at the front of the
-    cbq_linear_bf16_ws workspace (the rest holds split-K partials: whole
-    small grids, or the tiles left after the last full round of CUs)."""
-    return ((T + 15) // 16 * 16 * K * 2 + 255) // 256 * 256
-
-
 def prefill_section(torch, nat, lib, dev, fixed, kinds, args):
     """benchmark config 4: bf16 MFMA prefill over the same fixed-width weights,
     T = 512 and 2048 tokens of bf16 N(0, 1) activations; per shape the mean
-    time of one cbq_linear_bf16_ws call (the x fragment-order copy, the GEMM
-    and, when K is split, the partial sum) over 8 layers' distinct weights
+    time of one cbq_linear_bf16_ws call with the workspace the module gives it
+    (x and, where that is faster, the weights as MFMA fragments, the GEMM and,
+    when K is split, the partial sum) over 8 layers' distinct weights
     (graph-replayed)."""
     out = {"peak_tflops": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "shapes": {}}
     for T in (512, 2048):
@@ -357,8 +351,8 @@ def prefill_section(torch, nat, lib, dev, fixed, kinds, args):
             M, K = t0.shape
             x = torch.randn(T, K, device=dev).bfloat16()
             o = torch.empty(T, M, device=dev, dtype=torch.bfloat16)
-            nws = int(lib.cbq_linear_bf16_workspace(T, M, K))
-            ws = torch.empty(max(1, nws // 4), dtype=torch.float32, device=dev)
+            nws = int(lib.cbq_linear_bf16_gemm_workspace(T, M, K, t0.bits))
+            ws = torch.empty(max(1, (nws + 3) // 4), dtype=torch.float32, device=dev)
 
             def run(ns=ns, x=x, o=o, ws=ws, nws=nws):
                 st = nat.stream_ptr(dev)
@@ -373,7 +367,7 @@ def prefill_section(torch, nat, lib, dev, fixed, kinds, args):
             us = ms * 1e3 / len(ns)
             tf = 2.0 * T * M * K / (us * 1e-6) / 1e12
             out["shapes"][f"T{T}_{kind}"] = {"shape": f"{K}->{M}", "us_per_launch": round(us, 1),
-                                             "split_partials_MB": round((nws - xf_bytes(T, K)) / 1e6, 1),
+                                             "workspace_MB": round(nws / 1e6, 1),
                                              "TFLOP/s": round(tf, 1),
                                              "frac": round(tf / MFMA_BF16_PEAK_TFLOPS, 4)}
     g = out["shapes"]["T2048_gate_proj"]
