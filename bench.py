@@ -109,16 +109,7 @@ def timed_graph(torch, fn, reps, warmup):
     return e0.elapsed_time(e1) / reps, g
 
 
-PREFILL_PROFILE = "fixed_prefill_kernel_qwen3-8b_T512_T2048.md"
-
-
-def read_profile_value(name, pattern, scale=1.0):
-    """A figure from a committed rocprofv3 summary, if any."""
-    p = os.path.join(ROOT, "profiles", name)
-    if not os.path.exists(p):
-        return None
-    m = re.search(pattern, open(p).read())
-    return round(float(m.group(1)) * scale, 4) if m else None
+PREFILL_PROFILE = "frag_gemm_kernel_qwen3-8b_prompts.md"
 
 
 def read_traffic(name):
@@ -373,9 +364,8 @@ def prefill_section(torch, nat, lib, dev, fixed, kinds, args):
     g = out["shapes"]["T2048_gate_proj"]
     out["roofline"] = {"bound": "mfma", "achieved": g["TFLOP/s"], "peak": MFMA_BF16_PEAK_TFLOPS,
                        "unit": "TFLOP/s", "frac": g["frac"],
-                       "kernel": "fixed_prefill_kernel<13> gate/up 4096->12288, T=2048",
-                       "mfma_busy_rocprof_full_round_launch": read_profile_value(
-                           PREFILL_PROFILE, r"\*\*MFMA busy ([0-9.]+) %\*\*", 0.01),
+                       "kernel": "frag_prep_kernel<13, 1> + frag_gemm_kernel, gate/up "
+                                 "4096->12288, T=2048",
                        "profile": "profiles/" + PREFILL_PROFILE}
     return out
 
