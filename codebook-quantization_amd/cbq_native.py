@@ -131,6 +131,7 @@ SIGNATURES = {
                                          + [_vp]),
     "cbq_argmax_step": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i64, _i64, _vp]),
     "cbq_silu_mul_f32": (_i, [_vp, _vp, _vp, _i64, _vp]),
+    "cbq_causal_softmax_f32": (_i, [_vp, _i64, _i, _i, _i, ctypes.c_float, _vp]),
 }
 
 _lib: Optional[ctypes.CDLL] = None

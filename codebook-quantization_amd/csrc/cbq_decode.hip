@@ -1,7 +1,7 @@
 // Fused fp32 decoder glue for gfx950: residual add + RMSNorm, per-head
 // RMSNorm + rotary embedding + KV-cache write, single-token grouped-query
-// attention (alone or with the head norm, rope and cache write folded in),
-// the SiLU-gated product and the greedy pick.  HF Qwen3 semantics (the modelling
+// attention (alone or with the head norm, rope and cache write folded in), the
+// causal softmax of a prompt's scores, the SiLU-gated product and the greedy pick.  HF Qwen3 semantics (the modelling
 // code the reference's compressed modules plug into,
 // src/model_loader.py:213-277); products and sums that PyTorch rounds one at
 // a time are rounded one at a time here too (no contraction into FMAs),
@@ -669,6 +669,54 @@ __global__ __launch_bounds__(kGlueBlock) void silu_mul_kernel(const float *__res
     }
 }
 
+// Causal softmax over the rows of a prompt's scores, in place.  Row r of a kv
+// group's T * rep is token (r / rep) and sees the first L - T + r / rep + 1
+// keys; the rest become 0.  One wave per row, no LDS; rows of up to 64 N keys
+// stay in registers (one read, one write), N = 0 reads its row three times
+// (from the L2 by then).  Bound by launches at the lengths of a prompt: it
+// stands for seven elementwise launches and a softmax, with the same
+// roundings (product, difference, exp, quotient).
+template <int N>
+__global__ __launch_bounds__(kGlueBlock) void causal_softmax_kernel(float *__restrict__ s,
+                                                                   int64_t rows, int per, int rep,
+                                                                   int T, int L, float scale)
+{
+    const int64_t row = (int64_t)blockIdx.x * (kGlueBlock / CBQ_WAVE) + threadIdx.x / CBQ_WAVE;
+    if (row >= rows) return;
+    const int lane = threadIdx.x & (CBQ_WAVE - 1);
+    const int vis = L - T + (int)(row % per) / rep + 1;          // <= L
+    float *const p = s + row * L;
+    float m = -INFINITY, sum = 0.f;
+    if constexpr (N > 0) {
+        float v[N];
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const int j = i * CBQ_WAVE + lane;
+            v[i] = j < vis ? p[j] * scale : -INFINITY;
+            m = fmaxf(m, v[i]);
+        }
+        m = wave_max(m);
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            v[i] = i * CBQ_WAVE + lane < vis ? expf(v[i] - m) : 0.f;
+            sum += v[i];
+        }
+        sum = wave_sum(sum);
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const int j = i * CBQ_WAVE + lane;
+            if (j < L) p[j] = v[i] / sum;
+        }
+    } else {
+        for (int j = lane; j < vis; j += CBQ_WAVE) m = fmaxf(m, p[j] * scale);
+        m = wave_max(m);
+        for (int j = lane; j < vis; j += CBQ_WAVE) sum += expf(p[j] * scale - m);
+        sum = wave_sum(sum);
+        for (int j = lane; j < L; j += CBQ_WAVE)
+            p[j] = (j < vis ? expf(p[j] * scale - m) : 0.f) / sum;
+    }
+}
+
 }  // namespace
 
 int cbq_argmax_merge(const float *part_v, const int *part_i, int n_part, int n, int32_t *ids32,
@@ -912,6 +960,28 @@ int cbq_silu_mul_f32(const float *g, const float *u, float *out, int64_t n, hipS
     const int blocks = (int)(want < 4096 ? want : 4096);
     hipLaunchKernelGGL(silu_mul_kernel, dim3(blocks), dim3(kGlueBlock), 0, stream, g, u, out, n);
     return cbq_launch_status("silu_mul_kernel");
+}
+
+int cbq_causal_softmax_f32(float *scores, int64_t rows, int T, int rep, int L, float scale,
+                           hipStream_t stream)
+{
+    if (!scores || rows <= 0 || T <= 0 || rep <= 0 || L < T || (int64_t)T * rep > INT32_MAX ||
+        rows % ((int64_t)T * rep) != 0)
+        return CK_ERR_ARG;
+    constexpr int kRows = kGlueBlock / CBQ_WAVE;
+    const int64_t blocks = (rows + kRows - 1) / kRows;
+    if (blocks > INT32_MAX / kGlueBlock) return CK_ERR_ARG;
+    const dim3 grid((unsigned)blocks), block(kGlueBlock);
+    if (L <= 4 * CBQ_WAVE)
+        hipLaunchKernelGGL(causal_softmax_kernel<4>, grid, block, 0, stream, scores, rows, T * rep,
+                           rep, T, L, scale);
+    else if (L <= 16 * CBQ_WAVE)
+        hipLaunchKernelGGL(causal_softmax_kernel<16>, grid, block, 0, stream, scores, rows, T * rep,
+                           rep, T, L, scale);
+    else
+        hipLaunchKernelGGL(causal_softmax_kernel<0>, grid, block, 0, stream, scores, rows, T * rep,
+                           rep, T, L, scale);
+    return cbq_launch_status("causal_softmax_kernel");
 }
 
 }  // extern "C"

@@ -152,6 +152,14 @@ class _Glue:
             pos_dev.data_ptr(), first, toks.numel(), self.nat.stream_ptr(logits.device)),
             "cbq_argmax_step")
 
+    def causal_softmax(self, scores: torch.Tensor, T: int, rep: int, scale: float) -> torch.Tensor:
+        """softmax(scores * scale) over each token's keys, in place: scores
+        [n_kv, T * rep, L], the T tokens at the last positions."""
+        self.nat.check(self.lib.cbq_causal_softmax_f32(
+            scores.data_ptr(), scores.shape[0] * scores.shape[1], T, rep, scores.shape[2], scale,
+            self.nat.stream_ptr(scores.device)), "cbq_causal_softmax_f32")
+        return scores
+
     def silu_mul(self, g: torch.Tensor, u: torch.Tensor) -> torch.Tensor:
         out = torch.empty_like(g)
         self.nat.check(self.lib.cbq_silu_mul_f32(g.data_ptr(), u.data_ptr(), out.data_ptr(),
@@ -190,8 +198,9 @@ class Qwen3Decoder:
                       all(callable(getattr(linears.get(n), "xform", None)) for n in need))
 
     # ---- building blocks (HF Qwen3 semantics, fp32) -------------------------
-    def _attend(self, i: int, q: torch.Tensor, L: int, pos: torch.Tensor) -> torch.Tensor:
-        """Causal GQA over cache positions [0, L): q [T, n_q, hd] -> [T, n_q*hd].
+    def _attend(self, i: int, q: torch.Tensor, L: int) -> torch.Tensor:
+        """Causal GQA over cache positions [0, L): q [T, n_q, hd] at the last T
+        of them -> [T, n_q*hd].
         Query head h reads kv head h // (n_q / n_kv), as HF's repeat_kv; the
         grouping is a reshape, so no kv copy is made."""
         c = self.cfg
@@ -201,20 +210,16 @@ class Qwen3Decoder:
         vv = self.cache[i, 1, :, :L]
         qg = q.reshape(T, c.n_kv, rep, c.head_dim).permute(1, 0, 2, 3).reshape(c.n_kv, T * rep,
                                                                             c.head_dim)
-        scores = torch.matmul(qg, kk.transpose(1, 2).contiguous()) * (c.head_dim ** -0.5)
-        # query row r of group g is token r // rep
-        tpos = pos.repeat_interleave(rep)                               # [T * rep]
-        causal = torch.arange(L, device=self.device)[None, :] > tpos[:, None]
-        scores = scores.masked_fill(causal[None], float("-inf"))
-        probs = torch.softmax(scores, dim=-1)
+        scores = torch.matmul(qg, kk.transpose(1, 2).contiguous())
+        probs = self.glue.causal_softmax(scores, T, rep, c.head_dim ** -0.5)
         att = torch.matmul(probs, vv)                                   # [n_kv, T*rep, hd]
         return att.reshape(c.n_kv, T, rep, c.head_dim).permute(1, 0, 2, 3).reshape(
             T, c.n_q * c.head_dim)
 
-    def _layer(self, i: int, h: torch.Tensor, x: torch.Tensor, pos: torch.Tensor,
-               pos_dev: torch.Tensor, L: int) -> torch.Tensor:
-        """One layer over T tokens at positions pos (pos_dev: device int64
-        holding pos[0]; L = pos[-1] + 1, or max_len for the captured step).
+    def _layer(self, i: int, h: torch.Tensor, x: torch.Tensor, pos_dev: torch.Tensor,
+               L: int) -> torch.Tensor:
+        """One layer over T consecutive tokens (pos_dev: device int64 holding
+        the first position; L: the last + 1, or max_len for the captured step).
         x = rmsnorm(h) on entry; h is updated in place; returns the next
         rmsnorm(h)."""
         c = self.cfg
@@ -237,7 +242,7 @@ class Qwen3Decoder:
         else:
             q = g.head_norm_rope(q, k, v, self.cos, self.sin, pos_dev, self.cache[i, 0],
                                  self.cache[i, 1])
-            att = self._attend(i, q.view(T, c.n_q, c.head_dim), L, pos)
+            att = self._attend(i, q.view(T, c.n_q, c.head_dim), L)
         x = g.add_rms(h, self.linears[p + "self_attn.o_proj"](att))
         gu = self.linears.get(p + "mlp.gate_up_proj")
         if gu is not None:                           # row-stacked gate/up: one launch
@@ -263,7 +268,7 @@ class Qwen3Decoder:
         else:
             x = self.glue.add_rms(h, None)
             for i in range(c.layers):
-                x = self._layer(i, h, x, pos_buf, pos_buf, self.max_len)
+                x = self._layer(i, h, x, pos_buf, self.max_len)
             logits = self.linears["lm_head"](x).reshape(-1)
         self.glue.argmax_step(logits, ids_buf, toks, pos_buf, first_pos)
 
@@ -355,8 +360,7 @@ class Qwen3Decoder:
         T = int(ids.numel())
         if self.pos + T > self.max_len:
             raise ValueError(f"sequence of {self.pos + T} exceeds max_len {self.max_len}")
-        pos = torch.arange(self.pos, self.pos + T, device=self.device)
-        pos_dev = pos[:1].contiguous()
+        pos_dev = torch.full((1,), self.pos, dtype=torch.int64, device=self.device)
         h = self.embed(ids.to(self.device)).reshape(T, self.cfg.hidden).to(torch.float32)
         if T == 1 and self.fused:
             logits = self._forward1_fused(h, pos_dev)
@@ -364,7 +368,7 @@ class Qwen3Decoder:
             return logits
         x = self.glue.add_rms(h, None)
         for i in range(self.cfg.layers):
-            x = self._layer(i, h, x, pos, pos_dev, self.pos + T)
+            x = self._layer(i, h, x, pos_dev, self.pos + T)
         self.pos += T
         return self.linears["lm_head"](x[-1:]).reshape(-1)
 

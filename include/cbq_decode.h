@@ -118,6 +118,13 @@ int cbq_argmax_step(const float *logits, int n, void *workspace, int32_t *ids32,
 int cbq_silu_mul_f32(const float *g, const float *u, float *out, int64_t n,
                      hipStream_t stream);
 
+/* Causal softmax of a prompt's scores, in place: scores [rows, L], rows a
+ * multiple of T * rep (per kv head, T tokens of rep query heads each).  Token
+ * t sees keys 0 .. L - T + t: softmax(scores * scale) over them, 0 after
+ * them. */
+int cbq_causal_softmax_f32(float *scores, int64_t rows, int T, int rep, int L,
+                           float scale, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

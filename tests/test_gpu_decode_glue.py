@@ -137,6 +137,32 @@ def test_silu_mul(cuda, lib):
     assert _rel(out, ref) <= 1e-6
 
 
+@pytest.mark.parametrize("n_kv,rep,T,L", [(1, 1, 2, 2), (2, 3, 5, 63), (8, 2, 200, 200),
+                                          (2, 4, 7, 256), (2, 1, 257, 257), (1, 3, 3, 1024),
+                                          (2, 2, 9, 1025), (1, 2, 1100, 1500)])
+def test_causal_softmax(cuda, lib, n_kv, rep, T, L):
+    """Against float64 at the edges of the register sizes.  An element's error:
+    a product, a difference and a quotient of half an ulp each (the first two
+    scaled by |x| <= 16), an exp of 1 ulp and a sum of L / 64 + 6 roundings."""
+    s = torch.randn(n_kv, T * rep, L, device=cuda, generator=torch.Generator(device=cuda)
+                    .manual_seed(L)) * 10
+    s[0, 0, L - 1] = float("nan")                       # a key the first token does not see
+    s[0, T * rep - 1, 0] = float("-inf")
+    if rep > 1:
+        s[n_kv - 1, T * rep - 1, L - 1] = float("inf")   # inf - inf: the whole row NaN
+    scale = 0.088388346
+    first = torch.arange(T, device=cuda).repeat_interleave(rep) + L - T
+    masked = torch.arange(L, device=cuda)[None, :] > first[:, None]
+    ref = torch.softmax((s.double() * float(np.float32(scale))).masked_fill(masked, float("-inf")), -1)
+    nat.check(lib.cbq_causal_softmax_f32(s.data_ptr(), n_kv * T * rep, T, rep, L, scale,
+                                         nat.stream_ptr(cuda)), "softmax")
+    assert torch.equal(s.isnan(), ref.isnan())
+    assert bool((s.masked_select(masked[None] & ~ref.isnan()) == 0).all())
+    ok = ~ref.isnan()
+    bound = (2 * 16 + 2 + L / 64 + 6) * 2.0 ** -24
+    assert bool(((s.double() - ref).abs()[ok] <= bound * ref[ok] + 1e-37).all())
+
+
 @pytest.mark.parametrize("hd,n_q,n_kv,pos0,max_len", [(128, 32, 8, 0, 512), (128, 32, 8, 200, 512),
                                                       (64, 4, 2, 63, 64), (256, 8, 2, 17, 64)])
 def test_attn_rope_decode_matches_two_step(cuda, lib, hd, n_q, n_kv, pos0, max_len):
