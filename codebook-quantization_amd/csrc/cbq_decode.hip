@@ -672,10 +672,12 @@ __global__ __launch_bounds__(kGlueBlock) void silu_mul_kernel(const float *__res
 // Causal softmax over the rows of a prompt's scores, in place.  Row r of a kv
 // group's T * rep is token (r / rep) and sees the first L - T + r / rep + 1
 // keys; the rest become 0.  One wave per row, no LDS; rows of up to 64 N keys
-// stay in registers (one read, one write), N = 0 reads its row three times
-// (from the L2 by then).  Bound by launches at the lengths of a prompt: it
-// stands for seven elementwise launches and a softmax, with the same
-// roundings (product, difference, exp, quotient).
+// stay in registers (one read, one write), N = 0 reads its row three times.
+// Bound by the launch up to some 500 tokens, by memory beyond.  The product,
+// index range, comparison, mask fill and softmax it stands for, as torch
+// operations, with the same roundings: 37 us at T = L = 200 (8 kv heads,
+// rep 2), 96 at 1024, 1595 at 4096; here 6.7 (calls back to back from
+// Python), 24 and 650.
 template <int N>
 __global__ __launch_bounds__(kGlueBlock) void causal_softmax_kernel(float *__restrict__ s,
                                                                    int64_t rows, int per, int rep,
