@@ -346,13 +346,15 @@ struct GemmArgs {
 // One fragment (1 KiB, lane l's 16 bytes at + 16 l) from global memory to LDS
 // offset dst (wave-uniform).  Written as asm so that the compiler does not
 // order LDS reads behind it: the K loop's own waits do.  M0 holds the LDS
-// address; one wait state is needed between its write and the load.
+// address; one wait state is needed between its write and the load, and five
+// between a VALU write of the address's scalar registers (v_readfirstlane)
+// and the load: the compiler does not count them inside inline assembly.
 __device__ __forceinline__ void lds_copy_frag(uint32_t dst, const uint8_t *src, uint32_t lane16)
 {
     const uint64_t p = (uint64_t)src;              // wave-uniform, in scalar registers
     const uint64_t q = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)p) |
                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(p >> 32)) << 32;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2"
                  :: "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(lane16), "s"(q) : "m0");
 }
 
