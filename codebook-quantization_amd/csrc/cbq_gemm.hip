@@ -316,9 +316,13 @@ template <int NP_, int TB_, int MB_, int WT_, int WM_, int NST_> struct GemmCfg 
 // The K loop's stages for WP parts of W: one column group, all its parts.
 template <class C, int WP> struct GemmStage {
     static constexpr int NST = WP == 1 ? C::NST : 2;
-    // stages between a buffer's last read and its reuse: 1 leaves the reads in
+    // stages between a buffer's last read and its reuse: 1 leaves reads in
     // flight over the barrier, at the price of a stage of LDS
     static constexpr int LAG = NST >= 4 ? 1 : 0;
+    // LDS reads of the running stage that may be in flight at its barrier:
+    // those of its only product, or with several x parts of its last one.
+    // LDS answers in order, so the stage before it has been read.
+    static constexpr int READS = LAG == 0 ? 0 : C::NP > 1 ? C::TB : C::TB + C::MB;
     static constexpr int PIECES = C::NA * C::NP + C::NB * WP;
     static constexpr int PL = (PIECES + kGWaves - 1) / kGWaves;   // copies per wave and stage
     static constexpr int BYTES = PIECES * (int)kFrag;
@@ -358,14 +362,12 @@ __device__ __forceinline__ void lds_copy_frag(uint32_t dst, const uint8_t *src, 
                  :: "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(lane16), "s"(q) : "m0");
 }
 
-// The wave's copies but the newest N have landed in LDS (READS: and its LDS
-// reads are done); then the block's barrier: every wave's.
-template <int N, bool READS> __device__ __forceinline__ void stage_barrier()
+// The wave's copies but the newest N have landed in LDS, and its LDS reads but
+// the newest R are done; then the block's barrier: every wave's.
+template <int N, int R> __device__ __forceinline__ void stage_barrier()
 {
-    if constexpr (READS)
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
-    else
-        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(N) : "memory");
+    static_assert(N >= 0 && N < 64 && R >= 0 && R < 16, "counter widths");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(%1)\n\ts_barrier" :: "n"(N), "n"(R) : "memory");
 }
 
 __device__ __forceinline__ uint32_t bf16_pair(float a, float b)
@@ -538,10 +540,9 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
         uint32_t old = (NST - 1) * STAGE;                   // and of the one before it
         // One stage whose first fragments are in fa[P0] / fb[Q0]: the next
         // product's fragments are read while the current one runs.  Before
-        // the last product's MFMAs every wave has read the stage (LAG 0:
-        // waited for here) or at least the one before it, whose MFMAs have
-        // been issued (LAG 1), so the barrier frees that LDS for the next
-        // copies and publishes the next stage.
+        // the last product's MFMAs every wave has waited for its reads of the
+        // stage (LAG 0) or of the one before it (LAG 1), so the barrier frees
+        // that LDS for the next copies and publishes the next stage.
         // With three x parts the copies into it are spread over that
         // product's MFMAs: a wave that issues them all at once waits in the
         // memory pipeline's queue before its MFMAs (T = 1024, 8192 x 4096:
@@ -562,7 +563,7 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
                 cbq_u32x4 (&bn)[MB] = fb[q ^ 1];
                 const uint32_t free_buf = LAG ? old : cur;
                 if (last) {
-                    stage_barrier<(NST - 2 - LAG) * PL, LAG == 0>();
+                    stage_barrier<(NST - 2 - LAG) * PL, St::READS>();
                     old = cur;
                     cur = cur + STAGE == NST * STAGE ? 0u : cur + STAGE;
                 }
@@ -614,7 +615,7 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
             for (int i = 0; i < PL; i++) copy(b * STAGE, i);
             advance();
         }
-        stage_barrier<(NST - 1 - LAG) * PL, true>();
+        stage_barrier<(NST - 1 - LAG) * PL, 0>();
 #pragma unroll
         for (int i = 0; i < TB; i++) read_a(0, 0, i, fa[0]);
 #pragma unroll

@@ -80,3 +80,19 @@ def test_copy_addresses_wait_for_valu_writes(kernels):
                 states += int(args, 0) + 1 if op == "s_nop" else 1
     assert copies > 100
     assert not early, f"{len(early)} of {copies}: {early[0]}"
+
+
+def test_barriers_bound_the_lds_reads(kernels):
+    """The barrier before a stage's LDS is written again waits for the reads
+    of that stage: each carries a bound on the LDS reads in flight.  At most
+    the 12 of a stage's first product (8 + 4 fragments) may be newer."""
+    barriers = 0
+    for name, ins in kernels.items():
+        for i, line in enumerate(ins):
+            if line != "s_barrier":
+                continue
+            barriers += 1
+            m = re.search(r"lgkmcnt\((\d+)\)", ins[i - 1])
+            assert ins[i - 1].startswith("s_waitcnt") and m and int(m.group(1)) <= 12, \
+                (name, ins[i - 1])
+    assert barriers > 40
