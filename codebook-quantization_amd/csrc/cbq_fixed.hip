@@ -1095,7 +1095,8 @@ int cbq_prefill_bf16(const uint16_t *x, const uint8_t *packed, const float *cb, 
 size_t cbq_prefill_ws_bytes(int T, int M, int K);
 // fp32 MFMA prefill path (cbq_prefill_f32.hip); -1 = shape not handled there.
 int cbq_prefill_f32(const float *x, const uint8_t *packed, const float *cb, float *out, int T,
-                    int M, int K, int C, int bits, hipStream_t st);
+                    int M, int K, int C, int bits, hipStream_t st, int S, float *ws);
+int cbq_prefill_f32_splits(int T, int M, int K);
 // decode-first GEMM on the bf16 matrix cores, with a workspace (cbq_gemm.hip);
 // -1 = not handled there.
 int cbq_frag_linear(const void *x, bool f32, const uint8_t *packed, const float *cb, void *out,
@@ -1138,10 +1139,18 @@ int ck_linear_f32(const float *x, const uint8_t *packed, const float *codebook, 
     // T >= 64: the GEMM regime, fp32 MFMA (cbq_prefill_f32.hip)
     if (x && packed && codebook && out && T >= 64 && M > 0 && K > 0 && C > 0 && bits >= 1 &&
         bits <= 16) {
-        const int rc = cbq_prefill_f32(x, packed, codebook, out, T, M, K, C, bits, stream);
+        const int rc = cbq_prefill_f32(x, packed, codebook, out, T, M, K, C, bits, stream, 1,
+                                       nullptr);
         if (rc >= 0) return rc;
     }
     return linear_any_t<float, float>(x, packed, codebook, out, T, M, K, C, bits, stream);
+}
+
+// Bytes of the fp32 kernel's split-K partials (0: no split).
+static size_t prefill_f32_partials(int T, int M, int K)
+{
+    const int S = cbq_prefill_f32_splits(T, M, K);
+    return S > 1 ? (size_t)S * T * M * sizeof(float) : 0;
 }
 
 size_t cbq_linear_f32_workspace(int T, int M, int K)
@@ -1160,6 +1169,11 @@ int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebo
         if (rc < 0)
             rc = cbq_frag_linear(x, true, packed, codebook, out, T, M, K, C, bits, workspace,
                                  ws_bytes, stream);
+        // a workspace below the GEMM's: the fp32 kernel with split K
+        const size_t split = rc < 0 ? prefill_f32_partials(T, M, K) : 0;
+        if (split && workspace && ws_bytes >= split && ((uintptr_t)workspace & 15) == 0)
+            rc = cbq_prefill_f32(x, packed, codebook, out, T, M, K, C, bits, stream,
+                                 cbq_prefill_f32_splits(T, M, K), (float *)workspace);
         if (rc >= 0) return rc;
     }
     return ck_linear_f32(x, packed, codebook, out, T, M, K, C, bits, stream);

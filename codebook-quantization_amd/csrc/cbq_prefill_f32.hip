@@ -14,9 +14,11 @@
 // [128][32] (4 threads per row, 8 indices each, gathered from an LDS fp32
 // codebook padded to 2^BITS, which is the reference's clamp) into LDS; each
 // wave then runs 2 x 2 x 16 MFMAs on its 64 x 64 sub-tile.  x and index
-// words of the next two K steps are held in registers.  This is the path of
-// callers without a workspace (ck_linear_f32); with one, cbq_linear_f32_ws
-// runs the decode-first GEMM of cbq_gemm.hip on the bf16 matrix cores.
+// words of the next two K steps are held in registers.  With split K (a
+// caller workspace), block z sums only its share of the K steps and writes an
+// fp32 partial tile; a second kernel adds the partials in order.
+// This is the path of callers without a workspace (ck_linear_f32) or with one
+// below what the decode-first GEMM of cbq_gemm.hip needs (cbq_linear_f32_ws).
 #include "cbq_device.h"
 
 #include <algorithm>
@@ -153,10 +155,13 @@ __device__ __forceinline__ void prefill_f32_loop(
     }
 }
 
-template <int BITS>
+// SPLIT: block z sums only K groups [z * gs, z * gs + gs) and writes its fp32
+// partial tile to ws + z * T * M; prefill_f32_reduce_kernel adds the partials.
+template <int BITS, bool SPLIT>
 __global__ __launch_bounds__(kFBlock) void fixed_prefill_f32_kernel(
     const float *__restrict__ x, const uint32_t *__restrict__ words,
-    const float *__restrict__ cb, float *__restrict__ out, int T, int M, int K, int C)
+    const float *__restrict__ cb, float *__restrict__ out, int T, int M, int K, int C,
+    float *__restrict__ ws, int gs)
 {
     __shared__ __attribute__((aligned(16))) float s_cb[1 << BITS];       // padded codebook
     __shared__ __attribute__((aligned(16))) float s_x[kFT * kFK];      // [256][32]
@@ -166,7 +171,9 @@ __global__ __launch_bounds__(kFBlock) void fixed_prefill_f32_kernel(
     const int lane = tid & (CBQ_WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / CBQ_WAVE);
     const int t0 = blockIdx.x * kFT, m0 = blockIdx.y * kFM;
-    const int G = K / kFK;
+    const int G_all = K / kFK;
+    const int g_lo = SPLIT ? (int)blockIdx.z * gs : 0;
+    const int G = SPLIT ? min(G_all, g_lo + gs) - g_lo : G_all;
 
     stage_clamped(s_cb, cb, C < (1 << BITS) ? C : (1 << BITS), 1 << BITS);
     // (the loop's first barrier publishes the codebook)
@@ -174,13 +181,13 @@ __global__ __launch_bounds__(kFBlock) void fixed_prefill_f32_kernel(
     // x staging: thread -> tile row tid/2, k half tid%2 (clamped row)
     const int xr = tid >> 1, hx = tid & 1;
     const int xt = min(t0 + xr, T - 1);
-    const float *xrow = x + (size_t)xt * K + hx * 16;
+    const float *xrow = x + (size_t)xt * K + (size_t)g_lo * kFK + hx * 16;
     // W decode: wave w takes part w % 4 (indices 8*part .. +7 of each group)
     // of tile rows 64*(w / 4) + lane, so the part is wave-uniform
     const int wr = ((wave >> 2) << 6) + lane, wp = wave & 3;
     const int wm = min(m0 + wr, M - 1);
     const int q0 = (wp * 8 * BITS) >> 5;
-    const uint32_t *wrow = words + (size_t)wm * G * BITS + q0;
+    const uint32_t *wrow = words + ((size_t)wm * G_all + g_lo) * BITS + q0;
 
     f32x16 acc[2][2];
 #pragma unroll
@@ -214,36 +221,81 @@ __global__ __launch_bounds__(kFBlock) void fixed_prefill_f32_kernel(
                 for (int j = 0; j < 4; j++) {
                     const int t = t0 + wt + a * 32 + i * 8 + (lane >> 5) * 4 + j;
                     if (t >= T) continue;
-                    out[(size_t)t * M + m] = acc[a][b][i * 4 + j];
+                    if (SPLIT)
+                        ws[((size_t)blockIdx.z * T + t) * M + m] = acc[a][b][i * 4 + j];
+                    else
+                        out[(size_t)t * M + m] = acc[a][b][i * 4 + j];
                 }
         }
 }
 
+// out = sum over s of ws[s], s in order.
+__global__ void prefill_f32_reduce_kernel(const float *__restrict__ ws, int S, int64_t n,
+                                          float *__restrict__ out)
+{
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+        float t = ws[i];
+        for (int s = 1; s < S; s++) t += ws[s * n + i];
+        out[i] = t;
+    }
+}
+
 template <int BITS>
 int launch_prefill_f32(const float *x, const uint8_t *packed, const float *cb, float *out, int T,
-                       int M, int K, int C, hipStream_t st)
+                       int M, int K, int C, int S, float *ws, hipStream_t st)
 {
-    dim3 grid((unsigned)((T + kFT - 1) / kFT), (unsigned)((M + kFM - 1) / kFM));
-    hipLaunchKernelGGL((fixed_prefill_f32_kernel<BITS>), grid, dim3(kFBlock), 0, st, x,
-                       (const uint32_t *)packed, cb, out, T, M, K, C);
-    return cbq_launch_status("fixed_prefill_f32_kernel");
+    const int G = K / kFK;
+    if (S <= 1) {
+        dim3 grid((unsigned)((T + kFT - 1) / kFT), (unsigned)((M + kFM - 1) / kFM));
+        hipLaunchKernelGGL((fixed_prefill_f32_kernel<BITS, false>), grid, dim3(kFBlock), 0, st,
+                           x, (const uint32_t *)packed, cb, out, T, M, K, C, (float *)nullptr, G);
+        return cbq_launch_status("fixed_prefill_f32_kernel");
+    }
+    const int gs = (G + S - 1) / S;
+    S = (G + gs - 1) / gs;                                   // no empty split
+    dim3 grid((unsigned)((T + kFT - 1) / kFT), (unsigned)((M + kFM - 1) / kFM), (unsigned)S);
+    hipLaunchKernelGGL((fixed_prefill_f32_kernel<BITS, true>), grid, dim3(kFBlock), 0, st, x,
+                       (const uint32_t *)packed, cb, out, T, M, K, C, ws, gs);
+    int rc = cbq_launch_status("fixed_prefill_f32_kernel");
+    if (rc) return rc;
+    const int64_t n = (int64_t)T * M;
+    const int blocks = (int)std::min<int64_t>((n + 255) / 256, 4096);
+    hipLaunchKernelGGL(prefill_f32_reduce_kernel, dim3(blocks), dim3(256), 0, st, ws, S, n, out);
+    return cbq_launch_status("prefill_f32_reduce_kernel");
 }
 
 }  // namespace
 
-// fp32 MFMA prefill used by ck_linear_f32; -1 = shape not handled here.
+// K splits for a T x M x K fp32 prefill: the matrix cores are the bound here,
+// so every grid under two blocks per CU splits, into enough blocks to cover
+// the CUs twice, with at least 8 K groups per split and at most 16 splits.
+int cbq_prefill_f32_splits(int T, int M, int K)
+{
+    if (T < 64 || K % kFK != 0) return 1;
+    const int64_t tiles = (int64_t)((T + kFT - 1) / kFT) * ((M + kFM - 1) / kFM);
+    const int64_t want = 2 * (int64_t)cbq_num_cus();
+    if (tiles >= want) return 1;
+    int S = (int)std::min<int64_t>((want + tiles - 1) / tiles, 16);
+    S = std::min(S, (K / kFK) / 8);
+    return S < 2 ? 1 : S;
+}
+
+// fp32 MFMA prefill used by ck_linear_f32; -1 = shape not handled here.  S > 1
+// splits K, with S * T * M floats of workspace.
 int cbq_prefill_f32(const float *x, const uint8_t *packed, const float *cb, float *out, int T,
-                    int M, int K, int C, int bits, hipStream_t st)
+                    int M, int K, int C, int bits, hipStream_t st, int S, float *ws)
 {
     if (T < 64 || K % kFK != 0 || (((uintptr_t)packed | (uintptr_t)x) & 15) != 0 ||
         (size_t)T > 65535ull * kFT || M > 65535 * kFM)
         return -1;
+    if (S > 1 && !ws) return -1;
     switch (bits) {
-    case 8: return launch_prefill_f32<8>(x, packed, cb, out, T, M, K, C, st);
-    case 10: return launch_prefill_f32<10>(x, packed, cb, out, T, M, K, C, st);
-    case 11: return launch_prefill_f32<11>(x, packed, cb, out, T, M, K, C, st);
-    case 12: return launch_prefill_f32<12>(x, packed, cb, out, T, M, K, C, st);
-    case 13: return launch_prefill_f32<13>(x, packed, cb, out, T, M, K, C, st);
+    case 8: return launch_prefill_f32<8>(x, packed, cb, out, T, M, K, C, S, ws, st);
+    case 10: return launch_prefill_f32<10>(x, packed, cb, out, T, M, K, C, S, ws, st);
+    case 11: return launch_prefill_f32<11>(x, packed, cb, out, T, M, K, C, S, ws, st);
+    case 12: return launch_prefill_f32<12>(x, packed, cb, out, T, M, K, C, S, ws, st);
+    case 13: return launch_prefill_f32<13>(x, packed, cb, out, T, M, K, C, S, ws, st);
     default: return -1;
     }
 }

@@ -59,7 +59,9 @@ size_t cbq_linear_f32_workspace(int T, int M, int K);
  * over blocks when the output tiles alone would leave CUs idle (partials in
  * the workspace, summed in split order).  A codebook with values that are
  * not bf16 numbers is split into bf16 parts as well.  With a smaller
- * workspace it is ck_linear_f32.  No counterpart in the reference: batched
+ * workspace it is ck_linear_f32, whose fp32 kernel (T >= 64) then splits K
+ * where it would leave CUs idle and the partials (fp32 [splits][T][M], at most
+ * 16 splits) fit.  No counterpart in the reference: batched
  * fp32 tokens through GPUAcceleratedLinear
  * (src/gpu_accelerated_functions.py:928-950), e.g. a prompt prefill. */
 int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebook, float *out,
