@@ -67,6 +67,9 @@ SIGNATURES = {
     "cbq_linear_bf16_workspace": (ctypes.c_size_t, [_i, _i, _i]),
     "cbq_linear_bf16_gemm_workspace": (ctypes.c_size_t, [_i, _i, _i, _i]),
     "cbq_linear_f32_workspace": (ctypes.c_size_t, [_i, _i, _i]),
+    "cbq_linear_gemm": (_i, [_vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp,
+                             ctypes.c_size_t, _vp]),
+    "cbq_linear_gemm_workspace": (ctypes.c_size_t, [_i, _i, _i, _i, _i, _i]),
     "cbq_linear_f32_ws": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, ctypes.c_size_t,
                                _vp]),
     "cbq_linear_bf16_ws": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, ctypes.c_size_t,

@@ -3,6 +3,8 @@ dispatcher (libcbq_torch.so, built from csrc/cbq_torch_ops.cpp over the C
 ABI of libcbq_hip.so).
 
     linear(x, packed, codebook, M, bits)              fixed-width GEMV / GEMM
+    linear_kind(x, packed, codebook, M, bits, cb_kind)    linear for a codebook whose
+                                                      codebook_kind is known
     embedding(ids, packed, codebook, vocab, bits, H)  fixed-width row gather
     split_linear(x, cwords, row_off, raw, lut, M)     Huffman (split format): T = 1 the
                                                       GEMV, T >= 2 the fused few-token
@@ -28,7 +30,22 @@ import cbq_native
 HERE = os.path.dirname(os.path.abspath(__file__))
 SO_PATH = os.path.join(HERE, "libcbq_torch.so")
 
+# cbq_linear_gemm's codebook kinds
+CB_UNKNOWN, CB_BF16, CB_FP32, CB_NON_FINITE = range(4)
+
 _loaded = False
+
+
+def codebook_kind(codebook: torch.Tensor) -> int:
+    """What a float32 codebook holds: CB_BF16 (finite bf16 numbers only),
+    CB_FP32 (finite) or CB_NON_FINITE.  Found out once, where a matrix is
+    loaded (one synchronisation); it chooses the kernel and its workspace, and
+    a codebook that is changed in place afterwards still gives its own
+    product."""
+    cb = codebook.detach().reshape(-1)
+    finite, exact = torch.stack([torch.isfinite(cb).all(),
+                                 ((cb.view(torch.int32) & 0xFFFF) == 0).all()]).tolist()
+    return CB_NON_FINITE if not finite else CB_BF16 if exact else CB_FP32
 
 
 def load(path: str = SO_PATH):

@@ -1136,9 +1136,10 @@ const char *cbq_version(void) { return "cbq_hip 0.1 gfx950"; }
 int ck_linear_f32(const float *x, const uint8_t *packed, const float *codebook, float *out,
                   int T, int M, int K, int C, int bits, hipStream_t stream)
 {
-    // T >= 64: the GEMM regime, fp32 MFMA (cbq_prefill_f32.hip)
+    // T >= 64: the GEMM regime, fp32 MFMA (cbq_prefill_f32.hip; 14 bits in
+    // token tiles)
     if (x && packed && codebook && out && T >= 64 && M > 0 && K > 0 && C > 0 && bits >= 1 &&
-        bits <= 16) {
+        bits <= 16 && bits != 14) {
         const int rc = cbq_prefill_f32(x, packed, codebook, out, T, M, K, C, bits, stream, 1,
                                        nullptr);
         if (rc >= 0) return rc;
@@ -1151,6 +1152,27 @@ static size_t prefill_f32_partials(int T, int M, int K)
 {
     const int S = cbq_prefill_f32_splits(T, M, K);
     return S > 1 ? (size_t)S * T * M * sizeof(float) : 0;
+}
+
+// The fp32 kernel with the split K that the workspace holds; -1: not handled.
+static int prefill_f32_ws(const float *x, const uint8_t *packed, const float *codebook, float *out,
+                          int T, int M, int K, int C, int bits, void *ws, size_t ws_bytes,
+                          hipStream_t stream)
+{
+    const size_t need = prefill_f32_partials(T, M, K);
+    const bool split = need && ws && ws_bytes >= need && ((uintptr_t)ws & 15) == 0;
+    return cbq_prefill_f32(x, packed, codebook, out, T, M, K, C, bits, stream,
+                           split ? cbq_prefill_f32_splits(T, M, K) : 1,
+                           split ? (float *)ws : nullptr);
+}
+
+// Calls of a non-finite codebook that run on the fp32 kernel: the GEMM's.  The
+// few-token kernels' parts of x would make a NaN of an infinite weight where a
+// part is zero.
+static bool non_finite_f32(int T, int K, int bits, int cb_kind)
+{
+    return cb_kind == CBQ_CB_NON_FINITE && T >= 33 && K % 32 == 0 &&
+           (bits == 8 || (bits >= 10 && bits <= 14));
 }
 
 size_t cbq_linear_f32_workspace(int T, int M, int K)
@@ -1170,10 +1192,9 @@ int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebo
             rc = cbq_frag_linear(x, true, packed, codebook, out, T, M, K, C, bits, workspace,
                                  ws_bytes, stream);
         // a workspace below the GEMM's: the fp32 kernel with split K
-        const size_t split = rc < 0 ? prefill_f32_partials(T, M, K) : 0;
-        if (split && workspace && ws_bytes >= split && ((uintptr_t)workspace & 15) == 0)
-            rc = cbq_prefill_f32(x, packed, codebook, out, T, M, K, C, bits, stream,
-                                 cbq_prefill_f32_splits(T, M, K), (float *)workspace);
+        if (rc < 0 && T >= 64 && bits != 14)
+            rc = prefill_f32_ws(x, packed, codebook, out, T, M, K, C, bits, workspace, ws_bytes,
+                                stream);
         if (rc >= 0) return rc;
     }
     return ck_linear_f32(x, packed, codebook, out, T, M, K, C, bits, stream);
@@ -1405,6 +1426,33 @@ int cbq_linear_bf16_ws(const void *x_bf16, const uint8_t *packed, const float *c
         if (rc >= 0) return rc;
     }
     return ck_linear_bf16(x_bf16, packed, codebook, out_bf16, T, M, K, C, bits, stream);
+}
+
+size_t cbq_linear_gemm_workspace(int T, int M, int K, int bits, int x_bf16, int cb_kind)
+{
+    if (T <= 0 || M <= 0 || K <= 0) return 0;
+    if (x_bf16) return cbq_linear_bf16_gemm_workspace(T, M, K, bits);
+    if (non_finite_f32(T, K, bits, cb_kind)) return prefill_f32_partials(T, M, K);
+    return cbq_linear_f32_workspace(T, M, K);
+}
+
+int cbq_linear_gemm(const void *x, int x_bf16, const uint8_t *packed, const float *codebook,
+                    void *out, int T, int M, int K, int C, int bits, int cb_kind,
+                    void *workspace, size_t ws_bytes, hipStream_t stream)
+{
+    if (x_bf16)
+        return cbq_linear_bf16_ws(x, packed, codebook, out, T, M, K, C, bits, workspace, ws_bytes,
+                                  stream);
+    if (x && packed && codebook && out && M > 0 && K > 0 && C > 0 &&
+        non_finite_f32(T, K, bits, cb_kind)) {
+        const int rc = prefill_f32_ws((const float *)x, packed, codebook, (float *)out, T, M, K, C,
+                                      bits, workspace, ws_bytes, stream);
+        return rc >= 0 ? rc
+                       : ck_linear_f32((const float *)x, packed, codebook, (float *)out, T, M, K, C,
+                                       bits, stream);
+    }
+    return cbq_linear_f32_ws((const float *)x, packed, codebook, (float *)out, T, M, K, C, bits,
+                             workspace, ws_bytes, stream);
 }
 
 int ck_embedding_f32(const int32_t *token_ids, const uint8_t *packed, const float *codebook,

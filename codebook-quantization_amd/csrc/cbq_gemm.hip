@@ -210,8 +210,9 @@ __device__ __forceinline__ void prep_w(const uint32_t *__restrict__ words,
         __syncthreads();
         if (p == 0) {
             const int f = *s_flag;
-            parts = f ? NW : 1;
-            if (blk == 0 && tid == 0) *flag = (f & 2) ? 0 : parts;
+            parts = (f & 2) ? 0 : f ? NW : 1;
+            if (blk == 0 && tid == 0) *flag = parts;
+            if (parts == 0) return;                        // the GEMM reads the indices
         }
         // this wave's rows 8 wave + 2 i + (lane >> 5), piece lane & 31
         const int c = lane & 31;
@@ -338,10 +339,14 @@ template <class C, int WP> struct GemmStage {
 struct GemmArgs {
     const uint8_t *xf;      // [T / 16][G][NP] fragments
     const uint8_t *wf;      // [M / 16][nw][G] fragments of the slab
-    const int *flag;        // W parts in use; 0: a non-finite codebook value
+    const int *flag;        // W parts in use; 0: the fragments do not hold W
     void *out;              // out + slab offset, row stride ldo
     float *part;            // split-K partials [S][tiles] in fragment order
-    const void *x;          // the caller's x (non-finite codebooks only)
+    // for flag 0: the caller's x, the slab's first index words, the codebook
+    const void *x;
+    const uint32_t *words;
+    const float *cb;
+    int C, bits;
     int T, M, ldo, G, nT, nM, S;
     int nw;                 // W parts the slab has room for
     int fold;               // column groups per chain (even)
@@ -420,26 +425,61 @@ __device__ __forceinline__ void tile_at(int tile, int nT, int nM, int &tt, int &
     tt = band * 8 + in - tm * bt;
 }
 
-// A non-finite codebook value times a zero part of x would be a NaN, so such
-// a matrix takes this loop: one output at a time, plain fp32.
+// One wave's products without the fragments, on the fp32 matrix cores from the
+// index stream: acc as the K loop leaves it.  For codebooks that the bf16
+// parts cannot stand for (flag 0: an infinite value times a zero part of x
+// would be a NaN).  Column group g's step e takes columns 8 q + e of lane
+// quarter q, for x and W alike.  Loads go out as the compiler places them and
+// every wave decodes its own rows: a path for callers that do not say what
+// their codebook holds, not for speed.
 template <class Cfg>
-__device__ float scalar_dot(const GemmArgs &a, int t, int m)
+__device__ __forceinline__ void fp32_fragments(const GemmArgs &a, uint8_t *lds, int t0, int m0,
+                                               int wt, int wm, int g0, int n,
+                                               cbq_f32x4 (&acc)[Cfg::TB][Cfg::MB], int lds_bytes)
 {
-    float s = 0.f;
-    const int mm = m & 31;
-    const uint8_t *w0 = a.wf + (size_t)((m >> 5) * 2 + frag_of(mm)) * a.nw * a.G * kFrag +
-                        frag_row(mm) * 16;
-    for (int k = 0; k < a.G * 32; k++) {
-        float w = 0.f;
-        for (int p = 0; p < Cfg::NW; p++) {
-            const uint16_t b = *(const uint16_t *)(w0 + ((size_t)p * a.G + (k >> 5)) * kFrag +
-                                                   ((k >> 3) & 3) * 256 + (k & 7) * 2);
-            const float v = bf16_to_f32(b);
-            if (p == 0 || (b & 0x7fffu) != 0x0080u) w += v;   // the stand-ins of zero parts
-        }
-        s = fmaf(((const float *)a.x)[(size_t)t * (a.G * 32) + k], w, s);
+    const int lane = threadIdx.x & (CBQ_WAVE - 1), q = lane >> 4, fr = lane & 15;
+    const int bits = a.bits, C = min(a.C, 1 << bits);
+    const uint32_t mask = (1u << bits) - 1u;
+    const float *tab = a.cb;
+    if (C * 4 <= lds_bytes) {
+        float *const s = (float *)lds;
+        for (int i = threadIdx.x; i < C; i += kGBlock) s[i] = a.cb[i];
+        lds_barrier();
+        tab = s;
     }
-    return s;
+    const uint32_t *row[Cfg::MB];
+#pragma unroll
+    for (int j = 0; j < Cfg::MB; j++) {
+        const int f = (m0 >> 4) + wm * Cfg::MB + j;            // fragment -> feature
+        const int m = (f >> 1) * 32 + (fr >> 2) * 8 + (f & 1) * 4 + (fr & 3);
+        row[j] = a.words + (int64_t)min(m, a.M - 1) * a.G * bits;
+    }
+#pragma unroll 1
+    for (int g = g0; g < g0 + n; g++) {
+#pragma unroll 4                                       // no more: the K loop sets the registers
+        for (int e = 0; e < 8; e++) {
+            float xv[Cfg::TB], w[Cfg::MB];
+            const int o = (q * 8 + e) * bits, k = o >> 5, k1 = min(k + 1, bits - 1);
+#pragma unroll
+            for (int j = 0; j < Cfg::MB; j++) {
+                const uint32_t *const p = row[j] + (int64_t)g * bits;
+                const uint32_t ix = __builtin_amdgcn_alignbit(p[k1], p[k], o & 31) & mask;
+                w[j] = tab[min((int)ix, C - 1)];
+            }
+#pragma unroll
+            for (int i = 0; i < Cfg::TB; i++) {
+                const int t = min(t0 + (wt * Cfg::TB + i) * 16 + fr, a.T - 1);
+                const size_t at = ((size_t)t * a.G + g) * 32 + q * 8 + e;
+                xv[i] = Cfg::NP == 3 ? ((const float *)a.x)[at]
+                                     : bf16_to_f32(((const uint16_t *)a.x)[at]);
+            }
+#pragma unroll
+            for (int i = 0; i < Cfg::TB; i++)
+#pragma unroll
+                for (int j = 0; j < Cfg::MB; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], xv[i], acc[i][j], 0, 0, 0);
+        }
+    }
 }
 
 template <class Cfg, bool SPLIT>
@@ -464,24 +504,6 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
     float *const part = SPLIT ? a.part + ((size_t)z * tiles + tile) * (Cfg::TT * Cfg::TM) : nullptr;
 
     const int nW = __builtin_amdgcn_readfirstlane(*a.flag);
-    if (NP == 3 && nW == 0) {
-        for (int e = threadIdx.x; e < Cfg::TT * Cfg::TM; e += kGBlock) {
-            const int tl = e / Cfg::TM, ml = e - tl * Cfg::TM;
-            const int t = t0 + tl, m = m0 + ml;
-            if (t >= a.T || m >= a.M) continue;
-            const float v = z == 0 ? scalar_dot<Cfg>(a, t, m) : 0.f;
-            if constexpr (SPLIT) {
-                const int tb = tl >> 4, mb = ml >> 5, mm = ml & 31;
-                const int w = (tb / TB) * Cfg::WM + mb / (MB / 2);
-                part[((((w * TB + tb % TB) * (MB / 2) + mb % (MB / 2)) * 2 + frag_of(mm)) * 64 +
-                      (mm >> 3) * 16 + (tl & 15)) * 4 + (mm & 3)] = v;
-            } else {
-                ((float *)a.out)[(int64_t)t * a.ldo + m] = v;
-            }
-        }
-        return;
-    }
-
     // this block's column groups [g0, g1)
     const int per = SPLIT ? (a.G + a.S - 1) / a.S : a.G;
     const int g0 = min(z * per, a.G), n = min(g0 + per, a.G) - g0;
@@ -644,12 +666,11 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
         // no copy into LDS may outlive the block
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     };
-    if (n > 0) {
-        if (nW == 1) all(std::integral_constant<int, 1>{});
-        else all(std::integral_constant<int, Cfg::NW>{});
-    }
-
-    if constexpr (FOLD)
+    if (n > 0 && nW == 1) all(std::integral_constant<int, 1>{});
+    else if (n > 0 && nW > 1) all(std::integral_constant<int, Cfg::NW>{});
+    if (NP == 3 && nW == 0)
+        fp32_fragments<Cfg>(a, lds, t0, m0, wt, wm, g0, n, acc, (int)sizeof(lds));
+    else if constexpr (FOLD)
 #pragma unroll
         for (int i = 0; i < TB; i++)
 #pragma unroll
@@ -871,6 +892,9 @@ GemmArgs gemm_args(const GemmPlan &p, int NP, int nw, const void *x, int T, int 
     a.out = nullptr;
     a.part = (float *)(wf + round256(w_bytes(p.rows, K, nw)));
     a.x = x;
+    a.words = nullptr;
+    a.cb = nullptr;
+    a.C = a.bits = 0;
     a.T = T;
     a.M = 0;
     a.ldo = M;
@@ -895,8 +919,12 @@ int frag_linear(int NP, const void *x, const uint32_t *words, const float *cb, v
 {
     const GemmPlan p = gemm_plan(T, M, K, NP, w_parts(NP));
     GemmArgs a = gemm_args(p, NP, w_parts(NP), x, T, M, K, ws);
+    a.cb = cb;
+    a.C = C;
+    a.bits = BITS;
     for (int r0 = 0; r0 < M; r0 += p.rows) {
         a.M = std::min(p.rows, M - r0);
+        a.words = words + (int64_t)r0 * (K >> 5) * BITS;
         a.out = (uint8_t *)out + (size_t)r0 * (NP == 3 ? 4 : 2);
         int rc = launch_prep<BITS>(NP, x, (uint8_t *)a.xf, T, K, r0 == 0, words, cb, C,
                                    (uint8_t *)a.wf, (int *)ws, r0, a.M, st);

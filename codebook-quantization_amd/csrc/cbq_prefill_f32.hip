@@ -2,7 +2,7 @@
 // matrix cores of gfx950 (v_mfma_f32_32x32x2_f32).
 //
 // out[t, m] = sum_k x[t, k] * codebook[min(idx[m*K + k], C-1)] with fp32 x,
-// the fp32 codebook and fp32 accumulation, for T >= 64 tokens: the batched
+// the fp32 codebook and fp32 accumulation, for T >= 64 tokens (33, non-finite codebooks): the batched
 // case of ck_linear_f32 (rocm/compressed_kernel.h:52-64), where one K-tile of
 // weights serves 256 tokens instead of being re-read per token tile.  Every
 // product is exact in fp32; only the summation order differs from a GEMV.
@@ -272,7 +272,7 @@ int launch_prefill_f32(const float *x, const uint8_t *packed, const float *cb, f
 // the CUs twice, with at least 8 K groups per split and at most 16 splits.
 int cbq_prefill_f32_splits(int T, int M, int K)
 {
-    if (T < 64 || K % kFK != 0) return 1;
+    if (K % kFK != 0) return 1;
     const int64_t tiles = (int64_t)((T + kFT - 1) / kFT) * ((M + kFM - 1) / kFM);
     const int64_t want = 2 * (int64_t)cbq_num_cus();
     if (tiles >= want) return 1;
@@ -286,7 +286,7 @@ int cbq_prefill_f32_splits(int T, int M, int K)
 int cbq_prefill_f32(const float *x, const uint8_t *packed, const float *cb, float *out, int T,
                     int M, int K, int C, int bits, hipStream_t st, int S, float *ws)
 {
-    if (T < 64 || K % kFK != 0 || (((uintptr_t)packed | (uintptr_t)x) & 15) != 0 ||
+    if (K % kFK != 0 || (((uintptr_t)packed | (uintptr_t)x) & 15) != 0 ||
         (size_t)T > 65535ull * kFT || M > 65535 * kFM)
         return -1;
     if (S > 1 && !ws) return -1;
@@ -296,6 +296,7 @@ int cbq_prefill_f32(const float *x, const uint8_t *packed, const float *cb, floa
     case 11: return launch_prefill_f32<11>(x, packed, cb, out, T, M, K, C, S, ws, st);
     case 12: return launch_prefill_f32<12>(x, packed, cb, out, T, M, K, C, S, ws, st);
     case 13: return launch_prefill_f32<13>(x, packed, cb, out, T, M, K, C, S, ws, st);
+    case 14: return launch_prefill_f32<14>(x, packed, cb, out, T, M, K, C, S, ws, st);
     default: return -1;
     }
 }

@@ -9,6 +9,7 @@
 // (src/gpu_accelerated_functions.py:415-543).
 //
 //   linear(x, packed, codebook, M, bits) -> out          ck_linear_f32 / ck_linear_bf16
+//   linear_kind(x, packed, codebook, M, bits, cb_kind) -> out     cbq_linear_gemm
 //   embedding(ids, packed, codebook, vocab, bits, H) -> out     cbq_embedding_f32
 //   split_linear(x, cwords, row_off, raw, lut, M) -> out         cbq_split_linear_f32
 //   split_gemm(x, cwords, row_off, raw, lut, M) -> out       cbq_split_linear_gemm
@@ -47,8 +48,8 @@ void check_dev(const at::Tensor &t, const at::Tensor &ref, const char *name)
 
 template <typename P> const P *cptr(const at::Tensor &t) { return (const P *)t.data_ptr(); }
 
-at::Tensor linear(const at::Tensor &x, const at::Tensor &packed, const at::Tensor &codebook,
-                  int64_t M, int64_t bits)
+at::Tensor linear_kind(const at::Tensor &x, const at::Tensor &packed, const at::Tensor &codebook,
+                       int64_t M, int64_t bits, int64_t cb_kind)
 {
     TORCH_CHECK(x.is_cuda(), "cbq::linear: x must be a device tensor");
     TORCH_CHECK(x.dim() == 2, "cbq::linear: x must be [T, K]");
@@ -72,21 +73,21 @@ at::Tensor linear(const at::Tensor &x, const at::Tensor &packed, const at::Tenso
     const hipStream_t st = current_stream(x);
     const bool bf16 = x.scalar_type() == at::kBFloat16;
     // batched tokens: MFMA path with its workspace from torch's allocator
-    const size_t nws = bf16 ? cbq_linear_bf16_gemm_workspace((int)T, (int)M, (int)K, (int)bits)
-                            : cbq_linear_f32_workspace((int)T, (int)M, (int)K);
+    const size_t nws = cbq_linear_gemm_workspace((int)T, (int)M, (int)K, (int)bits, bf16,
+                                                 (int)cb_kind);
     at::Tensor ws;
     if (nws) ws = at::empty({(int64_t)((nws + 255) / 256 * 256)}, x.options().dtype(at::kByte));
-    int rc;
-    if (bf16)
-        rc = cbq_linear_bf16_ws(x.data_ptr(), cptr<uint8_t>(packed), cptr<float>(codebook),
-                                out.data_ptr(), (int)T, (int)M, (int)K, (int)C, (int)bits,
-                                nws ? ws.data_ptr() : nullptr, nws, st);
-    else
-        rc = cbq_linear_f32_ws(cptr<float>(x), cptr<uint8_t>(packed), cptr<float>(codebook),
-                               (float *)out.data_ptr(), (int)T, (int)M, (int)K, (int)C, (int)bits,
-                               nws ? ws.data_ptr() : nullptr, nws, st);
-    check_rc(rc, bf16 ? "cbq_linear_bf16_ws" : "cbq_linear_f32_ws");
+    check_rc(cbq_linear_gemm(x.data_ptr(), bf16, cptr<uint8_t>(packed), cptr<float>(codebook),
+                             out.data_ptr(), (int)T, (int)M, (int)K, (int)C, (int)bits,
+                             (int)cb_kind, nws ? ws.data_ptr() : nullptr, nws, st),
+             "cbq_linear_gemm");
     return out;
+}
+
+at::Tensor linear(const at::Tensor &x, const at::Tensor &packed, const at::Tensor &codebook,
+                  int64_t M, int64_t bits)
+{
+    return linear_kind(x, packed, codebook, M, bits, CBQ_CB_UNKNOWN);
 }
 
 at::Tensor embedding(const at::Tensor &ids, const at::Tensor &packed, const at::Tensor &codebook,
@@ -295,6 +296,12 @@ at::Tensor linear_meta(const at::Tensor &x, const at::Tensor &, const at::Tensor
     return at::empty({x.size(0), M}, x.options());
 }
 
+at::Tensor linear_kind_meta(const at::Tensor &x, const at::Tensor &, const at::Tensor &, int64_t M,
+                            int64_t, int64_t)
+{
+    return at::empty({x.size(0), M}, x.options());
+}
+
 at::Tensor embedding_meta(const at::Tensor &ids, const at::Tensor &, const at::Tensor &codebook,
                           int64_t, int64_t, int64_t H)
 {
@@ -306,6 +313,8 @@ at::Tensor embedding_meta(const at::Tensor &ids, const at::Tensor &, const at::T
 TORCH_LIBRARY(cbq, m)
 {
     m.def("linear(Tensor x, Tensor packed, Tensor codebook, int M, int bits) -> Tensor");
+    m.def("linear_kind(Tensor x, Tensor packed, Tensor codebook, int M, int bits, int cb_kind) "
+          "-> Tensor");
     m.def("embedding(Tensor ids, Tensor packed, Tensor codebook, int vocab, int bits, int H) "
           "-> Tensor");
     m.def("split_linear(Tensor x, Tensor cwords, Tensor row_off, Tensor raw, Tensor lut, "
@@ -324,6 +333,7 @@ TORCH_LIBRARY(cbq, m)
 TORCH_LIBRARY_IMPL(cbq, CUDA, m)
 {
     m.impl("linear", &linear);
+    m.impl("linear_kind", &linear_kind);
     m.impl("embedding", &embedding);
     m.impl("split_linear", &split_linear);
     m.impl("split_gemm", &split_gemm);
@@ -334,5 +344,6 @@ TORCH_LIBRARY_IMPL(cbq, CUDA, m)
 TORCH_LIBRARY_IMPL(cbq, Meta, m)
 {
     m.impl("linear", &linear_meta);
+    m.impl("linear_kind", &linear_kind_meta);
     m.impl("embedding", &embedding_meta);
 }

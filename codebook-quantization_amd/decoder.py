@@ -434,6 +434,7 @@ def from_synthetic(cfg: DecoderConfig, tensors: Dict[str, object], device="cuda"
     device bytes."""
     import ctypes
     import cbq_native as nat
+    import cbq_ops
     import synthetic
     from gpu_huffman_functions import (SymbolDecoder, build_split, huffman_prefill,
                                        split_bytes, split_eligible, split_inverse,
@@ -498,19 +499,20 @@ def from_synthetic(cfg: DecoderConfig, tensors: Dict[str, object], device="cuda"
 
     def fixed_linear(t):
         M, K = t.shape
+        kind = cbq_ops.codebook_kind(t.codebook)
 
         def f(x):
             x = x.reshape(-1, K).contiguous()
             T = x.shape[0]
             out = torch.empty(T, M, device=dev)
             # a prompt's decoded fragments and partials: a torch workspace
-            nws = int(lib.cbq_linear_f32_workspace(T, M, K))
-            ws = torch.empty(max(1, nws // 4), device=dev) if nws else None
-            nat.check(lib.cbq_linear_f32_ws(x.data_ptr(), t.packed.data_ptr(),
-                                            t.codebook.data_ptr(), out.data_ptr(), T, M, K,
-                                            t.codebook.numel(), t.bits,
-                                            None if ws is None else ws.data_ptr(), nws,
-                                            nat.stream_ptr(dev)), "cbq_linear_f32_ws")
+            nws = int(lib.cbq_linear_gemm_workspace(T, M, K, t.bits, 0, kind))
+            ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws else None
+            nat.check(lib.cbq_linear_gemm(x.data_ptr(), 0, t.packed.data_ptr(),
+                                          t.codebook.data_ptr(), out.data_ptr(), T, M, K,
+                                          t.codebook.numel(), t.bits, kind,
+                                          None if ws is None else ws.data_ptr(), nws,
+                                          nat.stream_ptr(dev)), "cbq_linear_gemm")
             return out
 
         def xform(x0, x1, h_out, mode):
@@ -572,14 +574,14 @@ def from_synthetic(cfg: DecoderConfig, tensors: Dict[str, object], device="cuda"
         through its transient fragments.  Captures only the split format, so
         the tensor's stream can be freed."""
         inv = inv_of(cbt)
-        finite = bool(torch.isfinite(cbt).all())
+        kind = cbq_ops.codebook_kind(cbt)
         one, sxform = split_fns([sp], [M], K)
 
         def f(x):
             x = x.reshape(-1, K).contiguous()
             if x.shape[0] == 1:
                 return one(x)
-            return split_prefill(sp, inv, x, M, K, cbt, finite)
+            return split_prefill(sp, inv, x, M, K, cbt, kind != cbq_ops.CB_NON_FINITE, kind)
 
         def xform_argmax(x0, x1, mode, ids32, toks, pos, first, out=None, keep=sp):
             """One token, then the greedy pick in the GEMV's epilogue."""
@@ -602,6 +604,7 @@ def from_synthetic(cfg: DecoderConfig, tensors: Dict[str, object], device="cuda"
         sp = huff_split(t)
         if sp is not None:
             return split_linear(sp, M, K, cbt)
+        kind = cbq_ops.codebook_kind(cbt)
         resident[t.name] = t.nbytes
         desc = huff_desc(t)
 
@@ -610,7 +613,7 @@ def from_synthetic(cfg: DecoderConfig, tensors: Dict[str, object], device="cuda"
             T = x.shape[0]
             if T >= 64:
                 return huffman_prefill(SymbolDecoder(keep[0], keep[1], keep[2], keep[4], dev),
-                                       x, M, K, cbt)
+                                       x, M, K, cbt, kind)
             out = torch.empty(T, M, device=dev)
             for t0 in range(0, T, 16):
                 tt = min(16, T - t0)

@@ -65,6 +65,7 @@ class GPUAcceleratedLinear:
         device = _device_for(codebook)
         self.codebook = codebook.detach().to(device=device, dtype=torch.float32).contiguous()
         self.C = int(self.codebook.numel())
+        self.cb_kind = cbq_ops.codebook_kind(self.codebook)
         need = bitpack.calculate_packed_size(self.M * self.K, self.bits)
         raw = index_bytes(indices_np, self.bits)
         if raw.size < need:
@@ -84,6 +85,7 @@ class GPUAcceleratedLinear:
         self._lib = nat.load()
         self.codebook = t.codebook
         self.C = int(t.codebook.numel())
+        self.cb_kind = cbq_ops.codebook_kind(self.codebook)
         self.packed = t.packed
         return self
 
@@ -104,11 +106,12 @@ class GPUAcceleratedLinear:
         ops = cbq_ops.load()
         if in_dtype == torch.bfloat16:
             # bf16 I/O kernel (batched tokens: bf16 MFMA with fp32 accumulation)
-            out = ops.linear(x.reshape(T, self.K).contiguous(), self.packed, self.codebook,
-                             self.M, self.bits)
+            out = ops.linear_kind(x.reshape(T, self.K).contiguous(), self.packed, self.codebook,
+                                  self.M, self.bits, self.cb_kind)
             return out.reshape(*lead, self.M)
         xc = x.reshape(T, self.K).to(torch.float32).contiguous()
-        out = ops.linear(xc, self.packed, self.codebook, self.M, self.bits).reshape(*lead, self.M)
+        out = ops.linear_kind(xc, self.packed, self.codebook, self.M, self.bits,
+                              self.cb_kind).reshape(*lead, self.M)
         return out if in_dtype == torch.float32 else out.to(in_dtype)
 
 

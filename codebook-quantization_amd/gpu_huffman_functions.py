@@ -320,33 +320,33 @@ def _packed_for_gemm(idx_or_split, n: int, C: int, dev, inv: Optional[torch.Tens
 
 
 def linear_from_packed(x: torch.Tensor, packed: torch.Tensor, bits: int, M: int, K: int,
-                       codebook: torch.Tensor) -> torch.Tensor:
-    """y [T, M] = x [T, K] (fp32) @ W^T over a transient packed index stream:
-    ck_linear_f32's kernels for every T (the fp32 matrix cores for T >= 64,
-    with split K in a torch workspace)."""
+                       codebook: torch.Tensor,
+                       cb_kind: int = cbq_ops.CB_UNKNOWN) -> torch.Tensor:
+    """y [T, M] = x [T, K] (fp32) @ W^T over a transient packed index stream
+    (cbq_linear_gemm for every T, its workspace from torch's allocator)."""
     lib = nat.load()
     dev = x.device
     T = x.shape[0]
     C = int(codebook.numel())
     out = torch.empty(T, M, dtype=torch.float32, device=dev)
-    nws = int(lib.cbq_linear_f32_workspace(T, M, K))
-    ws = torch.empty(max(1, nws // 4), dtype=torch.float32, device=dev) if nws else None
-    nat.check(lib.cbq_linear_f32_ws(x.data_ptr(), packed.data_ptr(), codebook.data_ptr(),
-                                    out.data_ptr(), T, M, K, C, bits,
-                                    None if ws is None else ws.data_ptr(), nws,
-                                    nat.stream_ptr(dev)), "cbq_linear_f32_ws")
+    nws = int(lib.cbq_linear_gemm_workspace(T, M, K, bits, 0, cb_kind))
+    ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws else None
+    nat.check(lib.cbq_linear_gemm(x.data_ptr(), 0, packed.data_ptr(), codebook.data_ptr(),
+                                  out.data_ptr(), T, M, K, C, bits, cb_kind,
+                                  None if ws is None else ws.data_ptr(), nws,
+                                  nat.stream_ptr(dev)), "cbq_linear_gemm")
     return out
 
 
 def huffman_prefill(sym: "SymbolDecoder", x: torch.Tensor, M: int, K: int,
-                    codebook: torch.Tensor) -> torch.Tensor:
+                    codebook: torch.Tensor, cb_kind: int = cbq_ops.CB_UNKNOWN) -> torch.Tensor:
     """y [T, M] for batched fp32 tokens from the stream: decoded to transient
     fixed-width indices (cbq_huff_decode_indices, cbq_pack_indices) and
     multiplied by ck_linear_f32's kernels."""
     idx = sym.indices(M * K)
     packed, bits = _packed_for_gemm(idx, M * K, int(codebook.numel()), x.device)
     del idx
-    return linear_from_packed(x, packed, bits, M, K, codebook)
+    return linear_from_packed(x, packed, bits, M, K, codebook, cb_kind)
 
 
 FEWTOK_MAX_T = 32       # up to two 16-token launches of the fused kernel
@@ -386,7 +386,8 @@ def split_fewtok_eligible(K: int) -> bool:
 
 
 def split_prefill(split, inv: torch.Tensor, x: torch.Tensor, M: int, K: int,
-                  codebook: torch.Tensor, finite: bool = False) -> torch.Tensor:
+                  codebook: torch.Tensor, finite: bool = False,
+                  cb_kind: int = cbq_ops.CB_UNKNOWN) -> torch.Tensor:
     """y [T, M] for batched fp32 tokens from the split format.  From 33 tokens
     on and finite codebook values (finite=True): decoded to MFMA fragments
     and multiplied in one GEMM (split_gemm).  Else up to 32
@@ -402,7 +403,7 @@ def split_prefill(split, inv: torch.Tensor, x: torch.Tensor, M: int, K: int,
     if 1 <= T <= FEWTOK_MAX_T and split_fewtok_eligible(K) and x.data_ptr() % 16 == 0:
         return split_fewtok([split], x, [M], K)[0]
     packed, bits = _packed_for_gemm(split, M * K, int(codebook.numel()), x.device, inv)
-    return linear_from_packed(x, packed, bits, M, K, codebook)
+    return linear_from_packed(x, packed, bits, M, K, codebook, cb_kind)
 
 
 def split_fewtok(splits, x: torch.Tensor, Ms, K: int):
@@ -547,7 +548,7 @@ class HuffmanCodebookLinear:
         self.split = None
         self.cols = None
         self._inv = None
-        self._finite = bool(np.isfinite(self._cb_np).all())
+        self._cb_kind = cbq_ops.codebook_kind(torch.from_numpy(self._cb_np))
         if layout in ("auto", "split") and split_eligible(self.M, self.K):
             idx = SymbolDecoder(dev.words, dev.chunk_off, dev.sub_len, self._lengths,
                                 device).indices(self.M * self.K)
@@ -585,7 +586,7 @@ class HuffmanCodebookLinear:
         self.device = cb.device
         self._cb_dev = cb
         self._cb_np = cb.cpu().numpy()
-        self._finite = bool(np.isfinite(self._cb_np).all())
+        self._cb_kind = cbq_ops.codebook_kind(torch.from_numpy(self._cb_np))
         self._lengths = np.ascontiguousarray(t.lengths, np.uint8)
         self.cols = None
         if isinstance(t, dfm.SplitTensor):
@@ -599,6 +600,10 @@ class HuffmanCodebookLinear:
         else:
             raise TypeError(f"{name}: not a Huffman device tensor ({type(t).__name__})")
         return self
+
+    @property
+    def _finite(self) -> bool:
+        return self._cb_kind != cbq_ops.CB_NON_FINITE
 
     @property
     def resident_bytes(self) -> int:
@@ -640,9 +645,10 @@ class HuffmanCodebookLinear:
             cw, ro, raw, lut = self.split[0]
             out = cbq_ops.load().split_linear(xc, cw, ro, raw, lut, self.M)
         elif self.split is not None:
-            out = split_prefill(self.split, self._inv, xc, self.M, self.K, self._cb_dev)
+            out = split_prefill(self.split, self._inv, xc, self.M, self.K, self._cb_dev,
+                                cb_kind=self._cb_kind)
         elif T >= 64 or self.K % hc.SUB_SYMBOLS:
-            out = huffman_prefill(self._symbols(), xc, self.M, self.K, self._cb_dev)
+            out = huffman_prefill(self._symbols(), xc, self.M, self.K, self._cb_dev, self._cb_kind)
         elif T == 1 and self.cols is not None:
             out = torch.empty(1, self.M, dtype=torch.float32, device=self.device)
             nat.check(self._lib.cbq_huff_linear_col_f32(

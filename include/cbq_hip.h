@@ -68,6 +68,27 @@ int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebo
                       int T, int M, int K, int C, int bits, void *workspace, size_t ws_bytes,
                       hipStream_t stream);
 
+/* What a codebook holds, for cbq_linear_gemm: a hint that chooses the kernel
+ * and its workspace.  A hint that does not fit costs time, never the result. */
+#define CBQ_CB_UNKNOWN    0
+#define CBQ_CB_BF16       1     /* every value a finite bf16 number */
+#define CBQ_CB_FP32       2     /* every value finite */
+#define CBQ_CB_NON_FINITE 3     /* an infinity or NaN among them */
+
+/* The batched linear for fp32 or bf16 x (x_bf16 != 0; out likewise) with a
+ * workspace of cbq_linear_gemm_workspace bytes (256-byte aligned):
+ * cbq_linear_f32_ws / cbq_linear_bf16_ws for a codebook of cb_kind.  fp32 x
+ * and a non-finite codebook: ck_linear_f32's fp32 kernel with split K from 33
+ * tokens on (the bf16 parts of x cannot multiply an infinity).  No
+ * counterpart in the reference: GPUAcceleratedLinear
+ * (src/gpu_accelerated_functions.py:928-950) over batched tokens. */
+int cbq_linear_gemm(const void *x, int x_bf16, const uint8_t *packed, const float *codebook,
+                    void *out, int T, int M, int K, int C, int bits, int cb_kind,
+                    void *workspace, size_t ws_bytes, hipStream_t stream);
+
+/* Workspace bytes of cbq_linear_gemm (0: it needs none). */
+size_t cbq_linear_gemm_workspace(int T, int M, int K, int bits, int x_bf16, int cb_kind);
+
 /* Fixed-width GEMV with an implicit (affine) codebook: index i stands for
  * the bf16 value with bit pattern lo + i (i < w), 0x8000 + lo + i - w
  * (w <= i < 2w), and 0.0 for i >= 2w.  This is the load-time re-indexed

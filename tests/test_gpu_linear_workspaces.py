@@ -44,3 +44,85 @@ def test_f32_split_k_below_the_gemm_workspace(cuda, T, M, K, bits):
     assert _rel(y, ref) <= TOL_CHAIN and not torch.equal(y, one)
     assert torch.equal(_f32_ws(cuda, x, packed, cb, M, K, bits, 16), one)   # no room: one chain
     assert _rel(_f32_ws(cuda, x, packed, cb, M, K, bits, n), ref) <= TOL_F32
+
+
+def _indices(packed, M, K, bits):
+    """The stream's indices, unpacked bit by bit."""
+    b = packed[:M * K * bits // 8, None].to(torch.int64) >> torch.arange(8, device=packed.device)
+    b = (b & 1).reshape(M * K, bits)
+    return (b << torch.arange(bits, device=packed.device)).sum(1).reshape(M, K)
+
+
+def _layer(packed, cb, M, K, bits):
+    from device_formats import FixedTensor
+    from gpu_accelerated_functions import GPUAcceleratedLinear
+    return GPUAcceleratedLinear.from_device("w", FixedTensor("w", (M, K), bits, "x", packed, cb))
+
+
+def _us(fn):
+    fn()
+    e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    e[0].record()
+    for _ in range(3):
+        fn()
+    e[1].record()
+    torch.cuda.synchronize()
+    return e[0].elapsed_time(e[1]) / 3e-3
+
+
+@pytest.mark.parametrize("T,M,K,bits", [(33, 130, 96, 13), (40, 1024, 2048, 14), (64, 4096, 512, 13),
+                                        (70, 200, 4096, 8), (300, 1030, 2048, 12)])
+@pytest.mark.parametrize("declared", [True, False])
+def test_non_finite_codebook_keeps_its_rate(cuda, T, M, K, bits, declared):
+    """One infinity in the codebook: infinities and NaNs where the products
+    have them, with the kind the module found at load (the fp32 kernel) and
+    with none (the GEMM's own fp32 products); no more than ten times the time
+    of a finite codebook (one output at a time took 300 times)."""
+    from gpu_accelerated_functions import cbq_ops
+    print(f"non-finite T{T} M{M} K{K} bits{bits} declared {declared}", flush=True)
+    packed, cb, w = _matrix(cuda, M, K, bits, "inf", T + M)
+    x = torch.randn(T, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(K))
+    x[5] = x[5].bfloat16().float()                       # zero lower parts
+    x[7, ::3] = 0.0
+    x[9, 1] = float("-inf")
+    layer = _layer(packed, cb, M, K, bits)
+    assert layer.cb_kind == cbq_ops.CB_NON_FINITE
+    if not declared:
+        layer.cb_kind = cbq_ops.CB_UNKNOWN
+    y, ref = layer(x), x.double() @ w.T
+    assert torch.equal(y.isnan(), ref.isnan())
+    assert torch.equal(y.isposinf(), ref.isposinf()) and torch.equal(y.isneginf(), ref.isneginf())
+    ok = ref.isfinite()
+    if bool(ok.any()):
+        assert _rel(y[ok], ref[ok]) <= TOL_CHAIN
+    plain = _layer(packed, torch.where(cb.isfinite(), cb, 0.01), M, K, bits)
+    assert _us(lambda: layer(x)) <= 10 * _us(lambda: plain(x)) + 50
+
+
+def test_codebook_changed_in_place(cuda):
+    """The kind is a hint: a codebook written after the module was made gives
+    its own product, whatever it then holds."""
+    T, M, K, bits = 80, 320, 1024, 10
+    packed, cb, w = _matrix(cuda, M, K, bits, "bf16", 11)
+    x = torch.randn(T, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(2))
+    layer = _layer(packed, cb, M, K, bits)
+    assert _rel(layer(x), x.double() @ w.T) <= TOL_F32
+    g = torch.Generator(device="cuda").manual_seed(3)
+    for fill in ("fp32", "inf", "bf16"):
+        new = torch.randn(cb.numel(), device=cuda, generator=g) * 0.05
+        if fill != "fp32":
+            new = new.bfloat16().float()
+        if fill == "inf":
+            new[3] = float("inf")
+        idx = _indices(packed, M, K, bits).clamp_max(cb.numel() - 1)
+        cb.copy_(new)
+        ref = x.double() @ cb[idx].double().T
+        for xx in (x, x.bfloat16()):
+            r = ref if xx is x else xx.double() @ cb[idx].double().T
+            y = layer(xx)
+            if xx is not x and fill == "inf":
+                continue                                # (bf16 x: hi + lo parts, as ever)
+            assert torch.equal(y.isnan(), r.isnan())
+            ok = r.isfinite()
+            if bool(ok.any()):
+                assert _rel(y[ok], r[ok]) <= (TOL_CHAIN if xx is x else 2.0 ** -9)
