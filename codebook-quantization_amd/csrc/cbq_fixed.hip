@@ -1396,9 +1396,10 @@ size_t cbq_linear_bf16_workspace(int T, int M, int K)
 size_t cbq_linear_bf16_gemm_workspace(int T, int M, int K, int bits)
 {
     if (T <= 0 || M <= 0 || K <= 0) return 0;
-    return std::max(cbq_fewtok_ws_bytes(T, M, K, bits, false),
-                    std::max(cbq_prefill_ws_bytes(T, M, K),
-                             cbq_frag_ws_bytes(T, M, K, bits, false)));
+    const size_t few = cbq_fewtok_ws_bytes(T, M, K, bits, false);
+    if (bits != 8 && (bits < 10 || bits > 14)) return few;   // widths without a prompt kernel
+    return std::max(few, std::max(cbq_prefill_ws_bytes(T, M, K),
+                                  cbq_frag_ws_bytes(T, M, K, bits, false)));
 }
 
 int cbq_linear_bf16_ws(const void *x_bf16, const uint8_t *packed, const float *codebook,
@@ -1433,7 +1434,9 @@ size_t cbq_linear_gemm_workspace(int T, int M, int K, int bits, int x_bf16, int 
     if (T <= 0 || M <= 0 || K <= 0) return 0;
     if (x_bf16) return cbq_linear_bf16_gemm_workspace(T, M, K, bits);
     if (non_finite_f32(T, K, bits, cb_kind)) return prefill_f32_partials(T, M, K);
-    return cbq_linear_f32_workspace(T, M, K);
+    if (bits < 1) return 0;
+    return std::max(cbq_fewtok_ws_bytes(T, M, K, bits, true),
+                    cbq_frag_ws_bytes(T, M, K, bits, true));
 }
 
 int cbq_linear_gemm(const void *x, int x_bf16, const uint8_t *packed, const float *codebook,

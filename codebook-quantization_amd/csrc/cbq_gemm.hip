@@ -962,9 +962,11 @@ bool frag_shape(int T, int M, int K, bool f32)
 // read and fragments written at 4.8 TB/s, two launches, the GEMM's plan.
 // 8-bit codebooks are taken to be fp32 values (two parts of W: T = 512,
 // 4096 x 4096: 82 against 62 us fused).
+// bits 0: any width the GEMM takes.
 size_t cbq_frag_ws_bytes(int T, int M, int K, int bits, bool f32)
 {
-    if (!frag_shape(T, M, K, f32)) return 0;
+    if (!frag_shape(T, M, K, f32) || !(bits == 0 || bits == 8 || (bits >= 10 && bits <= 14)))
+        return 0;
     const int NP = f32 ? 3 : 1;
     const GemmPlan p = gemm_plan(T, M, K, NP, w_parts(NP));
     if (!f32) {

@@ -2,9 +2,10 @@
 // matrix cores of gfx950 (v_mfma_f32_32x32x2_f32).
 //
 // out[t, m] = sum_k x[t, k] * codebook[min(idx[m*K + k], C-1)] with fp32 x,
-// the fp32 codebook and fp32 accumulation, for T >= 64 tokens (33, non-finite codebooks): the batched
-// case of ck_linear_f32 (rocm/compressed_kernel.h:52-64), where one K-tile of
-// weights serves 256 tokens instead of being re-read per token tile.  Every
+// the fp32 codebook and fp32 accumulation, for T >= 64 tokens (33 for
+// non-finite codebooks): the batched case of ck_linear_f32
+// (rocm/compressed_kernel.h:52-64), where one K-tile of weights serves 256
+// tokens instead of being re-read per token tile.  Every
 // product is exact in fp32; only the summation order differs from a GEMV.
 // Index layout is the reference's LSB-first stream (src/bitpack.py:32-95);
 // K % 32 == 0, so each row's 32-index groups are BITS whole 32-bit words.

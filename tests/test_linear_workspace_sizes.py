@@ -1,0 +1,32 @@
+"""cbq_linear_gemm_workspace: what a batched call reserves (host arithmetic, no
+GPU needed)."""
+import pytest
+
+import cbq_native as nat
+
+
+@pytest.fixture(scope="module")
+def ws():
+    lib = nat.load()
+
+    def size(T, M, K, bits, x_bf16=0, kind=0):
+        return int(lib.cbq_linear_gemm_workspace(T, M, K, bits, x_bf16, kind))
+    return size
+
+
+@pytest.mark.parametrize("bits", [1, 4, 9, 15, 16])
+@pytest.mark.parametrize("x_bf16", [0, 1])
+@pytest.mark.parametrize("kind", [0, 1, 2, 3])
+def test_refused_widths_reserve_nothing(ws, bits, x_bf16, kind):
+    """No prompt kernel takes these widths, so no call may allocate for one
+    (16 bits: up to 64 tokens have the few-token kernel's copy of x)."""
+    for T in (70, 128, 512, 2048):
+        for M, K in ((1024, 2048), (12288, 4096), (4096, 12288)):
+            assert ws(T, M, K, bits, x_bf16, kind) == 0, (T, M, K)
+
+
+@pytest.mark.parametrize("x_bf16", [0, 1])
+def test_taken_widths_reserve(ws, x_bf16):
+    for bits in (8, 10, 11, 12, 13, 14):
+        assert ws(512, 4096, 4096, bits, x_bf16) > 512 * 4096 * 2
+        assert ws(1, 4096, 4096, bits, x_bf16) == 0
