@@ -28,6 +28,9 @@ import cbq_native as nat
 import cbq_ops
 
 
+KIND_MIN_T = 33         # tokens from which the codebook's kind chooses the kernel
+
+
 def _device_for(codebook: torch.Tensor) -> torch.device:
     if not torch.cuda.is_available():
         raise RuntimeError("the compressed GPU path needs a ROCm GPU (none visible)")
@@ -104,15 +107,15 @@ class GPUAcceleratedLinear:
         if T == 0:
             return torch.empty(*lead, self.M, dtype=in_dtype, device=dev)
         ops = cbq_ops.load()
-        if in_dtype == torch.bfloat16:
-            # bf16 I/O kernel (batched tokens: bf16 MFMA with fp32 accumulation)
-            out = ops.linear_kind(x.reshape(T, self.K).contiguous(), self.packed, self.codebook,
-                                  self.M, self.bits, self.cb_kind)
-            return out.reshape(*lead, self.M)
-        xc = x.reshape(T, self.K).to(torch.float32).contiguous()
-        out = ops.linear_kind(xc, self.packed, self.codebook, self.M, self.bits,
-                              self.cb_kind).reshape(*lead, self.M)
-        return out if in_dtype == torch.float32 else out.to(in_dtype)
+        # bf16 x keeps its type (batched tokens: bf16 MFMA with fp32 accumulation)
+        xc = x.reshape(T, self.K)
+        xc = (xc if in_dtype == torch.bfloat16 else xc.to(torch.float32)).contiguous()
+        if T < KIND_MIN_T:
+            out = ops.linear(xc, self.packed, self.codebook, self.M, self.bits)
+        else:
+            out = ops.linear_kind(xc, self.packed, self.codebook, self.M, self.bits, self.cb_kind)
+        out = out.reshape(*lead, self.M)
+        return out if out.dtype == in_dtype else out.to(in_dtype)
 
 
 class GPUAcceleratedEmbedding:
