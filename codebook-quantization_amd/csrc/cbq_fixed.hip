@@ -1100,9 +1100,9 @@ int cbq_prefill_f32_splits(int T, int M, int K);
 // decode-first GEMM on the bf16 matrix cores, with a workspace (cbq_gemm.hip);
 // -1 = not handled there.
 int cbq_frag_linear(const void *x, bool f32, const uint8_t *packed, const float *cb, void *out,
-                    int T, int M, int K, int C, int bits, void *ws, size_t ws_bytes,
-                    hipStream_t st);
-size_t cbq_frag_ws_bytes(int T, int M, int K, int bits, bool f32);
+                    int T, int M, int K, int C, int bits, int cb_kind, void *ws,
+                    size_t ws_bytes, hipStream_t st);
+size_t cbq_frag_ws_bytes(int T, int M, int K, int bits, bool f32, int cb_kind);
 
 int cbq_num_cus()
 {
@@ -1178,19 +1178,20 @@ static bool non_finite_f32(int T, int K, int bits, int cb_kind)
 size_t cbq_linear_f32_workspace(int T, int M, int K)
 {
     if (T <= 0 || M <= 0 || K <= 0) return 0;
-    return std::max(cbq_fewtok_ws_bytes(T, M, K, 0, true), cbq_frag_ws_bytes(T, M, K, 0, true));
+    return std::max(cbq_fewtok_ws_bytes(T, M, K, 0, true),
+                    cbq_frag_ws_bytes(T, M, K, 0, true, CBQ_CB_UNKNOWN));
 }
 
-int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebook, float *out,
-                      int T, int M, int K, int C, int bits, void *workspace, size_t ws_bytes,
-                      hipStream_t stream)
+static int linear_f32_kind(const float *x, const uint8_t *packed, const float *codebook,
+                           float *out, int T, int M, int K, int C, int bits, int cb_kind,
+                           void *workspace, size_t ws_bytes, hipStream_t stream)
 {
     if (x && packed && codebook && out && M > 0 && K > 0 && C > 0 && bits >= 1 && bits <= 16) {
         int rc = cbq_fixed_fewtok_ws(x, true, packed, codebook, out, T, M, K, C, bits, workspace,
                                      ws_bytes, stream);
         if (rc < 0)
-            rc = cbq_frag_linear(x, true, packed, codebook, out, T, M, K, C, bits, workspace,
-                                 ws_bytes, stream);
+            rc = cbq_frag_linear(x, true, packed, codebook, out, T, M, K, C, bits, cb_kind,
+                                 workspace, ws_bytes, stream);
         // a workspace below the GEMM's: the fp32 kernel with split K
         if (rc < 0 && T >= 64 && bits != 14)
             rc = prefill_f32_ws(x, packed, codebook, out, T, M, K, C, bits, workspace, ws_bytes,
@@ -1198,6 +1199,14 @@ int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebo
         if (rc >= 0) return rc;
     }
     return ck_linear_f32(x, packed, codebook, out, T, M, K, C, bits, stream);
+}
+
+int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebook, float *out,
+                      int T, int M, int K, int C, int bits, void *workspace, size_t ws_bytes,
+                      hipStream_t stream)
+{
+    return linear_f32_kind(x, packed, codebook, out, T, M, K, C, bits, CBQ_CB_UNKNOWN, workspace,
+                           ws_bytes, stream);
 }
 
 int cbq_linear_xform_f32(const float *x0, const float *x1, float *h_out, int mode, float eps,
@@ -1399,12 +1408,12 @@ size_t cbq_linear_bf16_gemm_workspace(int T, int M, int K, int bits)
     const size_t few = cbq_fewtok_ws_bytes(T, M, K, bits, false);
     if (bits != 8 && (bits < 10 || bits > 14)) return few;   // widths without a prompt kernel
     return std::max(few, std::max(cbq_prefill_ws_bytes(T, M, K),
-                                  cbq_frag_ws_bytes(T, M, K, bits, false)));
+                                  cbq_frag_ws_bytes(T, M, K, bits, false, CBQ_CB_UNKNOWN)));
 }
 
-int cbq_linear_bf16_ws(const void *x_bf16, const uint8_t *packed, const float *codebook,
-                       void *out_bf16, int T, int M, int K, int C, int bits, void *workspace,
-                       size_t ws_bytes, hipStream_t stream)
+static int linear_bf16_kind(const void *x_bf16, const uint8_t *packed, const float *codebook,
+                            void *out_bf16, int T, int M, int K, int C, int bits, int cb_kind,
+                            void *workspace, size_t ws_bytes, hipStream_t stream)
 {
     if (x_bf16 && packed && codebook && out_bf16 && M > 0 && K > 0 && C > 0 && bits >= 1 &&
         bits <= 16) {
@@ -1419,7 +1428,7 @@ int cbq_linear_bf16_ws(const void *x_bf16, const uint8_t *packed, const float *c
         // cbq_linear_bf16_workspace: [x in fragment order][fp32 split
         // partials] of the fused kernel; a smaller one runs as ck_linear_bf16
         int rc = cbq_frag_linear(x_bf16, false, packed, codebook, out_bf16, T, M, K, C, bits,
-                                 workspace, ws_bytes, stream);
+                                 cb_kind, workspace, ws_bytes, stream);
         if (rc < 0)
             rc = cbq_prefill_bf16((const uint16_t *)x_bf16, packed, codebook,
                                   (uint16_t *)out_bf16, T, M, K, C, bits, stream, workspace,
@@ -1429,14 +1438,22 @@ int cbq_linear_bf16_ws(const void *x_bf16, const uint8_t *packed, const float *c
     return ck_linear_bf16(x_bf16, packed, codebook, out_bf16, T, M, K, C, bits, stream);
 }
 
+int cbq_linear_bf16_ws(const void *x_bf16, const uint8_t *packed, const float *codebook,
+                       void *out_bf16, int T, int M, int K, int C, int bits, void *workspace,
+                       size_t ws_bytes, hipStream_t stream)
+{
+    return linear_bf16_kind(x_bf16, packed, codebook, out_bf16, T, M, K, C, bits, CBQ_CB_UNKNOWN,
+                            workspace, ws_bytes, stream);
+}
+
 size_t cbq_linear_gemm_workspace(int T, int M, int K, int bits, int x_bf16, int cb_kind)
 {
-    if (T <= 0 || M <= 0 || K <= 0) return 0;
-    if (x_bf16) return cbq_linear_bf16_gemm_workspace(T, M, K, bits);
-    if (non_finite_f32(T, K, bits, cb_kind)) return prefill_f32_partials(T, M, K);
-    if (bits < 1) return 0;
-    return std::max(cbq_fewtok_ws_bytes(T, M, K, bits, true),
-                    cbq_frag_ws_bytes(T, M, K, bits, true));
+    if (T <= 0 || M <= 0 || K <= 0 || bits < 1) return 0;
+    if (!x_bf16 && non_finite_f32(T, K, bits, cb_kind)) return prefill_f32_partials(T, M, K);
+    size_t need = cbq_frag_ws_bytes(T, M, K, bits, !x_bf16, cb_kind);
+    if (x_bf16 && !need && (bits == 8 || (bits >= 10 && bits <= 14)))
+        need = cbq_prefill_ws_bytes(T, M, K);                // the fused kernel's
+    return std::max(need, cbq_fewtok_ws_bytes(T, M, K, bits, !x_bf16));
 }
 
 int cbq_linear_gemm(const void *x, int x_bf16, const uint8_t *packed, const float *codebook,
@@ -1444,8 +1461,8 @@ int cbq_linear_gemm(const void *x, int x_bf16, const uint8_t *packed, const floa
                     void *workspace, size_t ws_bytes, hipStream_t stream)
 {
     if (x_bf16)
-        return cbq_linear_bf16_ws(x, packed, codebook, out, T, M, K, C, bits, workspace, ws_bytes,
-                                  stream);
+        return linear_bf16_kind(x, packed, codebook, out, T, M, K, C, bits, cb_kind, workspace,
+                                ws_bytes, stream);
     if (x && packed && codebook && out && M > 0 && K > 0 && C > 0 &&
         non_finite_f32(T, K, bits, cb_kind)) {
         const int rc = prefill_f32_ws((const float *)x, packed, codebook, (float *)out, T, M, K, C,
@@ -1454,8 +1471,8 @@ int cbq_linear_gemm(const void *x, int x_bf16, const uint8_t *packed, const floa
                        : ck_linear_f32((const float *)x, packed, codebook, (float *)out, T, M, K, C,
                                        bits, stream);
     }
-    return cbq_linear_f32_ws((const float *)x, packed, codebook, (float *)out, T, M, K, C, bits,
-                             workspace, ws_bytes, stream);
+    return linear_f32_kind((const float *)x, packed, codebook, (float *)out, T, M, K, C, bits,
+                           cb_kind, workspace, ws_bytes, stream);
 }
 
 int ck_embedding_f32(const int32_t *token_ids, const uint8_t *packed, const float *codebook,

@@ -159,7 +159,9 @@ template <int NW> __device__ __forceinline__ uint32_t cb_part(float v, int p)
 __device__ __forceinline__ int frag_of(int m) { return (m >> 2) & 1; }
 __device__ __forceinline__ int frag_row(int m) { return ((m >> 3) << 2) + (m & 3); }
 
-// Fixed-width indices of rows [row0, row0 + M) -> fragments [M / 16][NW][G].
+// Fixed-width indices of rows [row0, row0 + M) -> fragments [M / 16][nw][G],
+// nw the parts there is room for (1 or NW); a codebook that needs more leaves
+// flag 0.
 // A tile is 32 rows x 8 groups: the rows' words arrive in 16-byte pieces
 // (two rows per wave load), go to LDS with an odd row stride, and thread
 // (row, group) unpacks its 32 indices, gathers bf16 values from the LDS
@@ -169,9 +171,9 @@ __device__ __forceinline__ int frag_row(int m) { return ((m >> 3) << 2) + (m & 3
 template <int BITS, int NW>
 __device__ __forceinline__ void prep_w(const uint32_t *__restrict__ words,
                                        const float *__restrict__ cb, int C,
-                                       uint8_t *__restrict__ wf, int *__restrict__ flag, int row0,
-                                       int M, int G, int blk, int nblk, uint16_t *s_tab,
-                                       uint32_t *s_raw, int *s_flag)
+                                       uint8_t *__restrict__ wf, int nw,
+                                       int *__restrict__ flag, int row0, int M, int G, int blk,
+                                       int nblk, uint16_t *s_tab, uint32_t *s_raw, int *s_flag)
 {
     constexpr int NE = (1 << BITS) / kPBlock, NB = NE < 8 ? NE : 8;   // table entries per thread
     static_assert(NE % NB == 0, "whole batches");
@@ -211,6 +213,7 @@ __device__ __forceinline__ void prep_w(const uint32_t *__restrict__ words,
         if (p == 0) {
             const int f = *s_flag;
             parts = (f & 2) ? 0 : f ? NW : 1;
+            if (parts > nw) parts = 0;
             if (blk == 0 && tid == 0) *flag = parts;
             if (parts == 0) return;                        // the GEMM reads the indices
         }
@@ -255,7 +258,7 @@ __device__ __forceinline__ void prep_w(const uint32_t *__restrict__ words,
             for (int i = 0; i < BITS; i++) w[i] = s_raw[row * RS + (tid >> 5) * BITS + i];
             if (g < G) {
                 constexpr uint32_t mask2 = ((1u << BITS) - 1u) << 1;
-                uint8_t *dst = wf + ((size_t)(b * 2 + frag_of(row)) * NW * G + (size_t)p * G + g) *
+                uint8_t *dst = wf + ((size_t)(b * 2 + frag_of(row)) * nw * G + (size_t)p * G + g) *
                                         kFrag + frag_row(row) * 16;
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
@@ -285,7 +288,7 @@ template <int BITS, int NP>
 __global__ __launch_bounds__(kPBlock, 4) void frag_prep_kernel(
     const void *__restrict__ x, uint8_t *__restrict__ xf, int T, int K, int nxb,
     const uint32_t *__restrict__ words, const float *__restrict__ cb, int C,
-    uint8_t *__restrict__ wf, int *__restrict__ flag, int row0, int M)
+    uint8_t *__restrict__ wf, int nw, int *__restrict__ flag, int row0, int M)
 {
     constexpr int NW = NP == 3 ? 3 : 2;
     __shared__ __attribute__((aligned(64))) uint16_t s_tab[1 << BITS];
@@ -298,7 +301,7 @@ __global__ __launch_bounds__(kPBlock, 4) void frag_prep_kernel(
                    (int64_t)nxb * (kPBlock / CBQ_WAVE));
         return;
     }
-    prep_w<BITS, NW>(words, cb, C, wf, flag, row0, M, K >> 5, blockIdx.x - nxb,
+    prep_w<BITS, NW>(words, cb, C, wf, nw, flag, row0, M, K >> 5, blockIdx.x - nxb,
                      gridDim.x - nxb, s_tab, s_raw, &s_flag);
 }
 
@@ -339,7 +342,7 @@ template <class C, int WP> struct GemmStage {
 struct GemmArgs {
     const uint8_t *xf;      // [T / 16][G][NP] fragments
     const uint8_t *wf;      // [M / 16][nw][G] fragments of the slab
-    const int *flag;        // W parts in use; 0: the fragments do not hold W
+    const int *flag;        // W parts in use; 0: the slab does not hold W
     void *out;              // out + slab offset, row stride ldo
     float *part;            // split-K partials [S][tiles] in fragment order
     // for flag 0: the caller's x, the slab's first index words, the codebook
@@ -428,7 +431,7 @@ __device__ __forceinline__ void tile_at(int tile, int nT, int nM, int &tt, int &
 // One wave's products without the fragments, on the fp32 matrix cores from the
 // index stream: acc as the K loop leaves it.  For codebooks that the bf16
 // parts cannot stand for (flag 0: an infinite value times a zero part of x
-// would be a NaN).  Column group g's step e takes columns 8 q + e of lane
+// would be a NaN) or that need more parts than their caller reserved.  Column group g's step e takes columns 8 q + e of lane
 // quarter q, for x and W alike.  Loads go out as the compiler places them and
 // every wave decodes its own rows: a path for callers that do not say what
 // their codebook holds, not for speed.
@@ -440,6 +443,7 @@ __device__ __forceinline__ void fp32_fragments(const GemmArgs &a, uint8_t *lds, 
     const int lane = threadIdx.x & (CBQ_WAVE - 1), q = lane >> 4, fr = lane & 15;
     const int bits = a.bits, C = min(a.C, 1 << bits);
     const uint32_t mask = (1u << bits) - 1u;
+    constexpr int kSteps = Cfg::NP == 3 ? 4 : 1;     // in flight; the K loop sets the registers
     const float *tab = a.cb;
     if (C * 4 <= lds_bytes) {
         float *const s = (float *)lds;
@@ -456,7 +460,7 @@ __device__ __forceinline__ void fp32_fragments(const GemmArgs &a, uint8_t *lds, 
     }
 #pragma unroll 1
     for (int g = g0; g < g0 + n; g++) {
-#pragma unroll 4                                       // no more: the K loop sets the registers
+#pragma unroll kSteps
         for (int e = 0; e < 8; e++) {
             float xv[Cfg::TB], w[Cfg::MB];
             const int o = (q * 8 + e) * bits, k = o >> 5, k1 = min(k + 1, bits - 1);
@@ -668,7 +672,7 @@ __global__ __launch_bounds__(kGBlock, 2) void frag_gemm_kernel(GemmArgs a)
     };
     if (n > 0 && nW == 1) all(std::integral_constant<int, 1>{});
     else if (n > 0 && nW > 1) all(std::integral_constant<int, Cfg::NW>{});
-    if (NP == 3 && nW == 0)
+    if (nW == 0)
         fp32_fragments<Cfg>(a, lds, t0, m0, wt, wm, g0, n, acc, (int)sizeof(lds));
     else if constexpr (FOLD)
 #pragma unroll
@@ -811,8 +815,8 @@ int launch_gemm(int NP, int shape, GemmArgs a, hipStream_t st)
 
 template <int BITS>
 int launch_prep(int NP, const void *x, uint8_t *xf, int T, int K, bool with_x,
-                const uint32_t *words, const float *cb, int C, uint8_t *wf, int *flag, int row0,
-                int M, hipStream_t st)
+                const uint32_t *words, const float *cb, int C, uint8_t *wf, int nw, int *flag,
+                int row0, int M, hipStream_t st)
 {
     const int cus = cbq_num_cus();
     const int64_t units = (int64_t)((T + 15) >> 4) * (K >> 5);
@@ -821,10 +825,10 @@ int launch_prep(int NP, const void *x, uint8_t *xf, int T, int K, bool with_x,
     const int nwb = (int)std::min<int64_t>(tiles, kPrepBlocks * cus);
     if (NP == 3)
         hipLaunchKernelGGL((frag_prep_kernel<BITS, 3>), dim3(nxb + nwb), dim3(kPBlock), 0, st, x, xf,
-                           T, K, nxb, words, cb, C, wf, flag, row0, M);
+                           T, K, nxb, words, cb, C, wf, nw, flag, row0, M);
     else
         hipLaunchKernelGGL((frag_prep_kernel<BITS, 1>), dim3(nxb + nwb), dim3(kPBlock), 0, st, x, xf,
-                           T, K, nxb, words, cb, C, wf, flag, row0, M);
+                           T, K, nxb, words, cb, C, wf, nw, flag, row0, M);
     return cbq_launch_status("frag_prep_kernel");
 }
 
@@ -834,8 +838,14 @@ size_t w_bytes(int rows, int K, int nw)
 {
     return (size_t)((rows + 31) >> 5) * 2 * (K >> 5) * nw * kFrag;
 }
-// W parts a fixed-width slab has room for
-int w_parts(int NP) { return NP == 3 ? 3 : 2; }
+// W parts a fixed-width slab has room for: one where the codebook is said to
+// hold bf16 numbers only (every lossless one), or a non-finite value (no
+// fragments are written then).
+int w_parts(int NP, int cb_kind)
+{
+    if (cb_kind == CBQ_CB_BF16 || (NP == 3 && cb_kind == CBQ_CB_NON_FINITE)) return 1;
+    return NP == 3 ? 3 : 2;
+}
 size_t part_bytes(const GemmPlan &p, int T, int NP)
 {
     if (p.S <= 1) return 0;
@@ -914,11 +924,11 @@ size_t gemm_ws_bytes(const GemmPlan &p, int NP, int nw, int T, int K)
 
 // out [T][M] = x @ W^T over the slabs of W; BITS-wide indices.
 template <int BITS>
-int frag_linear(int NP, const void *x, const uint32_t *words, const float *cb, void *out, int T,
-                int M, int K, int C, uint8_t *ws, hipStream_t st)
+int frag_linear(int NP, int nw, const void *x, const uint32_t *words, const float *cb, void *out,
+                int T, int M, int K, int C, uint8_t *ws, hipStream_t st)
 {
-    const GemmPlan p = gemm_plan(T, M, K, NP, w_parts(NP));
-    GemmArgs a = gemm_args(p, NP, w_parts(NP), x, T, M, K, ws);
+    const GemmPlan p = gemm_plan(T, M, K, NP, nw);
+    GemmArgs a = gemm_args(p, NP, nw, x, T, M, K, ws);
     a.cb = cb;
     a.C = C;
     a.bits = BITS;
@@ -927,7 +937,7 @@ int frag_linear(int NP, const void *x, const uint32_t *words, const float *cb, v
         a.words = words + (int64_t)r0 * (K >> 5) * BITS;
         a.out = (uint8_t *)out + (size_t)r0 * (NP == 3 ? 4 : 2);
         int rc = launch_prep<BITS>(NP, x, (uint8_t *)a.xf, T, K, r0 == 0, words, cb, C,
-                                   (uint8_t *)a.wf, (int *)ws, r0, a.M, st);
+                                   (uint8_t *)a.wf, nw, (int *)ws, r0, a.M, st);
         if (!rc) rc = launch_gemm(NP, p.shape, a, st);
         if (rc) return rc;
     }
@@ -960,38 +970,39 @@ bool frag_shape(int T, int M, int K, bool f32)
 // against 97 us fused, 12288 x 4096 100 / 100, 4096 x 4096 51 / 62; T = 2048,
 // 12288 x 4096: 221 / 263), so the smaller estimate is taken: 13-bit indices
 // read and fragments written at 4.8 TB/s, two launches, the GEMM's plan.
-// 8-bit codebooks are taken to be fp32 values (two parts of W: T = 512,
-// 4096 x 4096: 82 against 62 us fused).
+// Codebooks of other values have two parts of W (T = 512, 4096 x 4096: 82
+// against 62 us fused); of unknown kind, 8-bit ones are taken to.
 // bits 0: any width the GEMM takes.
-size_t cbq_frag_ws_bytes(int T, int M, int K, int bits, bool f32)
+size_t cbq_frag_ws_bytes(int T, int M, int K, int bits, bool f32, int cb_kind)
 {
     if (!frag_shape(T, M, K, f32) || !(bits == 0 || bits == 8 || (bits >= 10 && bits <= 14)))
         return 0;
     const int NP = f32 ? 3 : 1;
-    const GemmPlan p = gemm_plan(T, M, K, NP, w_parts(NP));
+    const int nw = w_parts(NP, cb_kind);
+    const GemmPlan p = gemm_plan(T, M, K, NP, nw);
     if (!f32) {
-        const bool two = bits == 8;
+        const bool two = cb_kind == CBQ_CB_UNKNOWN ? bits == 8 : nw == 2;
         const float prep = (float)M * (float)K * (two ? 5.f : 3.6f) / 4.8e6f;
         const float fused = cbq_prefill_us(T, M, K);
         if (fused > 0.f && prep + 6.f + p.us * (two ? 1.9f : 1.f) > fused) return 0;
     }
-    return gemm_ws_bytes(p, NP, w_parts(NP), T, K);
+    return gemm_ws_bytes(p, NP, nw, T, K);
 }
 
 // The batched linear over fixed-width indices with a workspace of at least
 // cbq_frag_ws_bytes (16-byte aligned); -1: not handled here.
 int cbq_frag_linear(const void *x, bool f32, const uint8_t *packed, const float *cb, void *out,
-                    int T, int M, int K, int C, int bits, void *ws, size_t ws_bytes,
-                    hipStream_t st)
+                    int T, int M, int K, int C, int bits, int cb_kind, void *ws,
+                    size_t ws_bytes, hipStream_t st)
 {
-    const size_t need = cbq_frag_ws_bytes(T, M, K, bits, f32);
+    const size_t need = cbq_frag_ws_bytes(T, M, K, bits, f32, cb_kind);
     if (!need || !ws || ws_bytes < need || (((uintptr_t)ws | (uintptr_t)x) & 15) != 0 ||
         ((uintptr_t)packed & 3) != 0)
         return -1;
 #define CBQ_FL(B)                                                                              \
     case B:                                                                                    \
-        return frag_linear<B>(f32 ? 3 : 1, x, (const uint32_t *)packed, cb, out, T, M, K, C,   \
-                              (uint8_t *)ws, st);
+        return frag_linear<B>(f32 ? 3 : 1, w_parts(f32 ? 3 : 1, cb_kind), x,                   \
+                              (const uint32_t *)packed, cb, out, T, M, K, C, (uint8_t *)ws, st);
     switch (bits) {
         CBQ_FL(8) CBQ_FL(10) CBQ_FL(11) CBQ_FL(12) CBQ_FL(13) CBQ_FL(14)
     default: return -1;

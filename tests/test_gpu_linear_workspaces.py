@@ -126,3 +126,32 @@ def test_codebook_changed_in_place(cuda):
             ok = r.isfinite()
             if bool(ok.any()):
                 assert _rel(y[ok], r[ok]) <= (TOL_CHAIN if xx is x else 2.0 ** -9)
+
+
+def _gemm(cuda, x, packed, cb, M, K, bits, kind):
+    lib = nat.load()
+    T, bf16 = x.shape[0], int(x.dtype == torch.bfloat16)
+    n = int(lib.cbq_linear_gemm_workspace(T, M, K, bits, bf16, kind))
+    buf = torch.full((max(n, 16) + 4096,), 0xA5, dtype=torch.uint8, device=cuda)
+    out = torch.full((T, M), float("nan"), dtype=x.dtype, device=cuda)
+    nat.check(lib.cbq_linear_gemm(x.data_ptr(), bf16, packed.data_ptr(), cb.data_ptr(),
+                                  out.data_ptr(), T, M, K, cb.numel(), bits, kind, buf.data_ptr(),
+                                  n, nat.stream_ptr(cuda)), "cbq_linear_gemm")
+    assert bool((buf[max(n, 16):] == 0xA5).all())        # nothing past the workspace
+    return out
+
+
+@pytest.mark.parametrize("T,M,K,bits", [(64, 33, 64, 12), (33, 4100, 1056, 13), (300, 520, 4096, 8),
+                                        (129, 2049, 96, 14), (700, 1030, 544, 11),
+                                        (1030, 3000, 544, 13), (2050, 4000, 1024, 10)])
+@pytest.mark.parametrize("kind", [0, 1, 2, 3])
+@pytest.mark.parametrize("holds", ["bf16", "fp32"])
+def test_every_kind_gives_the_product(cuda, T, M, K, bits, kind, holds):
+    """Declared as anything, a codebook's product is its own: one part of the
+    weights reserved where three are needed falls back to fp32 products."""
+    print(f"kind {kind} {holds} T{T} M{M} K{K} bits{bits}", flush=True)
+    packed, cb, w = _matrix(cuda, M, K, bits, holds, T + M)
+    x = torch.randn(T, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(K))
+    assert _rel(_gemm(cuda, x, packed, cb, M, K, bits, kind), x.double() @ w.T) <= TOL_CHAIN
+    xb = x.bfloat16()
+    assert _rel(_gemm(cuda, xb, packed, cb, M, K, bits, kind), xb.double() @ w.T) <= 2.0 ** -9

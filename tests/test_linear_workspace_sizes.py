@@ -30,3 +30,20 @@ def test_taken_widths_reserve(ws, x_bf16):
     for bits in (8, 10, 11, 12, 13, 14):
         assert ws(512, 4096, 4096, bits, x_bf16) > 512 * 4096 * 2
         assert ws(1, 4096, 4096, bits, x_bf16) == 0
+
+
+def test_one_part_of_a_lossless_codebook(ws):
+    """A codebook of bf16 numbers reserves two bytes a weight beside x's
+    fragments and the partials, one of other values three (fp32 x) or two
+    (bf16 x) times that; an unknown one as much as any."""
+    M, K, BF16, FP32 = 12288, 4096, 1, 2
+    w = 2 * M * K
+    for T in (33, 512, 2048):
+        assert 2 * w > ws(T, M, K, 13, 0, BF16) > w
+        assert ws(T, M, K, 13, 0, FP32) >= 3 * w
+        assert ws(T, M, K, 13, 0, 0) >= ws(T, M, K, 13, 0, FP32)
+    T = 2048                                       # (decodes first)
+    assert 2 * w > ws(T, M, K, 13, 1, BF16) > w
+    # a lossless lm_head: slabs of at most 384 MiB
+    x = 512 * 4096 * 6
+    assert ws(512, 151936, 4096, 13, 0, BF16) <= (384 << 20) + x + (1 << 20)
