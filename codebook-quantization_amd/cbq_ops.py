@@ -23,6 +23,7 @@ from __future__ import annotations
 
 import os
 
+import numpy as np
 import torch
 
 import cbq_native
@@ -36,16 +37,16 @@ CB_UNKNOWN, CB_BF16, CB_FP32, CB_NON_FINITE = range(4)
 _loaded = False
 
 
-def codebook_kind(codebook: torch.Tensor) -> int:
-    """What a float32 codebook holds: CB_BF16 (finite bf16 numbers only),
-    CB_FP32 (finite) or CB_NON_FINITE.  Found out once, where a matrix is
-    loaded (one synchronisation); it chooses the kernel and its workspace, and
-    a codebook that is changed in place afterwards still gives its own
-    product."""
-    cb = codebook.detach().reshape(-1)
-    finite, exact = torch.stack([torch.isfinite(cb).all(),
-                                 ((cb.view(torch.int32) & 0xFFFF) == 0).all()]).tolist()
-    return CB_NON_FINITE if not finite else CB_BF16 if exact else CB_FP32
+def codebook_kind(codebook) -> int:
+    """What a float32 codebook (a tensor or an array) holds: CB_BF16 (finite
+    bf16 numbers only), CB_FP32 (finite) or CB_NON_FINITE.  Found out once,
+    where a matrix is loaded (one copy to the host); it chooses the kernel and
+    its workspace, and a codebook that is changed in place afterwards still
+    gives its own product."""
+    cb = codebook.detach().cpu().numpy() if isinstance(codebook, torch.Tensor) else codebook
+    if not np.isfinite(cb).all():
+        return CB_NON_FINITE
+    return CB_FP32 if (cb.reshape(-1).view(np.uint32) & 0xFFFF).any() else CB_BF16
 
 
 def load(path: str = SO_PATH):

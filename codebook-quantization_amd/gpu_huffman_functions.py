@@ -548,7 +548,7 @@ class HuffmanCodebookLinear:
         self.split = None
         self.cols = None
         self._inv = None
-        self._cb_kind = cbq_ops.codebook_kind(torch.from_numpy(self._cb_np))
+        self._cb_kind = cbq_ops.codebook_kind(self._cb_np)
         if layout in ("auto", "split") and split_eligible(self.M, self.K):
             idx = SymbolDecoder(dev.words, dev.chunk_off, dev.sub_len, self._lengths,
                                 device).indices(self.M * self.K)
@@ -586,7 +586,7 @@ class HuffmanCodebookLinear:
         self.device = cb.device
         self._cb_dev = cb
         self._cb_np = cb.cpu().numpy()
-        self._cb_kind = cbq_ops.codebook_kind(torch.from_numpy(self._cb_np))
+        self._cb_kind = cbq_ops.codebook_kind(self._cb_np)
         self._lengths = np.ascontiguousarray(t.lengths, np.uint8)
         self.cols = None
         if isinstance(t, dfm.SplitTensor):

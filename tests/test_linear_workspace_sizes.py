@@ -47,3 +47,15 @@ def test_one_part_of_a_lossless_codebook(ws):
     # a lossless lm_head: slabs of at most 384 MiB
     x = 512 * 4096 * 6
     assert ws(512, 151936, 4096, 13, 0, BF16) <= (384 << 20) + x + (1 << 20)
+
+
+def test_codebook_kind():
+    import numpy as np
+    import torch
+    import cbq_ops as o
+    cb = np.array([0.0, -0.0, 1.5, -2.0 ** -126, 2.0 ** -133], np.float32)
+    for values, want in (([], o.CB_BF16), ([0.1], o.CB_FP32), ([2.0 ** -140], o.CB_FP32),
+                         ([np.inf], o.CB_NON_FINITE), ([0.1, -np.inf], o.CB_NON_FINITE),
+                         ([np.nan], o.CB_NON_FINITE)):
+        a = np.concatenate([cb, np.array(values, np.float32)])
+        assert o.codebook_kind(a) == want == o.codebook_kind(torch.from_numpy(a))
