@@ -1421,13 +1421,18 @@ static int linear_bf16_kind(const void *x_bf16, const uint8_t *packed, const flo
                                            bits, workspace, ws_bytes, stream);
         if (rc >= 0) return rc;
     }
-    // (64 tokens that the few-token kernel takes go there)
     if (x_bf16 && packed && codebook && out_bf16 && T >= 64 && M > 0 && K > 0 && C > 0 &&
-        bits >= 1 && bits <= 16 && (T > 64 || K % 128 != 0)) {
-        // a workspace of cbq_linear_bf16_gemm_workspace: decode first; of
+        bits >= 1 && bits <= 16) {
+        // 64 tokens: the few-token kernel where it takes them.  A workspace of
+        // cbq_linear_gemm_workspace: decode first; of
         // cbq_linear_bf16_workspace: [x in fragment order][fp32 split
         // partials] of the fused kernel; a smaller one runs as ck_linear_bf16
-        int rc = cbq_frag_linear(x_bf16, false, packed, codebook, out_bf16, T, M, K, C, bits,
+        int rc = -1;
+        if (T == 64)
+            rc = cbq_fixed_fewtok_t_bf16((const uint16_t *)x_bf16, packed, codebook,
+                                         (uint16_t *)out_bf16, T, M, K, C, bits, stream);
+        if (rc < 0)
+            rc = cbq_frag_linear(x_bf16, false, packed, codebook, out_bf16, T, M, K, C, bits,
                                  cb_kind, workspace, ws_bytes, stream);
         if (rc < 0)
             rc = cbq_prefill_bf16((const uint16_t *)x_bf16, packed, codebook,
@@ -1450,10 +1455,12 @@ size_t cbq_linear_gemm_workspace(int T, int M, int K, int bits, int x_bf16, int 
 {
     if (T <= 0 || M <= 0 || K <= 0 || bits < 1) return 0;
     if (!x_bf16 && non_finite_f32(T, K, bits, cb_kind)) return prefill_f32_partials(T, M, K);
+    const size_t few = cbq_fewtok_ws_bytes(T, M, K, bits, !x_bf16);
+    if (x_bf16 && T <= 64 && K % 128 == 0) return few;   // the few-token kernel's tokens
     size_t need = cbq_frag_ws_bytes(T, M, K, bits, !x_bf16, cb_kind);
     if (x_bf16 && !need && (bits == 8 || (bits >= 10 && bits <= 14)))
         need = cbq_prefill_ws_bytes(T, M, K);                // the fused kernel's
-    return std::max(need, cbq_fewtok_ws_bytes(T, M, K, bits, !x_bf16));
+    return std::max(need, few);
 }
 
 int cbq_linear_gemm(const void *x, int x_bf16, const uint8_t *packed, const float *codebook,

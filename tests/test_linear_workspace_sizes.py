@@ -59,3 +59,11 @@ def test_codebook_kind():
                          ([np.nan], o.CB_NON_FINITE)):
         a = np.concatenate([cb, np.array(values, np.float32)])
         assert o.codebook_kind(a) == want == o.codebook_kind(torch.from_numpy(a))
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_64_bf16_tokens_reserve_for_the_few_token_kernel(ws, kind):
+    """K % 128 == 0: at most x's fragments."""
+    for M, K in ((4096, 4096), (12288, 4096), (4096, 12288)):
+        assert ws(64, M, K, 13, 1, kind) <= 64 * K * 2
+    assert ws(64, 4096, 4064, 13, 1, kind) > 4096 * 4064      # a prompt kernel's shape
