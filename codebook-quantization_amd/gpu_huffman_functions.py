@@ -399,7 +399,7 @@ def split_prefill(split, inv: torch.Tensor, x: torch.Tensor, M: int, K: int,
     kernels."""
     T = int(x.shape[0])
     if finite and T >= SPLIT_GEMM_MIN_T[torch.float32]:
-        return split_gemm(split, x, M)
+        return split_gemm(split, x.detach(), M)     # as the calls below: no autograd
     if 1 <= T <= FEWTOK_MAX_T and split_fewtok_eligible(K) and x.data_ptr() % 16 == 0:
         return split_fewtok([split], x, [M], K)[0]
     packed, bits = _packed_for_gemm(split, M * K, int(codebook.numel()), x.device, inv)
@@ -633,6 +633,10 @@ class HuffmanCodebookLinear:
         gemm_dtype = torch.bfloat16 if in_dtype == torch.bfloat16 else torch.float32
         if self.split is not None and self._finite and T >= SPLIT_GEMM_MIN_T[gemm_dtype]:
             xg = x.reshape(T, self.K).to(gemm_dtype)
+            if T > FEWTOK_MAX_T or not split_fewtok_eligible(self.K):
+                # no backward: an operator's output would ask for gradients all
+                # the same (and refuse .numpy()); split_linear's, below, does
+                xg = xg.detach()
             out = split_gemm(self.split, xg, self.M).reshape(*lead, self.M)
             return out if out.dtype == in_dtype else out.to(in_dtype)
         xc = x.reshape(T, self.K).to(torch.float32).contiguous()
