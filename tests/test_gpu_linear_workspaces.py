@@ -155,3 +155,94 @@ def test_every_kind_gives_the_product(cuda, T, M, K, bits, kind, holds):
     assert _rel(_gemm(cuda, x, packed, cb, M, K, bits, kind), x.double() @ w.T) <= TOL_CHAIN
     xb = x.bfloat16()
     assert _rel(_gemm(cuda, xb, packed, cb, M, K, bits, kind), xb.double() @ w.T) <= 2.0 ** -9
+
+
+@pytest.mark.parametrize("dtype,K,kind,holds", [
+    (torch.bfloat16, 524320, 0, "fp32"), (torch.bfloat16, 524320, 1, "bf16"),
+    (torch.float32, 262176, 2, "fp32"), (torch.float32, 262176, 1, "fp32"),
+    (torch.float32, 786464, 1, "bf16")])
+def test_slabs(cuda, dtype, K, kind, holds):
+    """Rows so long that the weights go slab by slab (256 rows each at least):
+    two and three parts of the weights, one, and the fp32 products of a
+    codebook declared to need one."""
+    T, M, bits = 80, 520, 12
+    print(f"slabs {dtype} K{K} kind {kind} {holds}", flush=True)
+    packed, cb, w = _matrix(cuda, M, K, bits, holds, 3)
+    x = torch.randn(T, K, device=cuda).to(dtype)
+    y, ref = _gemm(cuda, x, packed, cb, M, K, bits, kind), x.double() @ w.T
+    if dtype == torch.bfloat16:
+        assert _rel(y, ref) <= 2.0 ** -9
+    else:
+        # A sum of n terms of random sign in one chain of roundings, each half
+        # an ulp (2^-24) of a partial sum that grows as the root of its length:
+        # rel-L2 <= 2^-24 sqrt(n / 2).  Fragments: a chain of 16 groups x 3 (6
+        # with three parts of W) MFMAs, then one of K / 512 totals; fp32
+        # products: one of K / 4 MFMAs.  (No more where K is split.)
+        n = 48 * (2 if holds == "fp32" else 1) + K / 512
+        if kind == 1 and holds == "fp32":
+            n = K / 4
+        assert _rel(y, ref) <= 2.0 ** -24 * (n / 2) ** 0.5
+
+
+@pytest.mark.parametrize("M,K", [(200704, 1024), (66000, 3072), (49300, 4096)])
+def test_split_slabs(cuda, M, K):
+    """Split-format matrices of more than 384 MiB of fragments: the second
+    slab's rows start inside the matrix, in each chunk geometry (whole rows
+    per chunk, chunks across rows, whole chunks per row)."""
+    import cbq_ops
+    from test_gpu_frag_gemm import _split_matrix
+    print(f"split slabs M{M} K{K}", flush=True)
+    assert 2 * M * K > 384 << 20
+    t, w = _split_matrix(cuda, M, K, 5)
+    x = torch.randn(33, K, device=cuda)
+    op = cbq_ops.load().split_gemm
+    y, ref = op(x, *t.keep, M), x.double() @ w.T
+    assert _rel(y, ref) <= TOL_F32
+    rows = (y.double() - ref).norm(dim=0) / ref.norm(dim=0)    # every row, both slabs
+    assert float(rows.max()) <= 10 * TOL_F32
+    yb = op(x.bfloat16(), *t.keep, M)
+    assert _rel(yb, x.bfloat16().double() @ w.T) <= 2.0 ** -9
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+def test_bf16_non_finite_x(cuda, kind):
+    """Infinities and NaNs of bf16 x over a lossless codebook."""
+    T, M, K, bits = 300, 1040, 2048, 13
+    packed, cb, w = _matrix(cuda, M, K, bits, "bf16", 5)
+    x = torch.randn(T, K, device=cuda).bfloat16()
+    x[3, 7], x[9, 100], x[11, 0] = float("inf"), float("-inf"), float("nan")
+    x[20] = 0.0
+    assert nat.load().cbq_linear_gemm_workspace(T, M, K, bits, 1, kind) > 0
+    y, ref = _gemm(cuda, x, packed, cb, M, K, bits, kind), x.double() @ w.T
+    assert torch.equal(y.isnan(), ref.isnan())
+    assert torch.equal(y.isposinf(), ref.isposinf()) and torch.equal(y.isneginf(), ref.isneginf())
+    ok = ref.isfinite()
+    assert _rel(y[ok], ref[ok]) <= 2.0 ** -9
+
+
+def test_huffman_non_finite_codebook(cuda):
+    """A Huffman matrix with an infinite value, batched: infinities and NaNs
+    where the products have them, in both formats."""
+    import numpy as np
+    import codebook_builder as cbb
+    import huffman_codebook as hc
+    from test_gpu_huffman import _lin
+    M, K = 64, 1024
+    rng = np.random.default_rng(3)
+    wn = cbb.bf16_round(rng.standard_normal((M, K)) * 0.02)
+    cb, idx = cbb.frequency_sorted_codebook(wn)
+    cb = cb.copy()
+    cb[len(cb) // 2] = np.inf
+    enc = hc.huffman_encode_indices(idx, shape=(M, K))
+    w = torch.from_numpy(cb).to(cuda)[torch.from_numpy(idx.astype(np.int64)).to(cuda)]
+    w = w.reshape(M, K).double()
+    for layout in ("auto", "stream"):
+        lin = _lin(enc, cb, M, K, layout=layout)
+        for T in (64, 100):
+            x = torch.randn(T, K, device=cuda)
+            x[1] = x[1].bfloat16().float()
+            y, ref = lin(x), x.double() @ w.T
+            assert torch.equal(y.isnan(), ref.isnan()), (layout, T)
+            assert torch.equal(y.isposinf(), ref.isposinf())
+            ok = ref.isfinite()
+            assert _rel(y[ok], ref[ok]) <= TOL_CHAIN
