@@ -1166,13 +1166,15 @@ static int prefill_f32_ws(const float *x, const uint8_t *packed, const float *co
                            split ? (float *)ws : nullptr);
 }
 
-// Calls of a non-finite codebook that run on the fp32 kernel: the GEMM's.  The
-// few-token kernels' parts of x would make a NaN of an infinite weight where a
-// part is zero.
-static bool non_finite_f32(int T, int K, int bits, int cb_kind)
+// Calls that run on the fp32 kernel in place of the decode-first GEMM: of a
+// non-finite codebook (the few-token kernels' parts of x would make a NaN of an
+// infinite weight where a part is zero) and of an fp32 codebook below 256
+// columns (the GEMM leaves out the smallest part products; cbq_gemm.hip has
+// the errors).
+static bool fp32_kernel(int T, int K, int bits, int cb_kind)
 {
-    return cb_kind == CBQ_CB_NON_FINITE && T >= 33 && K % 32 == 0 &&
-           (bits == 8 || (bits >= 10 && bits <= 14));
+    return (cb_kind == CBQ_CB_NON_FINITE || (cb_kind == CBQ_CB_FP32 && K < 256)) && T >= 33 &&
+           K % 32 == 0 && (bits == 8 || (bits >= 10 && bits <= 14));
 }
 
 size_t cbq_linear_f32_workspace(int T, int M, int K)
@@ -1454,7 +1456,7 @@ int cbq_linear_bf16_ws(const void *x_bf16, const uint8_t *packed, const float *c
 size_t cbq_linear_gemm_workspace(int T, int M, int K, int bits, int x_bf16, int cb_kind)
 {
     if (T <= 0 || M <= 0 || K <= 0 || bits < 1) return 0;
-    if (!x_bf16 && non_finite_f32(T, K, bits, cb_kind)) return prefill_f32_partials(T, M, K);
+    if (!x_bf16 && fp32_kernel(T, K, bits, cb_kind)) return prefill_f32_partials(T, M, K);
     const size_t few = cbq_fewtok_ws_bytes(T, M, K, bits, !x_bf16);
     if (x_bf16 && T <= 64 && K % 128 == 0) return few;   // the few-token kernel's tokens
     size_t need = cbq_frag_ws_bytes(T, M, K, bits, !x_bf16, cb_kind);
@@ -1471,7 +1473,7 @@ int cbq_linear_gemm(const void *x, int x_bf16, const uint8_t *packed, const floa
         return linear_bf16_kind(x, packed, codebook, out, T, M, K, C, bits, cb_kind, workspace,
                                 ws_bytes, stream);
     if (x && packed && codebook && out && M > 0 && K > 0 && C > 0 &&
-        non_finite_f32(T, K, bits, cb_kind)) {
+        fp32_kernel(T, K, bits, cb_kind)) {
         const int rc = prefill_f32_ws((const float *)x, packed, codebook, (float *)out, T, M, K, C,
                                       bits, workspace, ws_bytes, stream);
         return rc >= 0 ? rc

@@ -16,7 +16,14 @@
 //   3. frag_reduce_kernel adds the split-K partials in split order.
 // Products of fp32 x with bf16 weights are exact (24-bit significands as
 // 8 + 8 + 8 bits); with other weights the sum of the six largest of the nine
-// part products.
+// part products, short of the whole by less than 2^-22.  From K = 256 on the
+// folded sums more than make up for that; rel-L2 against 64 bits, this /
+// exact products in the fp32 kernel's one chain: K = 32 1.3e-7 / 1.0e-7, 128
+// 2.0e-7 / 2.0e-7, 256 2.0e-7 / 2.8e-7, 1024 2.1e-7 / 2.9e-7, 12288 2.3e-7 /
+// 5.0e-7 (of one sign throughout: 1.2e-7 / 0.8e-7, 1.6e-7 / 1.6e-7, 1.2e-7 /
+// 2.3e-7, 0.8e-7 / 1.2e-7, 0.8e-7 / 1.2e-7, with a mean of -5e-8).  Below,
+// such a codebook is multiplied in fp32.  x's lower parts go down to 2^-133:
+// of |x| under 2^-110 an absolute 2^-133 may be lost.
 //
 // Why decode first: a fused kernel gathers every weight again for each 512
 // tokens, and on this chip the decode's VALU and LDS work adds to the MFMA
@@ -48,6 +55,7 @@ constexpr size_t kSlabBytes = (size_t)384 << 20;
 // 1.8e-7 at K = 2048, 2.5e-7 at 12288, for one addition per accumulator and
 // 3 f MFMAs (T = 512, 4096 x 12288: 130 -> 142 us at f = 16).
 int fold_groups(int n) { return n < 96 ? 4 : n < 400 ? 8 : 16; }
+constexpr int kSixMinK = 256;                  // K of fp32 x times three-part weights
 constexpr int kHeader = 256;                   // workspace header: the W part count
 
 typedef unsigned short g_u16x2 __attribute__((ext_vector_type(2)));
@@ -213,7 +221,7 @@ __device__ __forceinline__ void prep_w(const uint32_t *__restrict__ words,
         if (p == 0) {
             const int f = *s_flag;
             parts = (f & 2) ? 0 : f ? NW : 1;
-            if (parts > nw) parts = 0;
+            if (parts > nw || (NW == 3 && parts > 1 && G < kSixMinK / 32)) parts = 0;
             if (blk == 0 && tid == 0) *flag = parts;
             if (parts == 0) return;                        // the GEMM reads the indices
         }
@@ -431,7 +439,8 @@ __device__ __forceinline__ void tile_at(int tile, int nT, int nM, int &tt, int &
 // One wave's products without the fragments, on the fp32 matrix cores from the
 // index stream: acc as the K loop leaves it.  For codebooks that the bf16
 // parts cannot stand for (flag 0: an infinite value times a zero part of x
-// would be a NaN) or that need more parts than their caller reserved.  Column group g's step e takes columns 8 q + e of lane
+// would be a NaN), that need more parts than their caller reserved, or that
+// are short of kSixMinK columns.  Column group g's step e takes columns 8 q + e of lane
 // quarter q, for x and W alike.  Loads go out as the compiler places them and
 // every wave decodes its own rows: a path for callers that do not say what
 // their codebook holds, not for speed.

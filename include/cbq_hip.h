@@ -58,7 +58,10 @@ size_t cbq_linear_f32_workspace(int T, int M, int K);
  * multiplied on the bf16 matrix cores with fp32 accumulation; K is split
  * over blocks when the output tiles alone would leave CUs idle (partials in
  * the workspace, summed in split order).  A codebook with values that are
- * not bf16 numbers is split into bf16 parts as well.  With a smaller
+ * not bf16 numbers is split into bf16 parts as well, and the six largest of a
+ * product's nine parts are summed (short by less than 2^-22 each; in total
+ * closer to the exact sum than ck_linear_f32), below 256 columns the fp32
+ * products themselves.  |x| under 2^-110 may lose an absolute 2^-133.  With a smaller
  * workspace it is ck_linear_f32, whose fp32 kernel (T >= 64) then splits K
  * where it would leave CUs idle and the partials (fp32 [splits][T][M], at most
  * 16 splits) fit.  No counterpart in the reference: batched
@@ -78,8 +81,9 @@ int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebo
 /* The batched linear for fp32 or bf16 x (x_bf16 != 0; out likewise) with a
  * workspace of cbq_linear_gemm_workspace bytes (256-byte aligned):
  * cbq_linear_f32_ws / cbq_linear_bf16_ws for a codebook of cb_kind.  fp32 x
- * and a non-finite codebook: ck_linear_f32's fp32 kernel with split K from 33
- * tokens on (the bf16 parts of x cannot multiply an infinity).  No
+ * and a non-finite codebook, or one of other than bf16 values and K < 256:
+ * ck_linear_f32's fp32 kernel with split K from 33 tokens on (the bf16 parts of
+ * x cannot multiply an infinity, and short sums keep every part product).  No
  * counterpart in the reference: GPUAcceleratedLinear
  * (src/gpu_accelerated_functions.py:928-950) over batched tokens. */
 int cbq_linear_gemm(const void *x, int x_bf16, const uint8_t *packed, const float *codebook,

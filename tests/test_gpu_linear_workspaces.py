@@ -246,3 +246,24 @@ def test_huffman_non_finite_codebook(cuda):
             assert torch.equal(y.isposinf(), ref.isposinf())
             ok = ref.isfinite()
             assert _rel(y[ok], ref[ok]) <= TOL_CHAIN
+
+
+@pytest.mark.parametrize("K", [32, 64, 128, 256, 1024, 8192])
+@pytest.mark.parametrize("kind", [0, 2])
+@pytest.mark.parametrize("one_sign", [False, True])
+def test_fp32_codebook_no_further_off_than_fp32_products(cuda, K, kind, one_sign):
+    """A k-means codebook under fp32 x: the error against 64 bits is no larger
+    than that of ck_linear_f32's exact products in one chain (5% for the
+    chance of these values)."""
+    T, M, bits = 512, 1024, 8
+    packed, cb, _ = _matrix(cuda, M, K, bits, "fp32", K)
+    x = torch.randn(T, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(K))
+    if one_sign:
+        cb, x = cb.abs(), x.abs()
+    ref = x.double() @ cb[_indices(packed, M, K, bits).clamp_max(cb.numel() - 1)].double().T
+    one = torch.empty(T, M, device=cuda)
+    lib = nat.load()
+    nat.check(lib.ck_linear_f32(x.data_ptr(), packed.data_ptr(), cb.data_ptr(), one.data_ptr(), T,
+                                M, K, cb.numel(), bits, nat.stream_ptr(cuda)), "ck_linear_f32")
+    y = _gemm(cuda, x, packed, cb, M, K, bits, kind)
+    assert _rel(y, ref) <= 1.05 * _rel(one, ref)
