@@ -112,6 +112,15 @@ def timed_graph(torch, fn, reps, warmup):
 PREFILL_PROFILE = "frag_gemm_kernel_qwen3-8b_prompts.md"
 
 
+def read_profile_value(name, pattern, scale=1.0):
+    """A figure from a committed rocprofv3 summary, if any."""
+    p = os.path.join(ROOT, "profiles", name)
+    if not os.path.exists(p):
+        return None
+    m = re.search(pattern, open(p).read())
+    return round(float(m.group(1)) * scale, 4) if m else None
+
+
 def read_traffic(name):
     """HBM bytes per launch from a committed rocprofv3 PMC summary, if any."""
     p = os.path.join(ROOT, "profiles", name)
@@ -330,10 +339,11 @@ def huffman_sweep(torch, nat, lib, dev, huff, splits, plan, steps, warmup):
 def prefill_section(torch, nat, lib, dev, fixed, kinds, args):
     """benchmark config 4: bf16 MFMA prefill over the same fixed-width weights,
     T = 512 and 2048 tokens of bf16 N(0, 1) activations; per shape the mean
-    time of one cbq_linear_bf16_ws call with the workspace the module gives it
+    time of one cbq_linear_gemm call with the workspace the module gives it
     (x and, where that is faster, the weights as MFMA fragments, the GEMM and,
     when K is split, the partial sum) over 8 layers' distinct weights
     (graph-replayed)."""
+    import cbq_ops
     out = {"peak_tflops": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "shapes": {}}
     for T in (512, 2048):
         for kind in ("q_proj", "k_proj", "gate_proj", "down_proj"):
@@ -342,18 +352,20 @@ def prefill_section(torch, nat, lib, dev, fixed, kinds, args):
             M, K = t0.shape
             x = torch.randn(T, K, device=dev).bfloat16()
             o = torch.empty(T, M, device=dev, dtype=torch.bfloat16)
-            nws = int(lib.cbq_linear_bf16_gemm_workspace(T, M, K, t0.bits))
+            kind_of = cbq_ops.codebook_kind(t0.codebook)
+            nws = int(lib.cbq_linear_gemm_workspace(T, M, K, t0.bits, 1, kind_of))
             ws = torch.empty(max(1, (nws + 3) // 4), dtype=torch.float32, device=dev)
 
-            def run(ns=ns, x=x, o=o, ws=ws, nws=nws):
+            def run(ns=ns, x=x, o=o, ws=ws, nws=nws, kind_of=kind_of):
                 st = nat.stream_ptr(dev)
                 for n in ns:
                     t = fixed[n]
-                    rc = lib.cbq_linear_bf16_ws(x.data_ptr(), t.packed.data_ptr(),
-                                                t.codebook.data_ptr(), o.data_ptr(), T, M, K,
-                                                t.codebook.numel(), t.bits, ws.data_ptr(), nws, st)
+                    rc = lib.cbq_linear_gemm(x.data_ptr(), 1, t.packed.data_ptr(),
+                                             t.codebook.data_ptr(), o.data_ptr(), T, M, K,
+                                             t.codebook.numel(), t.bits, kind_of, ws.data_ptr(),
+                                             nws, st)
                     if rc:
-                        raise RuntimeError(f"cbq_linear_bf16_ws rc={rc} on {n}")
+                        raise RuntimeError(f"cbq_linear_gemm rc={rc} on {n}")
             ms, _ = timed_graph(torch, run, max(2, args.steps // 4), 1)
             us = ms * 1e3 / len(ns)
             tf = 2.0 * T * M * K / (us * 1e-6) / 1e12
@@ -366,6 +378,8 @@ def prefill_section(torch, nat, lib, dev, fixed, kinds, args):
                        "unit": "TFLOP/s", "frac": g["frac"],
                        "kernel": "frag_prep_kernel<13, 1> + frag_gemm_kernel, gate/up "
                                  "4096->12288, T=2048",
+                       "mfma_busy_rocprof_gemm_launch": read_profile_value(
+                           PREFILL_PROFILE, r"\*\*MFMA busy ([0-9.]+) %\*\*", 0.01),
                        "profile": "profiles/" + PREFILL_PROFILE}
     return out
 
