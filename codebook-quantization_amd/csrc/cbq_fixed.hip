@@ -1097,12 +1097,14 @@ size_t cbq_prefill_ws_bytes(int T, int M, int K);
 int cbq_prefill_f32(const float *x, const uint8_t *packed, const float *cb, float *out, int T,
                     int M, int K, int C, int bits, hipStream_t st, int S, float *ws);
 int cbq_prefill_f32_splits(int T, int M, int K);
+float cbq_prefill_f32_us(int T, int M, int K);
 // decode-first GEMM on the bf16 matrix cores, with a workspace (cbq_gemm.hip);
 // -1 = not handled there.
 int cbq_frag_linear(const void *x, bool f32, const uint8_t *packed, const float *cb, void *out,
                     int T, int M, int K, int C, int bits, int cb_kind, void *ws,
                     size_t ws_bytes, hipStream_t st);
 size_t cbq_frag_ws_bytes(int T, int M, int K, int bits, bool f32, int cb_kind);
+float cbq_frag_six_us(int T, int M, int K, int bits);
 
 int cbq_num_cus()
 {
@@ -1166,15 +1168,34 @@ static int prefill_f32_ws(const float *x, const uint8_t *packed, const float *co
                            split ? (float *)ws : nullptr);
 }
 
-// Calls that run on the fp32 kernel in place of the decode-first GEMM: of a
-// non-finite codebook (the few-token kernels' parts of x would make a NaN of an
-// infinite weight where a part is zero) and of an fp32 codebook below 256
-// columns (the GEMM leaves out the smallest part products; cbq_gemm.hip has
-// the errors).
-static bool fp32_kernel(int T, int K, int bits, int cb_kind)
+// How a batched fp32 call over a codebook of other than bf16 numbers goes, where
+// the decode-first GEMM would take it.
+enum F32Route { kRouteGemm, kRouteFp32, kRoutePlain };
+
+// Non-finite codebooks run on the fp32 kernel: the GEMM's and the few-token
+// kernels' parts of x would make a NaN of an infinite weight where a part is
+// zero.  Finite ones do below 256 columns (the GEMM leaves out the smallest
+// part products; cbq_gemm.hip has the errors) and wherever that or, up to 63
+// tokens, ck_linear_f32's token tiles are estimated faster than the GEMM's
+// three parts of W: 33 tokens, 4096 x 12288, 83 us in tiles against 178; 128
+// tokens 138 on the fp32 kernel against 196, 4096 x 4096 of 13 bits 63 / 76;
+// the GEMM from about 200 (300 tokens: 428 / 306, 4096 x 4096 155 / 90) and
+// for small matrices from about 48 (1024 x 2048, 63 tokens: 33 / 22).  Of 156
+// calls measured the choice is at most 6% behind the faster one but in four.
+// An 8-bit codebook of unknown kind is taken to hold such values.
+static F32Route f32_route(int T, int M, int K, int bits, int cb_kind)
 {
-    return (cb_kind == CBQ_CB_NON_FINITE || (cb_kind == CBQ_CB_FP32 && K < 256)) && T >= 33 &&
-           K % 32 == 0 && (bits == 8 || (bits >= 10 && bits <= 14));
+    if (T < 33 || K % 32 != 0 || (bits != 8 && (bits < 10 || bits > 14))) return kRouteGemm;
+    if (cb_kind == CBQ_CB_NON_FINITE) return kRouteFp32;
+    if (cb_kind != CBQ_CB_FP32 && !(cb_kind == CBQ_CB_UNKNOWN && bits == 8)) return kRouteGemm;
+    const bool tiles = T < 64 || bits == 14;
+    if (K >= 256) {
+        const float plain = tiles ? (float)((T + 15) / 16) *
+                                        (6.5f + 0.44e-6f * (float)M * (float)K)
+                                  : cbq_prefill_f32_us(T, M, K);
+        if (cbq_frag_six_us(T, M, K, bits) < plain) return kRouteGemm;
+    }
+    return tiles ? kRoutePlain : kRouteFp32;
 }
 
 size_t cbq_linear_f32_workspace(int T, int M, int K)
@@ -1191,11 +1212,12 @@ static int linear_f32_kind(const float *x, const uint8_t *packed, const float *c
     if (x && packed && codebook && out && M > 0 && K > 0 && C > 0 && bits >= 1 && bits <= 16) {
         int rc = cbq_fixed_fewtok_ws(x, true, packed, codebook, out, T, M, K, C, bits, workspace,
                                      ws_bytes, stream);
-        if (rc < 0)
+        const F32Route route = f32_route(T, M, K, bits, cb_kind);
+        if (rc < 0 && route == kRouteGemm)
             rc = cbq_frag_linear(x, true, packed, codebook, out, T, M, K, C, bits, cb_kind,
                                  workspace, ws_bytes, stream);
-        // a workspace below the GEMM's: the fp32 kernel with split K
-        if (rc < 0 && T >= 64 && bits != 14)
+        // (or a workspace below the GEMM's) the fp32 kernel with split K
+        if (rc < 0 && (route == kRouteFp32 || (T >= 64 && bits != 14)))
             rc = prefill_f32_ws(x, packed, codebook, out, T, M, K, C, bits, workspace, ws_bytes,
                                 stream);
         if (rc >= 0) return rc;
@@ -1456,7 +1478,11 @@ int cbq_linear_bf16_ws(const void *x_bf16, const uint8_t *packed, const float *c
 size_t cbq_linear_gemm_workspace(int T, int M, int K, int bits, int x_bf16, int cb_kind)
 {
     if (T <= 0 || M <= 0 || K <= 0 || bits < 1) return 0;
-    if (!x_bf16 && fp32_kernel(T, K, bits, cb_kind)) return prefill_f32_partials(T, M, K);
+    if (!x_bf16) {
+        const F32Route route = f32_route(T, M, K, bits, cb_kind);
+        if (route == kRouteFp32) return prefill_f32_partials(T, M, K);
+        if (route == kRoutePlain) return 0;
+    }
     const size_t few = cbq_fewtok_ws_bytes(T, M, K, bits, !x_bf16);
     if (x_bf16 && T <= 64 && K % 128 == 0) return few;   // the few-token kernel's tokens
     size_t need = cbq_frag_ws_bytes(T, M, K, bits, !x_bf16, cb_kind);
@@ -1472,14 +1498,6 @@ int cbq_linear_gemm(const void *x, int x_bf16, const uint8_t *packed, const floa
     if (x_bf16)
         return linear_bf16_kind(x, packed, codebook, out, T, M, K, C, bits, cb_kind, workspace,
                                 ws_bytes, stream);
-    if (x && packed && codebook && out && M > 0 && K > 0 && C > 0 &&
-        fp32_kernel(T, K, bits, cb_kind)) {
-        const int rc = prefill_f32_ws((const float *)x, packed, codebook, (float *)out, T, M, K, C,
-                                      bits, workspace, ws_bytes, stream);
-        return rc >= 0 ? rc
-                       : ck_linear_f32((const float *)x, packed, codebook, (float *)out, T, M, K, C,
-                                       bits, stream);
-    }
     return linear_f32_kind((const float *)x, packed, codebook, (float *)out, T, M, K, C, bits,
                            cb_kind, workspace, ws_bytes, stream);
 }

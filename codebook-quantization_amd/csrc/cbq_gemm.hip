@@ -998,6 +998,18 @@ size_t cbq_frag_ws_bytes(int T, int M, int K, int bits, bool f32, int cb_kind)
     return gemm_ws_bytes(p, NP, nw, T, K);
 }
 
+// Estimated microseconds of the batched linear over a codebook of other than
+// bf16 numbers and fp32 x, all launches: three table passes, three parts of
+// every weight written (and, past the last-level cache, read from HBM), twice
+// the products of the plan's steps.  Within 19% of 156 calls measured (as
+// cbq_prefill_f32_us, 33 to 768 tokens, 8 and 13 bits).
+float cbq_frag_six_us(int T, int M, int K, int bits)
+{
+    const float mw = (float)M * (float)K * 1e-6f;
+    return 2.f + 1.4e-3f * (float)(1 << bits) + mw * (1.15f + 0.066f * (float)(bits - 8)) +
+           3.f * std::max(0.f, mw - 30.f) + 1.6f * gemm_plan(T, M, K, 3, 3).us;
+}
+
 // The batched linear over fixed-width indices with a workspace of at least
 // cbq_frag_ws_bytes (16-byte aligned); -1: not handled here.
 int cbq_frag_linear(const void *x, bool f32, const uint8_t *packed, const float *cb, void *out,

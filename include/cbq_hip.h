@@ -81,9 +81,10 @@ int cbq_linear_f32_ws(const float *x, const uint8_t *packed, const float *codebo
 /* The batched linear for fp32 or bf16 x (x_bf16 != 0; out likewise) with a
  * workspace of cbq_linear_gemm_workspace bytes (256-byte aligned):
  * cbq_linear_f32_ws / cbq_linear_bf16_ws for a codebook of cb_kind.  fp32 x
- * and a non-finite codebook, or one of other than bf16 values and K < 256:
- * ck_linear_f32's fp32 kernel with split K from 33 tokens on (the bf16 parts of
- * x cannot multiply an infinity, and short sums keep every part product).  No
+ * and a non-finite codebook: ck_linear_f32's fp32 kernel with split K from 33
+ * tokens on (the bf16 parts of x cannot multiply an infinity); of other than
+ * bf16 values: that kernel (up to 63 tokens token tiles) below 256 columns
+ * (short sums keep every part product) and where it is estimated faster.  No
  * counterpart in the reference: GPUAcceleratedLinear
  * (src/gpu_accelerated_functions.py:928-950) over batched tokens. */
 int cbq_linear_gemm(const void *x, int x_bf16, const uint8_t *packed, const float *codebook,
