@@ -28,8 +28,9 @@
 // Why decode first: a fused kernel gathers every weight again for each 512
 // tokens, and on this chip the decode's VALU and LDS work adds to the MFMA
 // time instead of running under it.  The transient fragments are bounded (a
-// slab of at most kSlabBytes), stay in the 256 MiB last-level cache, and
-// make both GEMM operands plain 1 KiB global -> LDS copies.
+// slab of kSlabBytes, or of 256 rows where those are more), mostly stay in the
+// 256 MiB last-level cache (12288 x 4096 in one part: 96 MiB), and make both
+// GEMM operands plain 1 KiB global -> LDS copies.
 #include "cbq_device.h"
 
 #include <algorithm>
@@ -42,7 +43,8 @@ namespace {
 constexpr int kGBlock = 512;                   // GEMM: 8 waves, two per SIMD
 constexpr int kGWaves = kGBlock / CBQ_WAVE;
 constexpr int kPBlock = 256;                   // prep: 4 waves
-constexpr int kPrepBlocks = 5;                 // prep blocks per CU (30 KiB of LDS each)
+constexpr int kPrepBlocks = 5;                 // prep blocks per CU (13 bits: 30 KiB of LDS each;
+                                               // at 14, 47 KiB, three of them run at once)
 constexpr int kPrepGroups = 8;                 // column groups (of 32) per W prep tile
 constexpr size_t kFrag = 1024;                 // bytes of one fragment
 constexpr size_t kSlabBytes = (size_t)384 << 20;
@@ -962,7 +964,7 @@ __global__ __launch_bounds__(kPBlock) void frag_x_kernel(const void *__restrict_
                (int64_t)((T + 15) >> 4) * (K >> 5), (int64_t)gridDim.x * (kPBlock / CBQ_WAVE));
 }
 
-// Below 33 tokens of fp32 (65 of bf16) the few-token kernels of cbq_tiny.hip
+// Below 33 tokens of fp32 (64 of bf16; 65 where K % 128 == 0) the few-token kernels of cbq_tiny.hip
 // read the weights in place: T = 32 fp32, 12288 x 4096: 52 us against 66 here;
 // T = 48: 77 against 68.
 bool frag_shape(int T, int M, int K, bool f32)

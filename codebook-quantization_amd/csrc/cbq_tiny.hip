@@ -649,7 +649,7 @@ int cbq_fixed_fewtok_t_bf16(const uint16_t *x, const uint8_t *packed, const floa
 // 4 to 5 us; measured break-even at 12000 (fp32, which also saves the split
 // in the kernel) and 16000 lines saved per CU: bf16 T = 40 4096 x 4096
 // (14300) 15.8 by rows against 16.6, T = 48 (18400) 17.1 / 15.8, T = 64
-// 4096 x 12288 51.7 / 30.2; fp32 T = 16 4096 x 12288 35.0 / 31.4, 4096 x 1024
+// 4096 x 12288 51.7 / 30.2; fp32 T = 16 4096 x 12288 32.4 / 24.9, 4096 x 1024
 // (10200) 14.0 / 14.7.  17 to 32 fp32 tokens have no one-launch path without
 // it (12288 x 4096, T = 32: 51 us in two launches, 29 here).
 size_t cbq_fewtok_ws_bytes(int T, int M, int K, int bits, bool f32)

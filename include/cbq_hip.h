@@ -52,9 +52,10 @@ size_t cbq_linear_f32_workspace(int T, int M, int K);
 
 /* ck_linear_f32 with a caller workspace (>= cbq_linear_f32_workspace bytes,
  * 16-byte aligned): 17 to 32 tokens (fewer where it pays; K % 128 == 0) run in
- * one launch with x's bf16 parts there in MFMA fragment order; for T >= 33 (K % 32 == 0, widths 8 and 10..14, x 16-byte
- * aligned) x (three exact bf16 parts) and the weights are first written there
- * in MFMA fragment order, the weights in slabs of at most 384 MiB, and
+ * one launch with x's bf16 parts there in MFMA fragment order; for T >= 33
+ * (K % 32 == 0, widths 8 and 10..14, x 16-byte aligned) x (three exact bf16
+ * parts) and the weights are first written there in MFMA fragment order, the
+ * weights in slabs of 384 MiB (256 rows where those take more), and
  * multiplied on the bf16 matrix cores with fp32 accumulation; K is split
  * over blocks when the output tiles alone would leave CUs idle (partials in
  * the workspace, summed in split order).  A codebook with values that are
@@ -460,8 +461,8 @@ size_t cbq_split_fewtok_ws_bytes(int K);
 /* y [T, M] = x [T, K] @ W^T for one split-format matrix and any T >= 1 (meant
  * for more tokens than the few-token kernel takes in one launch): x (fp32 as
  * three exact bf16 parts, or x_bf16 != 0: bf16) and the decoded weights go to
- * the workspace in MFMA fragment order, the weights in slabs of at most 384
- * MiB, and are multiplied on the bf16 matrix cores with fp32 accumulation.
+ * the workspace in MFMA fragment order, the weights in slabs of 384 MiB (256
+ * rows where those take more), and are multiplied on the bf16 matrix cores with fp32 accumulation.
  * out is fp32 (bf16 for bf16 x).  K % 1024 == 0, M * K a whole number of
  * chunks, x and ws 16-byte aligned, ws of at least
  * cbq_split_linear_gemm_ws_bytes; CK_ERR_ARG otherwise.  Weights are finite

@@ -1,8 +1,11 @@
-"""fp32 MFMA path of ck_linear_f32 (T >= 64) and its split-K form
-cbq_linear_f32_ws vs the oracle (compressed_matmul_f32_chunk restated).
+"""fp32 MFMA path of ck_linear_f32 (T >= 64), and cbq_linear_f32_ws with its
+whole workspace (weights decoded first, bf16 matrix cores), vs the oracle
+(compressed_matmul_f32_chunk restated).  (Split K of the fp32 path, with a
+smaller workspace: test_gpu_linear_workspaces.py.)
 
-Products are exact in fp32 (v_mfma_f32_32x32x2_f32) and only the summation
-order differs, so the bar is the fp32 GEMV's: rel-L2 <= 1e-5."""
+Products are exact (fp32 on v_mfma_f32_32x32x2_f32, or three bf16 parts of x
+with bf16 weights) and only the summation order differs, so the bar is the
+fp32 GEMV's: rel-L2 <= 1e-5."""
 import numpy as np
 import pytest
 import torch
@@ -79,10 +82,10 @@ def test_matches_token_tile_path(cuda):
 
 @pytest.mark.parametrize("M,K", [(300, 4096), (70, 12288)])
 def test_huffman_module_batched_tokens(cuda, oracle, M, K):
-    """HuffmanCodebookLinear with T >= 64 decodes its format to transient
-    fixed-width indices (the split format through cbq_split_to_packed, the
-    stream through cbq_huff_decode_indices + cbq_pack_indices) and runs the
-    fp32 matrix-core GEMM; both layouts against the reference C kernel."""
+    """HuffmanCodebookLinear with T >= 64 decodes the split format to MFMA
+    fragments (split_gemm), and the stream to transient fixed-width indices
+    (cbq_huff_decode_indices + cbq_pack_indices) for cbq_linear_gemm; both
+    layouts against the reference C kernel."""
     import huffman_codebook as hc
     from test_gpu_huffman import _lin
     rng = np.random.default_rng(M)
@@ -102,7 +105,7 @@ def test_huffman_module_batched_tokens(cuda, oracle, M, K):
 def test_split_to_packed(cuda, oracle, M, K):
     """cbq_split_to_packed turns the split format back into the reference's
     LSB-first index stream bit for bit, and the module's batched-token path
-    on it equals the stream-decode path exactly."""
+    (the split format as fragments) equals the stream-decode path exactly."""
     import ctypes
     import cbq_native as nat
     import huffman_codebook as hc
