@@ -1180,8 +1180,10 @@ enum F32Route { kRouteGemm, kRouteFp32, kRoutePlain };
 // three parts of W: 33 tokens, 4096 x 12288, 83 us in tiles against 178; 128
 // tokens 138 on the fp32 kernel against 196, 4096 x 4096 of 13 bits 63 / 76;
 // the GEMM from about 200 (300 tokens: 428 / 306, 4096 x 4096 155 / 90) and
-// for small matrices from about 48 (1024 x 2048, 63 tokens: 33 / 22).  Of 156
-// calls measured the choice is at most 6% behind the faster one but in four.
+// for small matrices from about 48 (1024 x 2048, 63 tokens: 33 / 22).  Of 316
+// calls measured the choice is 0.3% behind the faster one in the mean, at most
+// 6% slower than without the GEMM and 17% than with it.  A tie stays off the
+// GEMM (0.97).
 // An 8-bit codebook of unknown kind is taken to hold such values.
 static F32Route f32_route(int T, int M, int K, int bits, int cb_kind)
 {
@@ -1193,7 +1195,7 @@ static F32Route f32_route(int T, int M, int K, int bits, int cb_kind)
         const float plain = tiles ? (float)((T + 15) / 16) *
                                         (6.5f + 0.44e-6f * (float)M * (float)K)
                                   : cbq_prefill_f32_us(T, M, K);
-        if (cbq_frag_six_us(T, M, K, bits) < plain) return kRouteGemm;
+        if (cbq_frag_six_us(T, M, K, bits) < 0.97f * plain) return kRouteGemm;
     }
     return tiles ? kRoutePlain : kRouteFp32;
 }

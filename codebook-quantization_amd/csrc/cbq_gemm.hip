@@ -788,6 +788,7 @@ struct GemmPlan {
     int shape, S;
     int rows;               // rows per slab (a multiple of 256, or all M)
     float us;               // estimated time of the GEMM over all slabs
+    float chain;            // of that, the column groups' steps
 };
 
 template <class C>
@@ -887,13 +888,15 @@ GemmPlan gemm_plan(int T, int M, int K, int NP, int nw)
         for (int S = 1; S <= 16 && (S == 1 || G / S >= 8); S++) {
             if (S > 1 && tiles * S > 2 * cus) break;
             const float rounds = (float)((tiles * S + cus - 1) / cus);
-            float t = rounds * ((float)((G + S - 1) / S) * s.step + 5.f);
+            const float chain = rounds * (float)((G + S - 1) / S) * s.step;
+            float t = chain + rounds * 5.f;
             if (S > 1) t += 3.f + (float)(tiles * S) * (float)(s.TT * s.TM) * 8.f * 2e-7f;
             if (best == 0.f || t < best) {
                 best = t;
                 p.shape = i;
                 p.S = S;
                 p.us = t * slabs;
+                p.chain = chain * slabs;
             }
         }
     }
@@ -1002,14 +1005,16 @@ size_t cbq_frag_ws_bytes(int T, int M, int K, int bits, bool f32, int cb_kind)
 
 // Estimated microseconds of the batched linear over a codebook of other than
 // bf16 numbers and fp32 x, all launches: three table passes, three parts of
-// every weight written (and, past the last-level cache, read from HBM), twice
-// the products of the plan's steps.  Within 19% of 156 calls measured (as
-// cbq_prefill_f32_us, 33 to 768 tokens, 8 and 13 bits).
+// every weight written (and, past the last-level cache, read from HBM), half
+// as long again a step as with one part.  Fitted to 356 calls (M x K from
+// 512 x 2048 to 12288 x 4096 and 5000 x 12288, 33 to 768 tokens, 8 to 13 bits):
+// within 15%.
 float cbq_frag_six_us(int T, int M, int K, int bits)
 {
     const float mw = (float)M * (float)K * 1e-6f;
-    return 2.f + 1.4e-3f * (float)(1 << bits) + mw * (1.15f + 0.066f * (float)(bits - 8)) +
-           3.f * std::max(0.f, mw - 30.f) + 1.6f * gemm_plan(T, M, K, 3, 3).us;
+    const GemmPlan p = gemm_plan(T, M, K, 3, 3);
+    return 6.7f + 1.46e-3f * (float)(1 << bits) + mw * (1.5f + 0.058f * (float)(bits - 8)) +
+           2.3f * std::max(0.f, mw - 30.f) + 1.55f * p.chain + 0.95f * (p.us - p.chain);
 }
 
 // The batched linear over fixed-width indices with a workspace of at least
