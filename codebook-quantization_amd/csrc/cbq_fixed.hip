@@ -1192,9 +1192,13 @@ static F32Route f32_route(int T, int M, int K, int bits, int cb_kind)
     if (cb_kind != CBQ_CB_FP32 && !(cb_kind == CBQ_CB_UNKNOWN && bits == 8)) return kRouteGemm;
     const bool tiles = T < 64 || bits == 14;
     if (K >= 256) {
-        const float plain = tiles ? (float)((T + 15) / 16) *
-                                        (6.5f + 0.44e-6f * (float)M * (float)K)
-                                  : cbq_prefill_f32_us(T, M, K);
+        // a tile of 16 tokens: the few-token kernel, or the older one where
+        // K % 128 != 0 (bound by its chain along K: 512 x 4064, 48 tokens, 71
+        // us against 31 on the GEMM)
+        const float mk = (float)M * (float)K * 1e-6f;
+        const float tile = K % 128 == 0 ? 6.5f + 0.44f * mk
+                                        : 5.7f + 3.3e-3f * (float)K + 0.3f * mk;
+        const float plain = tiles ? (float)((T + 15) / 16) * tile : cbq_prefill_f32_us(T, M, K);
         if (cbq_frag_six_us(T, M, K, bits) < 0.97f * plain) return kRouteGemm;
     }
     return tiles ? kRoutePlain : kRouteFp32;

@@ -84,7 +84,8 @@ def test_fp32_codebooks_take_the_faster_route(ws):
     for T, M, K, bits, want in (
             (33, 4096, 12288, 8, "tiles"), (33, 12288, 4096, 13, "tiles"),
             (33, 4096, 4096, 8, "tiles"), (48, 2048, 1024, 13, "tiles"),
-            (63, 1024, 2048, 8, "gemm"), (64, 4096, 12288, 8, "fp32"),
+            (63, 1024, 2048, 8, "gemm"), (48, 512, 4064, 8, "gemm"),
+            (33, 9000, 4064, 13, "tiles"), (64, 4096, 12288, 8, "fp32"),
             (128, 4096, 12288, 13, "fp32"), (128, 4096, 4096, 13, "fp32"),
             (128, 6144, 2048, 13, "fp32"), (128, 6144, 2048, 8, "gemm"),
             (300, 4096, 12288, 8, "gemm"), (300, 12288, 4096, 13, "gemm"),
